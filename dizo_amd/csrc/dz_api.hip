@@ -674,7 +674,7 @@ int32_t dz_normals(uint64_t seed, uint32_t stream_id, uint64_t offset, int64_t n
   rc = ensure_device(dev, &ds);
   if (rc) return rc;
   hipError_t e = dz::launch_normals(dtype, ds->tab[dtype], seed, stream_id, offset, (uint64_t)n, d_out,
-                                    (hipStream_t)stream);
+                                    (uint32_t)ds->cus, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "normals kernel launch");
   return DZ_OK;
 }

@@ -181,8 +181,16 @@ struct StaticPlanBatch {
 };
 hipError_t launch_static_plan(const StaticPlanBatch& b, DzChunk* chunks, uint32_t* group_begin, uint32_t* counters,
                               hipStream_t st);
+// z export: ranges of at least kNormalsLdsGroups Philox blocks of 8 elements
+// run the persistent kernel with the quantile table in LDS. Kernel times by
+// elements, table in memory against in LDS: fp16 2^16 2.8 / 3.6 us, 2^18 3.0 /
+// 3.7, 2^19 3.5 / 3.8, 2^20 4.9 / 3.8, 2^22 12.7 / 5.4; fp32 2^18 3.5 / 4.1,
+// 2^19 4.2 / 4.3, 2^20 6.0 / 4.6. The gathers from memory run at about one
+// lane per clock and CU, so they cost more from 2^19 elements on.
+constexpr int kNormalsThreads = 1024;
+constexpr uint64_t kNormalsLdsGroups = 1u << 16;
 hipError_t launch_normals(int dtype, const void* tab, uint64_t seed, uint32_t stream, uint64_t offset,
-                          uint64_t n, void* out, hipStream_t st);
+                          uint64_t n, void* out, uint32_t cus, hipStream_t st);
 hipError_t launch_philox(uint64_t seed, uint32_t stream, uint64_t q0, uint64_t n, uint32_t* out,
                          hipStream_t st);
 

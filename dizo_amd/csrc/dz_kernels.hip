@@ -101,13 +101,6 @@ __device__ __forceinline__ uint32_t word_of(const DzU4& w, int i) {
   return i == 0 ? w.x : i == 1 ? w.y : i == 2 ? w.z : w.w;
 }
 
-// z bits of a 16-bit field h (sign bit + 15-bit index) from a quantile table.
-template <int DT>
-__device__ __forceinline__ uint32_t z_bits(const typename DT_<DT>::S* tab, uint32_t h) {
-  const uint32_t mag = (uint32_t)tab[h & 0x7fffu];
-  return mag | ((h & 0x8000u) << (DT_<DT>::kBits - 16));
-}
-
 // ---------------------------------------------------------------------------
 // Per-launch delta tables.
 //
@@ -458,6 +451,15 @@ __device__ __forceinline__ dz_u32x4 ld_stream(const void* p) {
 }
 __device__ __forceinline__ void st_stream(void* p, dz_u32x4 v) {
   __builtin_nontemporal_store(v, (dz_global_u32x4*)(uintptr_t)p);
+}
+
+// A 16-byte store at any element's address (gfx950 takes global accesses of
+// every size at any address; the declared alignment keeps the compiler from
+// assuming more).
+typedef dz_u32x4 dz_u32x4_any __attribute__((aligned(2)));
+typedef __attribute__((address_space(1))) dz_u32x4_any dz_global_u32x4_any;
+__device__ __forceinline__ void st_any(void* p, dz_u32x4 v) {
+  *(dz_global_u32x4_any*)(uintptr_t)p = v;
 }
 
 // Wave-uniform copy of a 32-bit value in a scalar register.
@@ -1488,20 +1490,102 @@ __global__ void __launch_bounds__(256) static_plan_kernel(StaticPlanBatch b, DzC
   }
 }
 
-// z(seed, stream, offset + i) for i < n, written densely in T.
+// The eight z of a Philox block in T, from a quantile table `tab` of T (in LDS
+// or in memory): 16-bit T packed into one vector, fp32 into two.
+template <int DT>
+struct ZVec {
+  static constexpr int kVecs = DT == DZ_F32 ? 2 : 1;
+  dz_u32x4 v[kVecs];
+};
+template <int DT>
+__device__ __forceinline__ ZVec<DT> z_vec(const typename DT_<DT>::S* tab, const DzU4& w) {
+  ZVec<DT> r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t x = word_of(w, i);
+    uint32_t e0, e1;
+    lookup2(tab, x, e0, e1);
+    if constexpr (DT == DZ_F32) {
+      r.v[i >> 1][2 * (i & 1)] = e0 | ((x & 0x8000u) << 16);
+      r.v[i >> 1][2 * (i & 1) + 1] = e1 | (x & 0x80000000u);
+    } else {
+      r.v[0][i] = (e0 | (e1 << 16)) | (x & 0x80008000u);
+    }
+  }
+  return r;
+}
+
+// The launch's range of z: n elements from element `offset` of the stream, so
+// group g (8 elements, one Philox block) covers outputs 8 g - skip .. 8 g -
+// skip + 7 for skip = offset mod 8. Element indices wrap modulo 2^64.
+template <int DT>
+__device__ __forceinline__ void store_z_group(const ZVec<DT>& z, uint64_t g, uint32_t skip, uint64_t n, void* out) {
+  using S = typename DT_<DT>::S;
+  const int64_t i0 = (int64_t)(g * 8u) - (int64_t)skip;
+  S* p = (S*)out + i0;
+  if (i0 >= 0 && (uint64_t)i0 + 8u <= n) {
+#pragma unroll
+    for (int k = 0; k < ZVec<DT>::kVecs; ++k) st_any((char*)p + 16 * k, z.v[k]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t b = DT == DZ_F32 ? z.v[DT == DZ_F32 ? j >> 2 : 0][j & 3] : z.v[0][j >> 1] >> (16 * (j & 1));
+      if (i0 + j >= 0 && (uint64_t)(i0 + j) < n) p[j] = (S)b;
+    }
+  }
+}
+
+// z(seed, stream, offset + i) for i < n, written densely in T: one thread per
+// Philox block of 8 elements, looked up in the quantile table in memory. For
+// short ranges, which a launch's start and one chain of latencies bound (1.5
+// us for a wave's worth, 2.8 at 2^16 fp16 elements).
 template <int DT>
 __global__ void __launch_bounds__(256) normals_kernel(const void* __restrict__ gtab, uint64_t seed,
                                                       uint32_t stream, uint64_t offset, uint64_t n,
                                                       void* __restrict__ out) {
+  const uint32_t skip = (uint32_t)(offset & 7u);
+  const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g * 8u >= n + skip) return;
+  const DzU4 w = dz_philox_group(seed, stream, (offset - skip + g * 8u) >> 3);
+  store_z_group<DT>(z_vec<DT>((const typename DT_<DT>::S*)gtab, w), g, skip, n, out);
+}
+
+// The same for long ranges: persistent workgroups copy the quantile table to
+// LDS once (64 KB for 16-bit T, two workgroups per CU; 128 KB for fp32, one),
+// then take tiles of 1024 groups in turn. 105 M fp16 elements into buffers
+// used in turn take 44 us, 4.8 TB/s of stores (with a thread and a block of
+// the generator per element 214 us); 2^27 fp16 elements into one buffer, which
+// the Infinity Cache holds, 44 us, where the Philox chain's VALU work is the
+// bound; 2^27 fp32 elements 124 us (4.3 TB/s). The stores are plain ones: with
+// the non-temporal hint 2^27 elements took 84 us (fp16) and 252 us (fp32), and
+// whoever asked for z reads it next.
+template <int DT>
+__global__ void __launch_bounds__(kNormalsThreads, DT == DZ_F32 ? 4 : 8)
+    normals_lds_kernel(const void* __restrict__ gtab, uint64_t seed, uint32_t stream, uint64_t offset, uint64_t n,
+                       void* __restrict__ out) {
   using S = typename DT_<DT>::S;
-  const S* tab = (const S*)gtab;
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t e = offset + i;
-  const DzU4 w = dz_philox_group(seed, stream, e >> 3);
-  const uint32_t j = (uint32_t)(e & 7u);
-  const uint32_t h = (word_of(w, (int)(j >> 1)) >> (16 * (j & 1))) & 0xffffu;
-  ((S*)out)[i] = (S)z_bits<DT>(tab, h);
+  __shared__ __attribute__((aligned(16))) S tab[kDzTabEntries];
+  constexpr int kSlices = kDzTabEntries * (int)sizeof(S) / (16 * kNormalsThreads);
+#pragma unroll
+  for (int v = 0; v < kSlices; ++v) {
+    const uint32_t at = (uint32_t)(v * kNormalsThreads + threadIdx.x) * 16u;
+    *(dz_u32x4*)((char*)tab + at) = *(const dz_u32x4*)((const char*)gtab + at);
+  }
+  __syncthreads();
+  const uint32_t skip = (uint32_t)(offset & 7u);
+  const uint64_t groups = (n + skip + 7u) >> 3;
+  const uint64_t first = offset - skip;
+  for (uint64_t t = blockIdx.x; t * kNormalsThreads < groups; t += gridDim.x) {
+    const uint64_t g = t * kNormalsThreads + threadIdx.x;
+    if (g >= groups) break;
+    const uint64_t q = (first + t * (kNormalsThreads * 8u)) >> 3;  // of the tile's first group
+    // the counters' high word is uniform over the tile unless the low word
+    // (or the element index) wraps in it
+    const DzU4 w = (uint32_t)q <= 0xffffffffu - (kNormalsThreads - 1u)
+                       ? dz_philox_counter(seed, stream, (uint32_t)q + threadIdx.x, (uint32_t)(q >> 32))
+                       : dz_philox_group(seed, stream, (first + g * 8u) >> 3);
+    store_z_group<DT>(z_vec<DT>(tab, w), g, skip, n, out);
+  }
 }
 
 // Raw Philox blocks for counter q = q0 + i (test and KAT use).
@@ -1672,24 +1756,27 @@ hipError_t launch_static_plan(const StaticPlanBatch& b, DzChunk* chunks, uint32_
   return hipGetLastError();
 }
 
+template <int DT>
+static void launch_normals_dt(const void* tab, uint64_t seed, uint32_t stream, uint64_t offset, uint64_t n, void* out,
+                              uint32_t cus, hipStream_t st) {
+  const uint64_t groups = ((offset & 7u) + n + 7u) >> 3;
+  if (groups >= kNormalsLdsGroups) {
+    const uint32_t grid = cus * (DT == DZ_F32 ? 1u : 2u);
+    hipLaunchKernelGGL((normals_lds_kernel<DT>), dim3(grid), dim3(kNormalsThreads), 0, st, tab, seed, stream, offset, n,
+                       out);
+  } else {
+    hipLaunchKernelGGL((normals_kernel<DT>), dim3((uint32_t)((groups + 255) / 256)), dim3(256), 0, st, tab, seed, stream,
+                       offset, n, out);
+  }
+}
+
 hipError_t launch_normals(int dtype, const void* tab, uint64_t seed, uint32_t stream, uint64_t offset,
-                          uint64_t n, void* out, hipStream_t st) {
-  const uint64_t blocks = (n + 255) / 256;
+                          uint64_t n, void* out, uint32_t cus, hipStream_t st) {
   switch (dtype) {
-    case DZ_F32:
-      hipLaunchKernelGGL((normals_kernel<DZ_F32>), dim3((uint32_t)blocks), dim3(256), 0, st, tab,
-                         seed, stream, offset, n, out);
-      break;
-    case DZ_F16:
-      hipLaunchKernelGGL((normals_kernel<DZ_F16>), dim3((uint32_t)blocks), dim3(256), 0, st, tab,
-                         seed, stream, offset, n, out);
-      break;
-    case DZ_BF16:
-      hipLaunchKernelGGL((normals_kernel<DZ_BF16>), dim3((uint32_t)blocks), dim3(256), 0, st, tab,
-                         seed, stream, offset, n, out);
-      break;
-    default:
-      return hipErrorInvalidValue;
+    case DZ_F32: launch_normals_dt<DZ_F32>(tab, seed, stream, offset, n, out, cus, st); break;
+    case DZ_F16: launch_normals_dt<DZ_F16>(tab, seed, stream, offset, n, out, cus, st); break;
+    case DZ_BF16: launch_normals_dt<DZ_BF16>(tab, seed, stream, offset, n, out, cus, st); break;
+    default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }

@@ -75,6 +75,30 @@ def test_z_export_matches_oracle(dt):
     tab.close()
 
 
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("offset,n", [(5, 3), (7, 2), (0, 8), (3, 2**19 - 11), (0, 2**19 - 8), (1, 2**19 - 1), (8, 2**19),
+                                      (2**35 - 8 * 700 + 3, 2**19 + 13), (0, 2**22 + 5), (2**64 - 8 * 9 + 2, 4096)])
+def test_normals_ranges_match_oracle(dt, offset, n):
+    """Ranges that start and end inside a Philox block, on both sides of 2^16 blocks (where the LDS
+    kernel takes over), across a wrap of the counter's low word and of the element index."""
+    from dizo_amd.table import normals
+    z = normals(99, 0, offset, n, DT_TORCH[dt], torch.device("cuda", 0))
+    idx = np.arange(n, dtype=np.uint64) + np.uint64(offset)
+    assert_bits_equal(to_bits(z), rng.z_bits(99, 0, idx, dt), dt, f"normals {offset} {n}")
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("n", [100, 2**19 + 3])
+def test_normals_into_a_misaligned_buffer(dt, n):
+    """z written one element past a vector boundary leaves its neighbours alone."""
+    from dizo_amd import _lib as L
+    from dizo_amd.table import dtype_code
+    buf = torch.full((n + 2,), 7.0, dtype=DT_TORCH[dt], device="cuda")
+    L.call("dz_normals", 5, 1, 11, n, dtype_code(buf.dtype), buf[1:].data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert float(buf[0]) == 7.0 and float(buf[-1]) == 7.0
+    assert_bits_equal(to_bits(buf[1:-1]), rng.z_bits(5, 1, np.arange(n, dtype=np.uint64) + np.uint64(11), dt), dt)
+
+
 def test_philox_blocks_match_oracle():
     from dizo_amd.table import philox_blocks
     for seed, stream, q0 in ((0, 0, 0), (26, 1, 2**32 - 3), (2**64 - 1, 2, 2**40)):
