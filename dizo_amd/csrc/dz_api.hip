@@ -213,7 +213,7 @@ struct dz_table {
   bool projection = false;
   int32_t n = 0;
   uint32_t chunk_elems = 0;  // tile size (elements)
-  uint32_t nchunks = 0;      // ZO tables: full, aligned tiles first (the prefetching loop runs them)
+  uint32_t nchunks = 0;      // ZO tables: full tiles first (the prefetching loop runs them)
   std::vector<uint64_t> ptrs, aux, zoff;
   std::vector<int64_t> numels;
   std::vector<uint32_t> group_begin;  // n + 1 chunk indices (projection tables)
@@ -343,13 +343,13 @@ void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
   }
 }
 
-// ZO tile lists: full, aligned tiles first (in tensor order), then the
-// partial or misaligned ones; returns the number of full tiles. The order of
+// ZO tile lists: full tiles first (in tensor order), then the partial ones;
+// returns the number of full tiles. The order of
 // the tiles changes no result (z is a function of the element index), and it
 // lets the RMW kernel run its full tiles without a per-tile shape test.
 uint32_t full_tiles_first(std::vector<DzChunk>* v, uint32_t elems) {
   auto it = std::stable_partition(v->begin(), v->end(), [elems](const DzChunk& c) {
-    return c.n == elems && (c.meta & kDzMetaAligned) != 0u;
+    return c.n == elems;
   });
   return (uint32_t)(it - v->begin());
 }

@@ -143,8 +143,7 @@ struct LaunchEvents {
   hipEvent_t stop = nullptr;
 };
 
-// The chunk list holds its full, aligned tiles first; the rest are partial
-// or misaligned. prefetch: run the prefetching tile loop where the mode
+// The chunk list holds its full tiles first; the rest are partial. prefetch: run the prefetching tile loop where the mode
 // allows it (rmw_prefetch_mode); the caller sets it for long launches.
 hipError_t launch_rmw(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t grid,
                       const void* qtab, const DzScalars& s, const DzScalarPtrs& p, uint32_t* counters,

@@ -444,7 +444,14 @@ __device__ __forceinline__ uint32_t apply_one(uint32_t th, uint32_t h, uint32_t 
 // which count only against the vector-memory wait counter. As generic (FLAT)
 // accesses they would also count against the LDS counter, and every wait for
 // an LDS table lookup would then wait for the tile loads in flight as well.
-typedef __attribute__((address_space(1))) dz_u32x4 dz_global_u32x4;
+//
+// The vectors are declared at element alignment: gfx950 takes global accesses
+// of every size at any address, and the instruction is the same, so tensors
+// that start anywhere (views into a packed buffer) go the same way as aligned
+// ones: a bf16 pass over 60 M elements of a packed buffer of odd sizes takes
+// 50 us against 96 when its groups went element by element.
+typedef dz_u32x4 dz_u32x4_any __attribute__((aligned(2)));
+typedef __attribute__((address_space(1))) dz_u32x4_any dz_global_u32x4;
 typedef __attribute__((address_space(1))) char dz_global_char;
 __device__ __forceinline__ dz_u32x4 ld_stream(const void* p) {
   return __builtin_nontemporal_load((const dz_global_u32x4*)(uintptr_t)p);
@@ -452,15 +459,8 @@ __device__ __forceinline__ dz_u32x4 ld_stream(const void* p) {
 __device__ __forceinline__ void st_stream(void* p, dz_u32x4 v) {
   __builtin_nontemporal_store(v, (dz_global_u32x4*)(uintptr_t)p);
 }
-
-// A 16-byte store at any element's address (gfx950 takes global accesses of
-// every size at any address; the declared alignment keeps the compiler from
-// assuming more).
-typedef dz_u32x4 dz_u32x4_any __attribute__((aligned(2)));
-typedef __attribute__((address_space(1))) dz_u32x4_any dz_global_u32x4_any;
-__device__ __forceinline__ void st_any(void* p, dz_u32x4 v) {
-  *(dz_global_u32x4_any*)(uintptr_t)p = v;
-}
+// The same store without the hint, for results that the next kernel reads.
+__device__ __forceinline__ void st_any(void* p, dz_u32x4 v) { *(dz_global_u32x4*)(uintptr_t)p = v; }
 
 // Wave-uniform copy of a 32-bit value in a scalar register.
 // __builtin_amdgcn_readfirstlane returns a signed int: cast back to uint32_t
@@ -565,7 +565,7 @@ struct TileRegs {
 
 template <int DT, int MODE>
 __device__ __forceinline__ bool full_tile(const DzChunk& ch) {
-  return ch.n == (uint32_t)RmwTraits<DT, MODE>::kChunk && (ch.meta & kDzMetaAligned) != 0u;
+  return ch.n == (uint32_t)RmwTraits<DT, MODE>::kChunk;
 }
 
 // Lane layout of a full tile: a thread's groups of 8 elements are
@@ -743,22 +743,22 @@ __device__ __forceinline__ void compute_store_tile(const DzChunk& ch, const Tile
   }
 }
 
-// Partial or misaligned tile, bounds-checked: groups threadIdx.x,
-// threadIdx.x + 1024, ... of the tile. In a 16-byte-aligned tensor a group
-// with all 8 elements inside the tile goes through vector loads and stores
-// like a full tile's; the tensor's last, incomplete group and every group of
-// a misaligned view go element by element.
+// Partial tile (a tensor's last), bounds-checked: groups threadIdx.x,
+// threadIdx.x + 1024, ... of the tile. A group with all 8 elements inside the
+// tile goes through vector loads and stores like a full tile's; the tensor's
+// last, incomplete group goes element by element. (A loop over the groups: with
+// the loop unrolled and all loads issued first, the compiler scheduled the full
+// tiles' code worse, 0.4-1 % in the long passes.)
 template <int DT, int MODE>
 __device__ __forceinline__ void rmw_partial(const DzChunk& ch, const typename RmwTraits<DT, MODE>::E* tab,
                                             const DzScalars& sc) {
   using S = typename DT_<DT>::S;
   constexpr bool kTwoSeeds = MODE == kModeRestoreUpdatePerturb;
   char* base = (char*)ch.ptr;
-  const bool aligned = (ch.meta & kDzMetaAligned) != 0u;
   for (uint32_t g = threadIdx.x; g * 8u < ch.n; g += kRmwThreads) {
     const DzU4 w = dz_philox_group(sc.seed, kDzStreamParam, ch.zgroup + g);
     const DzU4 w2 = kTwoSeeds ? dz_philox_group(sc.seed2, kDzStreamParam, ch.zgroup + g) : w;
-    if (aligned && (g + 1u) * 8u <= ch.n) {
+    if ((g + 1u) * 8u <= ch.n) {
       if constexpr (DT == DZ_F32) {
         char* p = base + (size_t)g * 32;
         const dz_u32x4 a = ld_stream(p), b = ld_stream(p + 16);
@@ -806,7 +806,7 @@ __device__ __forceinline__ void rmw_partial(const DzChunk& ch, const typename Rm
 // workgroups on every XCD; wave 0 keeps a ring in LDS (while tile k streams,
 // the index of tile k+3 is taken and the descriptor of tile k+2 is loaded,
 // with scalar loads) and a barrier ends each tile. The chunk list holds its
-// full, aligned tiles first. The last workgroup to finish resets the
+// full tiles first. The last workgroup to finish resets the
 // counters for the next launch.
 //
 // Two tile loops: the plain loop (rmw_tiles) loads each tile when its turn

@@ -121,6 +121,35 @@ def test_rmw_uses_exported_z(dt):
 
 
 @pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("prefetch", [True, False])
+@pytest.mark.parametrize("first", [1, 3, 7])
+def test_packed_odd_tensors_match_oracle(dt, prefetch, first):
+    """Tensors of odd sizes end to end in one buffer, from every kind of start address, full tiles
+    among them: every pass against the oracle, and the elements around the tensors untouched."""
+    sizes = [1, 7, 24576 + 5, 8193, 2 * 32768 + 1, 3, 32768, 999]
+    buf = torch.full((first + sum(sizes) + 9,), 3.0, dtype=DT_TORCH[dt], device="cuda")
+    tensors, host, at = [], [], first
+    for i, n in enumerate(sizes):
+        bits = random_theta(n, dt, 900 + i)
+        buf[at:at + n] = to_torch(bits, dt, "cuda")
+        tensors.append(buf[at:at + n])
+        host.append(bits)
+        at += n
+    tab = _fused_table(tensors, prefetch)
+    s1, s2, eps, g, lr = 5, 6, 1e-3, 0.75, 1e-3
+    tab.perturb(s1, -2.0, eps)
+    tab.restore_update_perturb(s1, s2, eps, g, lr)
+    tab.restore_update(s2, eps, g, lr)
+    tab.update(s1, g, lr)
+    for i, (t, h, z1, z2) in enumerate(zip(tensors, host, _z_host(tab, s1, dt), _z_host(tab, s2, dt))):
+        h = A.perturb(A.restore_update(A.perturb(h, z1, -2, eps, dt), z1, eps, g, lr, dt), z2, 1, eps, dt)
+        h = A.update(A.restore_update(h, z2, eps, g, lr, dt), z1, g, lr, dt)
+        assert_bits_equal(to_bits(t), h, dt, f"tensor {i}")
+    assert bool((buf[:first] == 3.0).all()) and bool((buf[at:] == 3.0).all())
+    tab.close()
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("scale", [1.0, -2.0, 0.5])
 def test_perturb_matches_oracle(dt, scale):
     from dizo_amd.table import ZOTable
