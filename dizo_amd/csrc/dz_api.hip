@@ -223,6 +223,10 @@ struct dz_table {
   uint32_t fused_elems = 0;
   uint32_t fused_nchunks = 0;
   DzChunk* d_fused_chunks = nullptr;
+  // short ZO tables: the tile list of their launches (empty in longer tables)
+  bool persistent_only = false;  // set by dz_table_set_prefetch_min_tiles
+  uint32_t short_nchunks = 0;
+  DzChunk* d_short_chunks = nullptr;
   uint32_t* d_group_begin = nullptr;
   double* d_partials = nullptr;
   uint32_t* d_counters = nullptr;  // work counters of the persistent RMW / projection kernels
@@ -268,6 +272,7 @@ int32_t check_table(const dz_table* t) {
 void free_table(dz_table* t) {
   if (t->d_chunks) (void)hipFree(t->d_chunks);
   if (t->d_fused_chunks) (void)hipFree(t->d_fused_chunks);
+  if (t->d_short_chunks) (void)hipFree(t->d_short_chunks);
   if (t->d_group_begin) (void)hipFree(t->d_group_begin);
   if (t->d_partials) (void)hipFree(t->d_partials);
   if (t->d_counters) (void)hipFree(t->d_counters);
@@ -304,6 +309,13 @@ int32_t rmw(dz_table* t, int mode, const dz::DzScalars& s, const dz::DzScalarPtr
   if (rc) return rc;
   const dz::LaunchEvents ev = take_timing(t);
   if (t->projection) return fail(DZ_ERR_INVALID, "perturb/update need a ZO table (created without anchors)");
+  if (t->short_nchunks > 0 && !t->persistent_only) {
+    const hipError_t e = dz::launch_rmw_short(t->dtype, mode, t->d_short_chunks, t->short_nchunks,
+                                              (uint32_t)t->dev->cus, t->dev->tab[t->dtype], s, p,
+                                              (hipStream_t)stream, ev);
+    if (e != hipSuccess) return hip_fail(e, "rmw kernel launch");
+    return DZ_OK;
+  }
   // the tile list whose tile size the launch's kernel takes
   const uint32_t want = (uint32_t)dz::rmw_chunk_elems(t->dtype, mode);
   const DzChunk* chunks = t->d_chunks;
@@ -566,6 +578,14 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     t->fused_nchunks = (uint32_t)fc.size();
     e = upload_chunks(fc, &t->d_fused_chunks);
   }
+  uint64_t elems = 0;
+  for (int64_t ne : t->numels) elems += (uint64_t)ne;
+  if (e == hipSuccess && !t->projection && elems <= dz::short_elems(dtype)) {
+    std::vector<DzChunk> sc;
+    build_chunks(t, dz::kShortTile, &sc, nullptr);
+    t->short_nchunks = (uint32_t)sc.size();
+    e = upload_chunks(sc, &t->d_short_chunks);
+  }
   if (e == hipSuccess && t->projection) {
     // The finalize kernel always runs, so these exist even with no chunks.
     e = hipMalloc(&t->d_group_begin, t->group_begin.size() * sizeof(uint32_t));
@@ -620,6 +640,7 @@ int32_t dz_table_set_prefetch_min_tiles(dz_table* t, uint32_t min_tiles) {
   int32_t rc = check_table(t);
   if (rc) return rc;
   t->prefetch_min_tiles = min_tiles;
+  t->persistent_only = true;
   return DZ_OK;
 }
 

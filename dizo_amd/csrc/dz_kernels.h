@@ -57,6 +57,15 @@ __host__ __device__ constexpr int rmw_chunk_elems(int dtype, int mode) {
   return kRmwThreads * rmw_groups(dtype, mode) * 8;
 }
 
+// Short tables: up to short_elems(dtype) elements in all, whose passes run
+// rmw_short_kernel over tiles of kShortTile elements. Where the line lies: the
+// two passes of a steady step, against the persistent kernel with plain
+// accesses (what tables just above the line run best): fp16 2^24 elements 32.6
+// and 41.5 us, 2^25 53.0 and 52.2, 2^26 96.7 and 87.5; fp32 2^23 25.4 and 31.6,
+// 2^24 46.2 and 46.4, 2^25 84.4 and 80.4.
+constexpr uint32_t kShortTile = kRmwThreads * 8;
+constexpr uint64_t short_elems(int dtype) { return dtype == DZ_F32 ? 1u << 24 : 1u << 25; }
+
 // LDS bytes of the per-launch delta table of an RMW launch: 16-bit entries
 // for perturb/update of 16-bit T, 32-bit entries otherwise (fp32 deltas, or
 // the (restore delta, update delta) pair of a fused restore+update).
@@ -148,6 +157,10 @@ struct LaunchEvents {
 hipError_t launch_rmw(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t grid,
                       const void* qtab, const DzScalars& s, const DzScalarPtrs& p, uint32_t* counters,
                       bool prefetch, hipStream_t st, const LaunchEvents& ev = {});
+// Launches of short tables, over tiles of kShortTile elements.
+hipError_t launch_rmw_short(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t cus,
+                            const void* qtab, const DzScalars& s, const DzScalarPtrs& p, hipStream_t st,
+                            const LaunchEvents& ev = {});
 // Persistent: `grid` workgroups share the chunks through `counters` (zero
 // before the launch; the launch leaves them at zero).
 hipError_t launch_proj(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t ngroups,

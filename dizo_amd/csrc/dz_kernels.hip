@@ -459,7 +459,9 @@ __device__ __forceinline__ dz_u32x4 ld_stream(const void* p) {
 __device__ __forceinline__ void st_stream(void* p, dz_u32x4 v) {
   __builtin_nontemporal_store(v, (dz_global_u32x4*)(uintptr_t)p);
 }
-// The same store without the hint, for results that the next kernel reads.
+// The same accesses without the hint, for data that the Infinity Cache holds
+// from one kernel to the next.
+__device__ __forceinline__ dz_u32x4 ld_any(const void* p) { return *(const dz_global_u32x4*)(uintptr_t)p; }
 __device__ __forceinline__ void st_any(void* p, dz_u32x4 v) { *(dz_global_u32x4*)(uintptr_t)p = v; }
 
 // Wave-uniform copy of a 32-bit value in a scalar register.
@@ -1084,6 +1086,199 @@ __global__ void __launch_bounds__(kRmwThreads, kRmwWavesPerEU) rmw_kernel(const 
 }
 
 // ---------------------------------------------------------------------------
+// Read-modify-write launches of short tables. The persistent kernel above pays
+// for its work counters, its descriptor ring and its delta table (3 to 10 us),
+// which a pass over a few million elements does not earn back. Here workgroups
+// of 1024 threads take tiles of 8 elements per thread in a fixed order (tile
+// blockIdx.x, then every gridDim.x-th), the quantile table is copied to LDS as
+// it is, and the deltas are evaluated for each pair of elements with the same
+// operations that the delta tables' entries take. The accesses are plain ones:
+// what a short pass writes stays in the 256 MB Infinity Cache for the forward
+// and the next pass (with the non-temporal hint, fp32, 2^24 elements: 30.5
+// against 22.6 us). Pass times in us (perturb / three-way), this kernel and the
+// persistent one with its hints: fp16 2^14 elements 4.0 / 4.1 and 6.8 / 9.0,
+// 2^20 4.3 / 4.4 and 10.2 / 14.3, 2^22 6.1 / 7.7 and 13.1 / 19.5, 2^25 22.2 /
+// 30.8 and 27.2 / 30.3; fp32 2^20 4.6 / 5.4 and 9.9 / 10.4, 2^24 22.7 / 23.5
+// and 27.6 / 28.2. A launch is bound by its latencies (about 4 us) up to 2^20
+// elements, then by the lookups (two in the three-way pass: about 8 clocks a
+// wave and lookup, which 2^25 elements' 30 us are) and the cache.
+// ---------------------------------------------------------------------------
+
+// The two 16-bit lanes of a packed word as fp32, and two fp32 values rounded
+// to T and packed: one conversion instruction each way.
+struct F32Pair {
+  float lo, hi;
+};
+template <int DT>
+__device__ __forceinline__ F32Pair widen_pair(uint32_t x) {
+  return F32Pair{DT_<DT>::to_f(x & 0xffffu), DT_<DT>::to_f(x >> 16)};
+}
+template <int DT>
+__device__ __forceinline__ uint32_t round_pair(float lo, float hi) {
+  if constexpr (DT == DZ_F16) {
+    const dz_half2 r = {(_Float16)dz_opq(lo), (_Float16)dz_opq(hi)};
+    return __builtin_bit_cast(uint32_t, r);
+  } else {
+    return pack_bf16(dz_opq(lo), dz_opq(hi));
+  }
+}
+// b = R(R(s z) eps) of two packed signed z. kUnit: s is 1 (the fused modes'
+// perturbations), so R(s z) is z.
+template <int DT, bool kUnit>
+__device__ __forceinline__ uint32_t delta_b_pair(uint32_t z, const DzScalars& sc) {
+  F32Pair a = widen_pair<DT>(z);
+  if constexpr (!kUnit) a = widen_pair<DT>(round_pair<DT>(sc.scale * a.lo, sc.scale * a.hi));
+  return round_pair<DT>(a.lo * sc.eps, a.hi * sc.eps);
+}
+// -d = -R(lr R(g z)) of two packed signed z.
+template <int DT>
+__device__ __forceinline__ uint32_t delta_nd_pair(uint32_t z, const DzScalars& sc) {
+  const F32Pair a = widen_pair<DT>(z);
+  const F32Pair c = widen_pair<DT>(round_pair<DT>(sc.grad * a.lo, sc.grad * a.hi));
+  return round_pair<DT>(sc.lr * c.lo, sc.lr * c.hi) ^ 0x80008000u;
+}
+// The launch's operation on two packed 16-bit elements with their signed z
+// (and next step's z).
+template <int DT, int MODE>
+__device__ __forceinline__ uint32_t apply_z_pair(uint32_t th, uint32_t z, uint32_t z2, const DzScalars& sc) {
+  if constexpr (MODE == kModeUpdate) return add_pair<DT>(th, delta_nd_pair<DT>(z, sc));
+  uint32_t r = add_pair<DT>(th, delta_b_pair<DT, rmw_pair_mode(MODE)>(z, sc));
+  if constexpr (rmw_pair_mode(MODE)) r = add_pair<DT>(r, delta_nd_pair<DT>(z, sc));
+  if constexpr (MODE == kModeRestoreUpdatePerturb) r = add_pair<DT>(r, delta_b_pair<DT, true>(z2, sc));
+  return r;
+}
+// The launch's operation on one fp32 element with its signed z.
+template <int MODE>
+__device__ __forceinline__ uint32_t apply_z_f32(uint32_t th, uint32_t z, uint32_t z2, const DzScalars& sc) {
+  const float zf = __uint_as_float(z);
+  if constexpr (MODE == kModePerturb) return op_perturb<DZ_F32>(__uint_as_float(th), zf, sc.scale, sc.eps);
+  if constexpr (MODE == kModeUpdate) return op_update<DZ_F32>(__uint_as_float(th), zf, sc.grad, sc.lr);
+  uint32_t r = op_perturb<DZ_F32>(__uint_as_float(th), zf, 1.0f, sc.eps);
+  r = op_update<DZ_F32>(__uint_as_float(r), zf, sc.grad, sc.lr);
+  if constexpr (MODE == kModeRestoreUpdatePerturb)
+    r = op_perturb<DZ_F32>(__uint_as_float(r), __uint_as_float(z2), 1.0f, sc.eps);
+  return r;
+}
+
+// The eight z of a Philox block in T, from a quantile table `tab` of T (in LDS
+// or in memory): 16-bit T packed into one vector, fp32 into two.
+template <int DT>
+struct ZVec {
+  static constexpr int kVecs = DT == DZ_F32 ? 2 : 1;
+  dz_u32x4 v[kVecs];
+};
+template <int DT>
+__device__ __forceinline__ ZVec<DT> z_vec(const typename DT_<DT>::S* tab, const DzU4& w) {
+  ZVec<DT> r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t x = word_of(w, i);
+    uint32_t e0, e1;
+    lookup2(tab, x, e0, e1);
+    if constexpr (DT == DZ_F32) {
+      r.v[i >> 1][2 * (i & 1)] = e0 | ((x & 0x8000u) << 16);
+      r.v[i >> 1][2 * (i & 1) + 1] = e1 | (x & 0x80000000u);
+    } else {
+      r.v[0][i] = (e0 | (e1 << 16)) | (x & 0x80008000u);
+    }
+  }
+  return r;
+}
+
+// A thread's group of 8 elements of a short table's tile.
+template <int DT>
+struct ShortGroup {
+  using S = typename DT_<DT>::S;
+  static constexpr int kVecs = ZVec<DT>::kVecs;
+  char* p;      // its first element
+  uint32_t n;   // elements of it inside the tile (0: none)
+  dz_u32x4 v[kVecs];
+
+  __device__ __forceinline__ ShortGroup() {}
+  __device__ __forceinline__ explicit ShortGroup(const DzChunk& ch) {
+    p = (char*)ch.ptr + (size_t)threadIdx.x * (8 * sizeof(S));
+    const uint32_t first = threadIdx.x * 8u;
+    n = first < ch.n ? min(ch.n - first, 8u) : 0u;
+    if (n == 8u) {
+#pragma unroll
+      for (int k = 0; k < kVecs; ++k) v[k] = ld_any(p + 16 * k);
+    } else if (n > 0u) {  // the tensor's last elements
+#pragma unroll
+      for (int j = 0; j < 8; ++j) set(j, (uint32_t)j < n ? (uint32_t)((const S*)p)[j] : 0u);
+    }
+  }
+  __device__ __forceinline__ void set(int j, uint32_t x) {
+    if constexpr (DT == DZ_F32)
+      v[j >> 2][j & 3] = x;
+    else
+      v[0][j >> 1] = j & 1 ? v[0][j >> 1] | (x << 16) : x;
+  }
+  __device__ __forceinline__ void store() const {
+    if (n == 8u) {
+#pragma unroll
+      for (int k = 0; k < kVecs; ++k) st_any(p + 16 * k, v[k]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t x = DT == DZ_F32 ? v[DT == DZ_F32 ? j >> 2 : 0][j & 3] : v[0][j >> 1] >> (16 * (j & 1));
+        if ((uint32_t)j < n) ((S*)p)[j] = (S)x;
+      }
+    }
+  }
+};
+
+template <int DT, int MODE>
+__global__ void __launch_bounds__(kRmwThreads, DT == DZ_F32 ? 4 : 8)
+    rmw_short_kernel(const DzChunk* __restrict__ chunks, uint32_t nchunks, const void* __restrict__ qtab,
+                     DzScalars sc_in, DzScalarPtrs sp) {
+  using S = typename DT_<DT>::S;
+  constexpr bool kNext = MODE == kModeRestoreUpdatePerturb;
+  constexpr int kSlices = kDzTabEntries * (int)sizeof(S) / (16 * kRmwThreads);
+  __shared__ __attribute__((aligned(16))) S tab[kDzTabEntries];
+  uint32_t t = blockIdx.x;
+  DzChunk ch = chunks[t];
+  ShortGroup<DT> cur(ch);  // in flight while the table is copied
+  {
+    dz_u32x4 q[kSlices];
+#pragma unroll
+    for (int k = 0; k < kSlices; ++k)
+      q[k] = *(const dz_u32x4*)((const char*)qtab + (size_t)(k * kRmwThreads + threadIdx.x) * 16);
+#pragma unroll
+    for (int k = 0; k < kSlices; ++k) *(dz_u32x4*)((char*)tab + (size_t)(k * kRmwThreads + threadIdx.x) * 16) = q[k];
+  }
+  const DzScalars sc = resolve_scalars<DT>(sc_in, sp);
+  __syncthreads();
+  for (;;) {
+    const uint64_t q = ch.zgroup + threadIdx.x;
+    const uint32_t tn = t + gridDim.x;
+    const bool more = tn < nchunks;
+    ShortGroup<DT> nxt;
+    if (more) {
+      ch = chunks[tn];
+      nxt = ShortGroup<DT>(ch);
+    }
+    if (cur.n > 0u) {
+      const ZVec<DT> z = z_vec<DT>(tab, dz_philox_group(sc.seed, kDzStreamParam, q));
+      const ZVec<DT> z2 = kNext ? z_vec<DT>(tab, dz_philox_group(sc.seed2, kDzStreamParam, q)) : z;
+#pragma unroll
+      for (int k = 0; k < ZVec<DT>::kVecs; ++k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (DT == DZ_F32)
+            cur.v[k][i] = apply_z_f32<MODE>(cur.v[k][i], z.v[k][i], z2.v[k][i], sc);
+          else
+            cur.v[k][i] = apply_z_pair<DT, MODE>(cur.v[k][i], z.v[k][i], z2.v[k][i], sc);
+        }
+      }
+      cur.store();
+    }
+    if (!more) break;
+    t = tn;
+    cur = nxt;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Projection kernels over the projected (k/v) tensors, one group per tensor.
 //   SUMSQ          partial[c] = sum over chunk of fp32(R_T(theta - theta0))^2
 //   APPLY          theta <- R_T(R_T(R_T(theta - theta0) * alpha) + theta0)   trainer.py:428-436
@@ -1490,31 +1685,6 @@ __global__ void __launch_bounds__(256) static_plan_kernel(StaticPlanBatch b, DzC
   }
 }
 
-// The eight z of a Philox block in T, from a quantile table `tab` of T (in LDS
-// or in memory): 16-bit T packed into one vector, fp32 into two.
-template <int DT>
-struct ZVec {
-  static constexpr int kVecs = DT == DZ_F32 ? 2 : 1;
-  dz_u32x4 v[kVecs];
-};
-template <int DT>
-__device__ __forceinline__ ZVec<DT> z_vec(const typename DT_<DT>::S* tab, const DzU4& w) {
-  ZVec<DT> r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t x = word_of(w, i);
-    uint32_t e0, e1;
-    lookup2(tab, x, e0, e1);
-    if constexpr (DT == DZ_F32) {
-      r.v[i >> 1][2 * (i & 1)] = e0 | ((x & 0x8000u) << 16);
-      r.v[i >> 1][2 * (i & 1) + 1] = e1 | (x & 0x80000000u);
-    } else {
-      r.v[0][i] = (e0 | (e1 << 16)) | (x & 0x80008000u);
-    }
-  }
-  return r;
-}
-
 // The launch's range of z: n elements from element `offset` of the stream, so
 // group g (8 elements, one Philox block) covers outputs 8 g - skip .. 8 g -
 // skip + 7 for skip = offset mod 8. Element indices wrap modulo 2^64.
@@ -1657,6 +1827,41 @@ hipError_t launch_rmw(int dtype, int mode, const DzChunk* chunks, uint32_t nchun
       return launch_rmw_dt<DZ_F16>(mode, chunks, nchunks, grid, tab, s, p, counters, prefetch, st, ev);
     case DZ_BF16:
       return launch_rmw_dt<DZ_BF16>(mode, chunks, nchunks, grid, tab, s, p, counters, prefetch, st, ev);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int DT>
+static hipError_t launch_rmw_short_dt(int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t cus, const void* tab,
+                                      const DzScalars& s, const DzScalarPtrs& p, hipStream_t st,
+                                      const LaunchEvents& ev) {
+  const uint32_t most = cus * (DT == DZ_F32 ? 1u : 2u);  // workgroups that the LDS tables leave room for
+  const dim3 grid(nchunks < most ? nchunks : most), block(kRmwThreads);
+  switch (mode) {
+    case kModePerturb:
+      DZ_LAUNCH((rmw_short_kernel<DT, kModePerturb>), grid, block, st, ev, chunks, nchunks, tab, s, p);
+      break;
+    case kModeUpdate:
+      DZ_LAUNCH((rmw_short_kernel<DT, kModeUpdate>), grid, block, st, ev, chunks, nchunks, tab, s, p);
+      break;
+    case kModeRestoreUpdate:
+      DZ_LAUNCH((rmw_short_kernel<DT, kModeRestoreUpdate>), grid, block, st, ev, chunks, nchunks, tab, s, p);
+      break;
+    case kModeRestoreUpdatePerturb:
+      DZ_LAUNCH((rmw_short_kernel<DT, kModeRestoreUpdatePerturb>), grid, block, st, ev, chunks, nchunks, tab, s, p);
+      break;
+    default:
+      return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_rmw_short(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t cus, const void* tab,
+                            const DzScalars& s, const DzScalarPtrs& p, hipStream_t st, const LaunchEvents& ev) {
+  switch (dtype) {
+    case DZ_F32: return launch_rmw_short_dt<DZ_F32>(mode, chunks, nchunks, cus, tab, s, p, st, ev);
+    case DZ_F16: return launch_rmw_short_dt<DZ_F16>(mode, chunks, nchunks, cus, tab, s, p, st, ev);
+    case DZ_BF16: return launch_rmw_short_dt<DZ_BF16>(mode, chunks, nchunks, cus, tab, s, p, st, ev);
     default: return hipErrorInvalidValue;
   }
 }

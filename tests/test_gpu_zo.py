@@ -150,6 +150,34 @@ def test_packed_odd_tensors_match_oracle(dt, prefetch, first):
 
 
 @pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("elems", [8192 * 256 - 3, 8192 * 1500 + 77, 2**24])
+def test_short_tables_match_the_persistent_kernel(dt, elems):
+    """Tables below the short-table line, with one to six tiles per workgroup and odd tensors among
+    them, across a wrap of the z counter's low word: every pass gives the persistent kernel's bits
+    (which the other tests hold against the oracle)."""
+    from dizo_amd.table import ZOTable
+    cut = [elems // 3 + 1, 5, elems // 2 + 3]
+    sizes = cut + [elems - sum(cut)]
+    gen = torch.Generator(device="cuda").manual_seed(elems)
+    start = (torch.randn(elems, device="cuda", generator=gen) * 0.02).to(DT_TORCH[dt])
+    offs, z = [], 2**35 - 8 * (elems // 16)
+    for n in sizes:
+        offs.append(z)
+        z += (n + 7) // 8 * 8
+    out = []
+    for short in (True, False):
+        flat = start.clone()
+        tab = ZOTable(list(flat.split(sizes)), z_offsets=offs) if short else _fused_table(list(flat.split(sizes)), True, z_offsets=offs)
+        tab.perturb(1, -2.0, 1e-3)
+        tab.restore_update_perturb(1, 2, 1e-3, 0.3, 1e-2)
+        tab.restore_update(2, 1e-3, -0.7, 1e-2)
+        tab.update(3, 1.25, 1e-2)
+        out.append(to_bits(flat))
+        tab.close()
+    assert_bits_equal(out[0], out[1], dt, f"{elems} elements")
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("scale", [1.0, -2.0, 0.5])
 def test_perturb_matches_oracle(dt, scale):
     from dizo_amd.table import ZOTable
