@@ -213,6 +213,7 @@ struct dz_table {
   bool projection = false;
   int32_t n = 0;
   uint32_t chunk_elems = 0;  // tile size (elements)
+  uint64_t bytes = 0;        // of the registered tensors (theta)
   uint32_t nchunks = 0;      // ZO tables: full tiles first (the prefetching loop runs them)
   std::vector<uint64_t> ptrs, aux, zoff;
   std::vector<int64_t> numels;
@@ -327,7 +328,8 @@ int32_t rmw(dz_table* t, int mode, const dz::DzScalars& s, const dz::DzScalarPtr
   }
   if (ntiles == 0) return record_unlaunched(ev, stream);
   hipError_t e = dz::launch_rmw(t->dtype, mode, chunks, ntiles, rmw_grid(t, ntiles), t->dev->tab[t->dtype], s, p,
-                                t->d_counters, ntiles >= t->prefetch_min_tiles, (hipStream_t)stream, ev);
+                                t->d_counters, ntiles >= t->prefetch_min_tiles,
+                                t->bytes <= dz::kPlainBytes, (hipStream_t)stream, ev);
   if (e != hipSuccess) return hip_fail(e, "rmw kernel launch");
   return DZ_OK;
 }
@@ -578,9 +580,8 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     t->fused_nchunks = (uint32_t)fc.size();
     e = upload_chunks(fc, &t->d_fused_chunks);
   }
-  uint64_t elems = 0;
-  for (int64_t ne : t->numels) elems += (uint64_t)ne;
-  if (e == hipSuccess && !t->projection && elems <= dz::short_elems(dtype)) {
+  for (int64_t ne : t->numels) t->bytes += (uint64_t)ne * es;
+  if (e == hipSuccess && !t->projection && t->bytes <= dz::short_elems(dtype) * es) {
     std::vector<DzChunk> sc;
     build_chunks(t, dz::kShortTile, &sc, nullptr);
     t->short_nchunks = (uint32_t)sc.size();

@@ -66,6 +66,16 @@ __host__ __device__ constexpr int rmw_chunk_elems(int dtype, int mode) {
 constexpr uint32_t kShortTile = kRmwThreads * 8;
 constexpr uint64_t short_elems(int dtype) { return dtype == DZ_F32 ? 1u << 24 : 1u << 25; }
 
+// Tensors of up to kPlainBytes in all, the size of the Infinity Cache, are read
+// and written with plain accesses by the persistent kernel; longer tables'
+// accesses carry the non-temporal hint. Pass times in us (perturb / three-way)
+// with the hint and without, three tables used in turn: fp16 2^26 elements (128
+// MB) 47.0 / 51.0 and 47.3 / 45.7, 2^27 87.5 / 91.6 and 82.9 / 84.7, 2^27.25
+// 104 / 110 and 113 / 115, 2^28 169 / 173 and 183 / 185; fp32 2^25 50.7 / 49.6
+// and 43.6 / 40.7, 2^26 (256 MB) 94.7 / 92.6 and 79.2 / 78.3, 2^26.5 130 / 127
+// and 129 / 126, 2^29 701 / 718 and 727 / 744.
+constexpr uint64_t kPlainBytes = 1u << 28;
+
 // LDS bytes of the per-launch delta table of an RMW launch: 16-bit entries
 // for perturb/update of 16-bit T, 32-bit entries otherwise (fp32 deltas, or
 // the (restore delta, update delta) pair of a fused restore+update).
@@ -156,7 +166,7 @@ struct LaunchEvents {
 // allows it (rmw_prefetch_mode); the caller sets it for long launches.
 hipError_t launch_rmw(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t grid,
                       const void* qtab, const DzScalars& s, const DzScalarPtrs& p, uint32_t* counters,
-                      bool prefetch, hipStream_t st, const LaunchEvents& ev = {});
+                      bool prefetch, bool plain, hipStream_t st, const LaunchEvents& ev = {});
 // Launches of short tables, over tiles of kShortTile elements.
 hipError_t launch_rmw_short(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t cus,
                             const void* qtab, const DzScalars& s, const DzScalarPtrs& p, hipStream_t st,

@@ -577,18 +577,28 @@ __device__ __forceinline__ bool full_tile(const DzChunk& ch) {
 // or i / 2 (fp32, two vectors per group). A tile holds at most 64 KB. The
 // offsets are loop-invariant 64-bit values, so each access adds one to the
 // tile's base (one v_lshl_add_u64).
-template <int DT, int MODE>
-struct TileOffsets {
+//
+// kPlain: plain loads and stores, else streaming (non-temporal) ones (see
+// kPlainBytes for which launches take which).
+template <int DT, int MODE, bool kPlain>
+struct TileAccess {
   __device__ __forceinline__ size_t at(int i) const {
     const size_t g0 = threadIdx.x;
     return DT != DZ_F32 ? (g0 + (size_t)i * kRmwThreads) * 16 : (g0 + (size_t)(i >> 1) * kRmwThreads) * 32 + (size_t)(i & 1) * 16;
   }
+  __device__ __forceinline__ dz_u32x4 load(const void* p) const { return kPlain ? ld_any(p) : ld_stream(p); }
+  __device__ __forceinline__ void store(void* p, dz_u32x4 v) const {
+    if constexpr (kPlain)
+      st_any(p, v);
+    else
+      st_stream(p, v);
+  }
 };
 
-template <int DT, int MODE>
-__device__ __forceinline__ void load_tile_at(uint64_t addr, const TileOffsets<DT, MODE>& to, TileRegs<DT, MODE>& r) {
+template <int DT, int MODE, class Access>
+__device__ __forceinline__ void load_tile_at(uint64_t addr, const Access& to, TileRegs<DT, MODE>& r) {
 #pragma unroll
-  for (int i = 0; i < TileRegs<DT, MODE>::kVecs; ++i) r.v[i] = ld_stream((const char*)addr + to.at(i));
+  for (int i = 0; i < TileRegs<DT, MODE>::kVecs; ++i) r.v[i] = to.load((const char*)addr + to.at(i));
 }
 
 // Philox block of group threadIdx.x + u * 1024 of a tile: counter zgroup +
@@ -608,8 +618,8 @@ __device__ __forceinline__ DzU4 tile_block(const DzChunk& ch, uint64_t seed, int
 
 // Group u of a full fp32 tile with its z words w (and next-step words w2):
 // the launch's operation applied and the group stored.
-template <int DT, int MODE>
-__device__ __forceinline__ void apply_store_group32(uint64_t base, const TileOffsets<DT, MODE>& to,
+template <int DT, int MODE, class Access>
+__device__ __forceinline__ void apply_store_group32(uint64_t base, const Access& to,
                                                     const TileRegs<DT, MODE>& r, int u,
                                                     const DzU4& w, const DzU4& w2,
                                                     const typename RmwTraits<DT, MODE>::E* tab, const DzScalars& sc) {
@@ -623,8 +633,8 @@ __device__ __forceinline__ void apply_store_group32(uint64_t base, const TileOff
   o1.y = apply_one<DT, MODE>(b.y, w.z >> 16, w2.z >> 16, tab, sc);
   o1.z = apply_one<DT, MODE>(b.z, w.w & 0xffffu, w2.w & 0xffffu, tab, sc);
   o1.w = apply_one<DT, MODE>(b.w, w.w >> 16, w2.w >> 16, tab, sc);
-  st_stream((char*)base + to.at(2 * u), o0);
-  st_stream((char*)base + to.at(2 * u + 1), o1);
+  to.store((char*)base + to.at(2 * u), o0);
+  to.store((char*)base + to.at(2 * u + 1), o1);
 }
 
 // A thread's share of a full tile as one straight-line block: the Philox
@@ -649,8 +659,8 @@ __device__ __forceinline__ void apply_store_group32(uint64_t base, const TileOff
 // Issued at the start, the next tile's reads meet this tile's first stores in
 // the memory system (rocprofv3 counts 18 % fewer reads in flight and 2.7
 // times the L2 tag stalls per cycle of the perturb pass).
-template <int DT, int MODE, bool kUniformHi, bool kLoadNext = false>
-__device__ __forceinline__ void tile_body(const DzChunk& ch, const TileOffsets<DT, MODE>& to,
+template <int DT, int MODE, bool kUniformHi, bool kLoadNext = false, class Access>
+__device__ __forceinline__ void tile_body(const DzChunk& ch, const Access& to,
                                           const TileRegs<DT, MODE>& r,
                                           const typename RmwTraits<DT, MODE>::E* tab, const DzScalars& sc,
                                           uint64_t nptr = 0, TileRegs<DT, MODE>* nxt = nullptr) {
@@ -679,7 +689,7 @@ __device__ __forceinline__ void tile_body(const DzChunk& ch, const TileOffsets<D
       o.y = combine_pair16<DT, MODE>(r.v[u].y, w[u].y, w2[u].y, lookup_pair16<DT, MODE>(w[u].y, w2[u].y, tab));
       o.z = combine_pair16<DT, MODE>(r.v[u].z, w[u].z, w2[u].z, lookup_pair16<DT, MODE>(w[u].z, w2[u].z, tab));
       o.w = combine_pair16<DT, MODE>(r.v[u].w, w[u].w, w2[u].w, lookup_pair16<DT, MODE>(w[u].w, w2[u].w, tab));
-      st_stream((char*)base + to.at(u), o);
+      to.store((char*)base + to.at(u), o);
     }
     if constexpr (kLoadNext && kLoadAfter >= 0) {
       if (u == kLoadAfter) {
@@ -733,8 +743,8 @@ __device__ __forceinline__ DzChunk uniform_next_chunk(const DzChunk& c) {
 
 // Applies the launch's operation to a thread's share of a full tile, already
 // in registers, and stores it.
-template <int DT, int MODE>
-__device__ __forceinline__ void compute_store_tile(const DzChunk& ch, const TileOffsets<DT, MODE>& to,
+template <int DT, int MODE, class Access>
+__device__ __forceinline__ void compute_store_tile(const DzChunk& ch, const Access& to,
                                                    const TileRegs<DT, MODE>& r,
                                                    const typename RmwTraits<DT, MODE>::E* tab,
                                                    const DzScalars& sc) {
@@ -751,8 +761,8 @@ __device__ __forceinline__ void compute_store_tile(const DzChunk& ch, const Tile
 // last, incomplete group goes element by element. (A loop over the groups: with
 // the loop unrolled and all loads issued first, the compiler scheduled the full
 // tiles' code worse, 0.4-1 % in the long passes.)
-template <int DT, int MODE>
-__device__ __forceinline__ void rmw_partial(const DzChunk& ch, const typename RmwTraits<DT, MODE>::E* tab,
+template <int DT, int MODE, class Access>
+__device__ __forceinline__ void rmw_partial(const DzChunk& ch, const Access& to, const typename RmwTraits<DT, MODE>::E* tab,
                                             const DzScalars& sc) {
   using S = typename DT_<DT>::S;
   constexpr bool kTwoSeeds = MODE == kModeRestoreUpdatePerturb;
@@ -763,7 +773,7 @@ __device__ __forceinline__ void rmw_partial(const DzChunk& ch, const typename Rm
     if ((g + 1u) * 8u <= ch.n) {
       if constexpr (DT == DZ_F32) {
         char* p = base + (size_t)g * 32;
-        const dz_u32x4 a = ld_stream(p), b = ld_stream(p + 16);
+        const dz_u32x4 a = to.load(p), b = to.load(p + 16);
         dz_u32x4 o0, o1;
         o0.x = apply_one<DT, MODE>(a.x, w.x & 0xffffu, w2.x & 0xffffu, tab, sc);
         o0.y = apply_one<DT, MODE>(a.y, w.x >> 16, w2.x >> 16, tab, sc);
@@ -773,17 +783,17 @@ __device__ __forceinline__ void rmw_partial(const DzChunk& ch, const typename Rm
         o1.y = apply_one<DT, MODE>(b.y, w.z >> 16, w2.z >> 16, tab, sc);
         o1.z = apply_one<DT, MODE>(b.z, w.w & 0xffffu, w2.w & 0xffffu, tab, sc);
         o1.w = apply_one<DT, MODE>(b.w, w.w >> 16, w2.w >> 16, tab, sc);
-        st_stream(p, o0);
-        st_stream(p + 16, o1);
+        to.store(p, o0);
+        to.store(p + 16, o1);
       } else {
         char* p = base + (size_t)g * 16;
-        const dz_u32x4 v = ld_stream(p);
+        const dz_u32x4 v = to.load(p);
         dz_u32x4 o;
         o.x = combine_pair16<DT, MODE>(v.x, w.x, w2.x, lookup_pair16<DT, MODE>(w.x, w2.x, tab));
         o.y = combine_pair16<DT, MODE>(v.y, w.y, w2.y, lookup_pair16<DT, MODE>(w.y, w2.y, tab));
         o.z = combine_pair16<DT, MODE>(v.z, w.z, w2.z, lookup_pair16<DT, MODE>(w.z, w2.z, tab));
         o.w = combine_pair16<DT, MODE>(v.w, w.w, w2.w, lookup_pair16<DT, MODE>(w.w, w2.w, tab));
-        st_stream(p, o);
+        to.store(p, o);
       }
       continue;
     }
@@ -818,10 +828,10 @@ __device__ __forceinline__ void rmw_partial(const DzChunk& ch, const typename Rm
 // each tile's first group is stored, and hands the workgroup's remaining
 // tiles to rmw_tiles at its first tile that is not full.
 // ---------------------------------------------------------------------------
-template <int DT, int MODE, bool kTagged = false>
+template <int DT, int MODE, bool kTagged = false, class Access>
 __device__ __forceinline__ void rmw_tiles(uint32_t k0, const DzChunk* __restrict__ chunks, uint32_t nchunks,
                                           const typename RmwTraits<DT, MODE>::E* tab, const DzScalars& sc,
-                                          const TileOffsets<DT, MODE>& to, uint32_t* sidx, DzChunk* sdesc,
+                                          const Access& to, uint32_t* sidx, DzChunk* sdesc,
                                           uint32_t* mine, uint32_t ncnt, uint32_t j) {
   const uint64_t nch = nchunks;
   TileRegs<DT, MODE> cur;
@@ -853,7 +863,7 @@ __device__ __forceinline__ void rmw_tiles(uint32_t k0, const DzChunk* __restrict
       load_tile_at<DT, MODE>(ch.ptr, to, cur);
       compute_store_tile<DT, MODE>(ch, to, cur, tab, sc);
     } else {
-      rmw_partial<DT, MODE>(ch, tab, sc);
+      rmw_partial<DT, MODE>(ch, to, tab, sc);
     }
     if (threadIdx.x == 0) {
       sidx[(k + 3) % 4] = (uint32_t)min((uint64_t)grabbed * ncnt + j, nch);
@@ -902,11 +912,11 @@ __device__ __forceinline__ void wait_vm_all() { __builtin_amdgcn_s_waitcnt(0x0F7
 // bf16 pass measured 1.4 % faster on one box and 2-3 % slower on two others,
 // also with the next index carried from the step before so that those loads
 // go out with no LDS read ahead of them.
-template <int DT, int MODE>
+template <int DT, int MODE, class Access>
 __device__ __forceinline__ bool rmw_prefetch_step(uint32_t k, const DzChunk& ch, DzChunk& ch1,
                                                   const DzChunk* __restrict__ chunks, uint32_t nchunks,
                                                   const typename RmwTraits<DT, MODE>::E* tab, const DzScalars& sc,
-                                                  const TileOffsets<DT, MODE>& to, uint32_t* sidx, DzChunk* sdesc,
+                                                  const Access& to, uint32_t* sidx, DzChunk* sdesc,
                                                   uint32_t* mine, uint32_t ncnt, uint32_t j, const void* dummy,
                                                   bool wave0, const TileRegs<DT, MODE>& cur,
                                                   TileRegs<DT, MODE>& nxt) {
@@ -977,10 +987,10 @@ __device__ __forceinline__ bool rmw_prefetch_step(uint32_t k, const DzChunk& ch,
 // atomic; and the barrier orders LDS only. With those, the compiler's waits for a tile's
 // data count the operations behind it (the previous tile's stores and the
 // next tile's loads) instead of draining everything in flight.
-template <int DT, int MODE>
+template <int DT, int MODE, class Access>
 __device__ __forceinline__ uint32_t rmw_tiles_prefetch(const DzChunk* __restrict__ chunks, uint32_t nchunks,
                                                        const typename RmwTraits<DT, MODE>::E* tab,
-                                                       const DzScalars& sc, const TileOffsets<DT, MODE>& to,
+                                                       const DzScalars& sc, const Access& to,
                                                        uint32_t* sidx, DzChunk* sdesc, uint32_t* mine, uint32_t ncnt,
                                                        uint32_t j, const void* dummy) {
   const uint32_t c0 = rfl_u32(sidx[0]);
@@ -1025,7 +1035,7 @@ struct RmwShared {
 
 // kPF: run the prefetching tile loop over the workgroup's leading full tiles
 // (only where RmwTraits::kPrefetch allows it; the launcher picks it by size).
-template <int DT, int MODE, bool kPF>
+template <int DT, int MODE, bool kPF, bool kPlain>
 __global__ void __launch_bounds__(kRmwThreads, kRmwWavesPerEU) rmw_kernel(const DzChunk* __restrict__ chunks,
                                                                           uint32_t nchunks,
                                                                           const void* __restrict__ qtab,
@@ -1070,7 +1080,7 @@ __global__ void __launch_bounds__(kRmwThreads, kRmwWavesPerEU) rmw_kernel(const 
     }
   }
   store_table<DT, MODE>(tab, qs, sc);
-  const TileOffsets<DT, MODE> to{};
+  const TileAccess<DT, MODE, kPlain> to{};
   __syncthreads();
   uint32_t k0 = 0;
   if constexpr (Tr::kPrefetch && kPF)
@@ -1784,30 +1794,30 @@ __global__ void __launch_bounds__(256) philox_kernel(uint64_t seed, uint32_t str
     }                                                                                           \
   } while (0)
 
-template <int DT>
+template <int DT, bool kPlain>
 static hipError_t launch_rmw_dt(int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t grid,
                                 const void* tab, const DzScalars& s, const DzScalarPtrs& p,
                                 uint32_t* counters, bool prefetch, hipStream_t st, const LaunchEvents& ev) {
   switch (mode) {
     case kModePerturb:
-      DZ_LAUNCH((rmw_kernel<DT, kModePerturb, false>), dim3(grid), dim3(kRmwThreads), st, ev,
+      DZ_LAUNCH((rmw_kernel<DT, kModePerturb, false, kPlain>), dim3(grid), dim3(kRmwThreads), st, ev,
                          chunks, nchunks, tab, s, p, counters);
       break;
     case kModeUpdate:
-      DZ_LAUNCH((rmw_kernel<DT, kModeUpdate, false>), dim3(grid), dim3(kRmwThreads), st, ev,
+      DZ_LAUNCH((rmw_kernel<DT, kModeUpdate, false, kPlain>), dim3(grid), dim3(kRmwThreads), st, ev,
                          chunks, nchunks, tab, s, p, counters);
       break;
     case kModeRestoreUpdate:
-      DZ_LAUNCH((rmw_kernel<DT, kModeRestoreUpdate, false>), dim3(grid), dim3(kRmwThreads),
+      DZ_LAUNCH((rmw_kernel<DT, kModeRestoreUpdate, false, kPlain>), dim3(grid), dim3(kRmwThreads),
                          st, ev, chunks, nchunks, tab, s, p, counters);
       break;
     case kModeRestoreUpdatePerturb:
       // the caller asks for the prefetching loop on long launches (the table's prefetch_min_tiles)
       if (RmwTraits<DT, kModeRestoreUpdatePerturb>::kPrefetch && prefetch) {
-        DZ_LAUNCH((rmw_kernel<DT, kModeRestoreUpdatePerturb, true>), dim3(grid), dim3(kRmwThreads),
+        DZ_LAUNCH((rmw_kernel<DT, kModeRestoreUpdatePerturb, true, kPlain>), dim3(grid), dim3(kRmwThreads),
                            st, ev, chunks, nchunks, tab, s, p, counters);
       } else {
-        DZ_LAUNCH((rmw_kernel<DT, kModeRestoreUpdatePerturb, false>), dim3(grid), dim3(kRmwThreads),
+        DZ_LAUNCH((rmw_kernel<DT, kModeRestoreUpdatePerturb, false, kPlain>), dim3(grid), dim3(kRmwThreads),
                            st, ev, chunks, nchunks, tab, s, p, counters);
       }
       break;
@@ -1819,14 +1829,14 @@ static hipError_t launch_rmw_dt(int mode, const DzChunk* chunks, uint32_t nchunk
 
 hipError_t launch_rmw(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t grid,
                       const void* tab, const DzScalars& s, const DzScalarPtrs& p, uint32_t* counters,
-                      bool prefetch, hipStream_t st, const LaunchEvents& ev) {
+                      bool prefetch, bool plain, hipStream_t st, const LaunchEvents& ev) {
+  const auto go = [&](auto launch) {
+    return launch(mode, chunks, nchunks, grid, tab, s, p, counters, prefetch, st, ev);
+  };
   switch (dtype) {
-    case DZ_F32:
-      return launch_rmw_dt<DZ_F32>(mode, chunks, nchunks, grid, tab, s, p, counters, prefetch, st, ev);
-    case DZ_F16:
-      return launch_rmw_dt<DZ_F16>(mode, chunks, nchunks, grid, tab, s, p, counters, prefetch, st, ev);
-    case DZ_BF16:
-      return launch_rmw_dt<DZ_BF16>(mode, chunks, nchunks, grid, tab, s, p, counters, prefetch, st, ev);
+    case DZ_F32: return plain ? go(launch_rmw_dt<DZ_F32, true>) : go(launch_rmw_dt<DZ_F32, false>);
+    case DZ_F16: return plain ? go(launch_rmw_dt<DZ_F16, true>) : go(launch_rmw_dt<DZ_F16, false>);
+    case DZ_BF16: return plain ? go(launch_rmw_dt<DZ_BF16, true>) : go(launch_rmw_dt<DZ_BF16, false>);
     default: return hipErrorInvalidValue;
   }
 }

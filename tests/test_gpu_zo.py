@@ -178,6 +178,31 @@ def test_short_tables_match_the_persistent_kernel(dt, elems):
 
 
 @pytest.mark.parametrize("dt", DTS)
+def test_tables_around_the_cache_size_agree(dt):
+    """The same elements in a table of 256 MB (plain accesses), in one a little longer (streaming
+    accesses) and in slices below the short-table line: the same bits from every pass."""
+    from dizo_amd.table import ZOTable
+    n = 2**28 // DT_TORCH[dt].itemsize
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    start = torch.empty(n + 12345, dtype=DT_TORCH[dt], device="cuda").normal_(0.0, 0.02, generator=gen)
+
+    def run(lo, hi):
+        flat = start[lo:hi].clone()
+        tab = ZOTable([flat], z_offsets=[lo])
+        tab.perturb(1, -2.0, 1e-3)
+        tab.restore_update_perturb(1, 2, 1e-3, 0.3, 1e-2)
+        tab.restore_update(2, 1e-3, -0.7, 1e-2)
+        tab.update(3, 1.25, 1e-2)
+        tab.close()
+        return flat.view(torch.int32 if dt == F32 else torch.int16)
+
+    plain, streamed = run(0, n), run(0, n + 12345)
+    assert torch.equal(plain, streamed[:n])
+    for lo in (0, n // 2 + 8, n - 2**20):
+        assert torch.equal(plain[lo:lo + 2**20], run(lo, lo + 2**20)), lo
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("scale", [1.0, -2.0, 0.5])
 def test_perturb_matches_oracle(dt, scale):
     from dizo_amd.table import ZOTable
