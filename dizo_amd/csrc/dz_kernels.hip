@@ -152,22 +152,68 @@ __device__ __forceinline__ uint32_t field_xor(uint32_t h) {
   return rmw_index_xor(DT, MODE) ? (h & 0xffffu) : (h & 0x8000u);
 }
 
-// Table entry for z = +Q_T[i] (qbits = bits of Q_T[i]).
-template <int DT, int MODE>
-__device__ __forceinline__ uint32_t table_entry(uint32_t qbits, const DzScalars& sc) {
-  constexpr uint32_t kSign = DT == DZ_F32 ? 0x80000000u : 0x8000u;
-  const float z = DT_<DT>::to_f(qbits);
-  const float b = rt<DT>(rt<DT>(sc.scale * z) * sc.eps);
-  const float d = rt<DT>(sc.lr * rt<DT>(sc.grad * z));
-  if constexpr (MODE == kModePerturb) {
-    return DT_<DT>::from_f(b);
-  } else if constexpr (MODE == kModeUpdate) {
-    return DT_<DT>::from_f(d) ^ kSign;
-  } else if constexpr (DT == DZ_F32) {
-    return qbits;  // restore+update(+perturb) in fp32: z itself
+typedef _Float16 dz_half2 __attribute__((ext_vector_type(2)));
+typedef __bf16 dz_bf2 __attribute__((ext_vector_type(2)));
+
+// bf16 lanes of a packed word as fp32 (a bf16 value is the high half of its
+// fp32 bit pattern), and two fp32 values rounded to bf16 and packed by one
+// v_cvt_pk_bf16_f32 (round to nearest even, as torch converts fp32 to bf16).
+__device__ __forceinline__ float bf16_lo_f(uint32_t x) { return __uint_as_float(x << 16); }
+__device__ __forceinline__ float bf16_hi_f(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  const dz_bf2 r = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, r);
+}
+// Low (pack_lo) or high (pack_hi) 16-bit halves of two words, a's in the low
+// lane and b's in the high lane: one v_perm_b32.
+__device__ __forceinline__ uint32_t pack_lo(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x05040100u);
+}
+__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+
+// The two 16-bit lanes of a packed word as fp32, and two fp32 values rounded
+// to T and packed: one conversion instruction each way.
+struct F32Pair {
+  float lo, hi;
+};
+template <int DT>
+__device__ __forceinline__ F32Pair widen_pair(uint32_t x) {
+  return F32Pair{DT_<DT>::to_f(x & 0xffffu), DT_<DT>::to_f(x >> 16)};
+}
+template <int DT>
+__device__ __forceinline__ uint32_t round_pair(float lo, float hi) {
+  if constexpr (DT == DZ_F16) {
+    const dz_half2 r = {(_Float16)dz_opq(lo), (_Float16)dz_opq(hi)};
+    return __builtin_bit_cast(uint32_t, r);
   } else {
-    return DT_<DT>::from_f(b) | ((DT_<DT>::from_f(d) ^ kSign) << 16);
+    return pack_bf16(dz_opq(lo), dz_opq(hi));
   }
+}
+// b = R(R(s z) eps) of two packed signed z. kUnit: s is 1 (the fused modes'
+// perturbations), so R(s z) is z.
+template <int DT, bool kUnit>
+__device__ __forceinline__ uint32_t delta_b_pair(uint32_t z, const DzScalars& sc) {
+  F32Pair a = widen_pair<DT>(z);
+  if constexpr (!kUnit) a = widen_pair<DT>(round_pair<DT>(sc.scale * a.lo, sc.scale * a.hi));
+  return round_pair<DT>(a.lo * sc.eps, a.hi * sc.eps);
+}
+// -d = -R(lr R(g z)) of two packed signed z.
+template <int DT>
+__device__ __forceinline__ uint32_t delta_nd_pair(uint32_t z, const DzScalars& sc) {
+  const F32Pair a = widen_pair<DT>(z);
+  const F32Pair c = widen_pair<DT>(round_pair<DT>(sc.grad * a.lo, sc.grad * a.hi));
+  return round_pair<DT>(sc.lr * c.lo, sc.lr * c.hi) ^ 0x80008000u;
+}
+// fp32 table entry for z = +Q_T[i] (qbits = its bits): the launch's delta, or
+// for the pair modes z itself.
+template <int MODE>
+__device__ __forceinline__ uint32_t table_entry_f32(uint32_t qbits, const DzScalars& sc) {
+  const float z = __uint_as_float(qbits);
+  if constexpr (MODE == kModePerturb) return __float_as_uint((sc.scale * z) * sc.eps);
+  if constexpr (MODE == kModeUpdate) return __float_as_uint(sc.lr * (sc.grad * z)) ^ 0x80000000u;
+  return qbits;
 }
 
 typedef uint32_t dz_u32x4 __attribute__((ext_vector_type(4)));
@@ -177,7 +223,10 @@ typedef uint32_t dz_u32x4 __attribute__((ext_vector_type(4)));
 // entries; slice t + v * 1024), all loads in flight at once (load_table), then
 // writes the slices' entries to the same indices of the LDS table
 // (store_table). A plain loop of one 32-bit load, a wait and one LDS store
-// per entry costs 32 memory latencies in a row per launch.
+// per entry costs 32 memory latencies in a row per launch. 16-bit entries are
+// evaluated two at a time (one rounding conversion for both): entry by entry,
+// the three-way pass took 1 (fp16) to 2 us (bf16) longer, 40.3 against 38.2 us
+// at 2^25.5 bf16 elements.
 template <int DT>
 struct TableSlices {
   static constexpr int kPer = DT == DZ_F32 ? 4 : 8;  // Q_T entries per 16-byte slice
@@ -196,45 +245,44 @@ __device__ __forceinline__ void load_table(TableSlices<DT>& t, const void* qtab)
 template <int DT, int MODE>
 __device__ __forceinline__ void store_table(typename RmwTraits<DT, MODE>::E* tab, const TableSlices<DT>& t,
                                             const DzScalars& sc) {
-  using E = typename RmwTraits<DT, MODE>::E;
   constexpr int kPer = TableSlices<DT>::kPer;
 #pragma unroll
   for (int v = 0; v < TableSlices<DT>::kSlices; ++v) {
-    uint32_t e[kPer];
     const uint32_t i0 = (uint32_t)(v * kRmwThreads + threadIdx.x) * kPer;
+    dz_u32x4* dst = (dz_u32x4*)(tab + i0);
+    if constexpr (DT == DZ_F32) {
+      dz_u32x4 o;
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const uint32_t w = t.q[v][kPer == 4 ? i : i >> 1];
-      const uint32_t qb = kPer == 4 ? w : (i & 1 ? w >> 16 : w & 0xffffu);
-      e[i] = table_entry<DT, MODE>(qb, sc);
-      if constexpr (rmw_index_xor(DT, MODE)) e[i] ^= (i0 + i) * 0x10001u;
-    }
-    E* dst = tab + i0;
-    if constexpr (sizeof(E) == 4) {
+      for (int i = 0; i < 4; ++i) o[i] = table_entry_f32<MODE>(t.q[v][i], sc);
+      dst[0] = o;
+    } else if constexpr (!rmw_pair_mode(MODE)) {  // two 16-bit entries a word
+      dz_u32x4 o;
 #pragma unroll
-      for (int h = 0; h < kPer / 4; ++h) {
-        const dz_u32x4 o = {e[4 * h], e[4 * h + 1], e[4 * h + 2], e[4 * h + 3]};
-        *(dz_u32x4*)(dst + 4 * h) = o;
+      for (int i = 0; i < 4; ++i)
+        o[i] = MODE == kModePerturb ? delta_b_pair<DT, false>(t.q[v][i], sc) : delta_nd_pair<DT>(t.q[v][i], sc);
+      dst[0] = o;
+    } else {  // entries b | (-d) << 16
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        dz_u32x4 o;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const uint32_t q = t.q[v][2 * h + i];
+          const uint32_t b = delta_b_pair<DT, true>(q, sc), nd = delta_nd_pair<DT>(q, sc);
+          o[2 * i] = pack_lo(b, nd);
+          o[2 * i + 1] = pack_hi(b, nd);
+          if constexpr (rmw_index_xor(DT, MODE)) {
+            const uint32_t at = i0 + 4 * h + 2 * i;
+            o[2 * i] ^= at * 0x10001u;
+            o[2 * i + 1] ^= (at + 1) * 0x10001u;
+          }
+        }
+        dst[h] = o;
       }
-    } else {
-      const dz_u32x4 o = {e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-      *(dz_u32x4*)dst = o;
     }
   }
 }
 
-typedef _Float16 dz_half2 __attribute__((ext_vector_type(2)));
-typedef __bf16 dz_bf2 __attribute__((ext_vector_type(2)));
-
-// bf16 lanes of a packed word as fp32 (a bf16 value is the high half of its
-// fp32 bit pattern), and two fp32 values rounded to bf16 and packed by one
-// v_cvt_pk_bf16_f32 (round to nearest even, as torch converts fp32 to bf16).
-__device__ __forceinline__ float bf16_lo_f(uint32_t x) { return __uint_as_float(x << 16); }
-__device__ __forceinline__ float bf16_hi_f(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-  const dz_bf2 r = {(__bf16)lo, (__bf16)hi};
-  return __builtin_bit_cast(uint32_t, r);
-}
 // R_bf16(a + b) lane by lane for packed bf16 words, the fp32 sums written out.
 __device__ __forceinline__ uint32_t add_pair_bf16(uint32_t a, uint32_t b) {
   return pack_bf16(bf16_lo_f(a) + bf16_lo_f(b), bf16_hi_f(a) + bf16_hi_f(b));
@@ -265,15 +313,6 @@ __device__ __forceinline__ uint32_t add_pair(uint32_t a, uint32_t b) {
   } else {
     return add_pair_bf16(a, b);
   }
-}
-
-// Low (pack_lo) or high (pack_hi) 16-bit halves of two words, a's in the low
-// lane and b's in the high lane: one v_perm_b32.
-__device__ __forceinline__ uint32_t pack_lo(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_perm(b, a, 0x05040100u);
-}
-__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
 // (half EH of e) ^ (half WH of w), placed in the high half over a zero low
@@ -1114,39 +1153,6 @@ __global__ void __launch_bounds__(kRmwThreads, kRmwWavesPerEU) rmw_kernel(const 
 // wave and lookup, which 2^25 elements' 30 us are) and the cache.
 // ---------------------------------------------------------------------------
 
-// The two 16-bit lanes of a packed word as fp32, and two fp32 values rounded
-// to T and packed: one conversion instruction each way.
-struct F32Pair {
-  float lo, hi;
-};
-template <int DT>
-__device__ __forceinline__ F32Pair widen_pair(uint32_t x) {
-  return F32Pair{DT_<DT>::to_f(x & 0xffffu), DT_<DT>::to_f(x >> 16)};
-}
-template <int DT>
-__device__ __forceinline__ uint32_t round_pair(float lo, float hi) {
-  if constexpr (DT == DZ_F16) {
-    const dz_half2 r = {(_Float16)dz_opq(lo), (_Float16)dz_opq(hi)};
-    return __builtin_bit_cast(uint32_t, r);
-  } else {
-    return pack_bf16(dz_opq(lo), dz_opq(hi));
-  }
-}
-// b = R(R(s z) eps) of two packed signed z. kUnit: s is 1 (the fused modes'
-// perturbations), so R(s z) is z.
-template <int DT, bool kUnit>
-__device__ __forceinline__ uint32_t delta_b_pair(uint32_t z, const DzScalars& sc) {
-  F32Pair a = widen_pair<DT>(z);
-  if constexpr (!kUnit) a = widen_pair<DT>(round_pair<DT>(sc.scale * a.lo, sc.scale * a.hi));
-  return round_pair<DT>(a.lo * sc.eps, a.hi * sc.eps);
-}
-// -d = -R(lr R(g z)) of two packed signed z.
-template <int DT>
-__device__ __forceinline__ uint32_t delta_nd_pair(uint32_t z, const DzScalars& sc) {
-  const F32Pair a = widen_pair<DT>(z);
-  const F32Pair c = widen_pair<DT>(round_pair<DT>(sc.grad * a.lo, sc.grad * a.hi));
-  return round_pair<DT>(sc.lr * c.lo, sc.lr * c.hi) ^ 0x80008000u;
-}
 // The launch's operation on two packed 16-bit elements with their signed z
 // (and next step's z).
 template <int DT, int MODE>
