@@ -39,9 +39,10 @@ struct DzPtrArray {
 // 6.05 with 16 KB tiles and two workgroups per CU (which a 64 KB table would
 // allow); 32 KB and 128 KB tiles were no better, and the three-way pass took
 // 7.96 ms with six groups per thread and spilled with eight. fp32 uses 32 KB
-// tiles (one group of 8 fp32 per thread): its only workload, OPT-125m (347 MB
-// of parameters, about 40 tiles per CU), runs a pass in 121 us that way
-// against 140 us with 64 KB tiles. The bf16 restore + update + next
+// tiles (one group of 8 fp32 per thread): OPT-125m (347 MB of parameters,
+// about 40 tiles per CU) runs its perturb / three-way pass in 108 / 109 us that
+// way against 112 / 114 us with 64 KB tiles, 2^28 elements in 322 / 324 against
+// 336 / 331 us. The bf16 restore + update + next
 // perturbation pass (prefetching loop, ALU-bound) takes three groups per
 // thread (48 KB tiles): at OPT-30B 18.87-18.94 ms against 19.79-19.86 ms with
 // four and 19.57-19.62 with two (same box, alternating builds), where the
@@ -61,8 +62,8 @@ __host__ __device__ constexpr int rmw_chunk_elems(int dtype, int mode) {
 // rmw_short_kernel over tiles of kShortTile elements. Where the line lies: the
 // two passes of a steady step, against the persistent kernel with plain
 // accesses (what tables just above the line run best): fp16 2^24 elements 32.6
-// and 41.5 us, 2^25 53.0 and 52.2, 2^26 96.7 and 87.5; fp32 2^23 25.4 and 31.6,
-// 2^24 46.2 and 46.4, 2^25 84.4 and 80.4.
+// and 41.5 us, 2^25 53.0 and 52.2, 2^26 96.7 and 87.5; fp32 2^23 26.8 and 31.1,
+// 2^24 44.9 and 46.2, 2^24.5 64.1 and 61.4, 2^25 87.2 and 83.9.
 constexpr uint32_t kShortTile = kRmwThreads * 8;
 constexpr uint64_t short_elems(int dtype) { return dtype == DZ_F32 ? 1u << 24 : 1u << 25; }
 
@@ -71,9 +72,9 @@ constexpr uint64_t short_elems(int dtype) { return dtype == DZ_F32 ? 1u << 24 : 
 // accesses carry the non-temporal hint. Pass times in us (perturb / three-way)
 // with the hint and without, three tables used in turn: fp16 2^26 elements (128
 // MB) 47.0 / 51.0 and 47.3 / 45.7, 2^27 87.5 / 91.6 and 82.9 / 84.7, 2^27.25
-// 104 / 110 and 113 / 115, 2^28 169 / 173 and 183 / 185; fp32 2^25 50.7 / 49.6
-// and 43.6 / 40.7, 2^26 (256 MB) 94.7 / 92.6 and 79.2 / 78.3, 2^26.5 130 / 127
-// and 129 / 126, 2^29 701 / 718 and 727 / 744.
+// 104 / 110 and 113 / 115, 2^28 169 / 173 and 183 / 185; fp32 2^25 44.9 / 45.4
+// and 43.1 / 40.8, 2^26 (256 MB) 83.7 / 85.0 and 78.2 / 78.0, 2^26.25 99 / 101
+// and 111 / 104, 2^28 323 / 326 and 358 / 356.
 constexpr uint64_t kPlainBytes = 1u << 28;
 
 // LDS bytes of the per-launch delta table of an RMW launch: 16-bit entries
@@ -99,12 +100,10 @@ constexpr int kCounterWords = (kDoneSlot + 1) * kCounterStride;
 // Tile loops of the RMW launches. The restore + update + next perturbation
 // passes, whose ALU work per tile is the largest, run the prefetching loop
 // (rmw_tiles_prefetch: the next full tile's loads go out once the tile's
-// first group is stored; with fp32's one group per thread, before the tile's
-// Philox chain). Measured on the MI355X, same box, alternating builds, kernel
-// microbench: OPT-13B fp16 7.86-7.90 -> 7.58-7.61 ms, OPT-30B bf16
-// 20.10-20.16 -> 19.83-19.95 ms, OPT-125m fp32 0.1220-0.1227 -> 0.1205-0.1207
-// ms (in the step 0.1216-0.1217 -> 0.1210-0.1211; with the loads issued after
-// the tile's store instead, 0.130 ms). The single-Philox passes run the same
+// first group is stored). Measured on the MI355X, same box, alternating builds,
+// kernel microbench, plain loop against loads half-way: OPT-13B fp16 7.86-7.90
+// -> 7.58-7.61 ms, OPT-30B bf16 20.10-20.16 -> 19.83-19.95 ms. The
+// single-Philox passes run the same
 // on either loop (OPT-13B fp16 perturb 7.66-7.69 ms both, OPT-30B bf16
 // 17.76 ms both) and keep the plain loop (rmw_tiles).
 __host__ __device__ constexpr bool rmw_prefetch_mode(int dtype, int mode) {

@@ -597,6 +597,34 @@ __device__ __forceinline__ DzChunk uniform_proj_chunk(const DzChunk& c) {
   return u;
 }
 
+// The group of a full tile whose Philox block the thread draws for its set u.
+// 16-bit T: the group the thread holds. fp32: of a wave's 64 groups, lanes 2k
+// and 2k + 1 hold the halves of groups k and 32 + k; the even lane draws the
+// block of k, the odd one that of 32 + k.
+template <int DT>
+__device__ __forceinline__ uint32_t tile_group(int u) {
+  const uint32_t t = threadIdx.x + (uint32_t)u * kRmwThreads;
+  return DT != DZ_F32 ? t : (t & ~63u) + ((t & 1u) << 5) + ((t & 63u) >> 1);
+}
+
+// fp32: the z words of the thread's two vectors (x, y: the first; z, w: the
+// second) from the block it drew and its neighbour's: even lanes hold the low
+// halves of both groups, odd lanes the high ones.
+__device__ __forceinline__ DzU4 exchange_halves(const DzU4& b) {
+  const bool odd = (threadIdx.x & 1u) != 0u;
+  // quad_perm [1, 0, 3, 2]
+  const uint32_t r0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? b.x : b.z), 0xB1, 0xF, 0xF, true);
+  const uint32_t r1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? b.y : b.w), 0xB1, 0xF, 0xF, true);
+  return DzU4{odd ? r0 : b.x, odd ? r1 : b.y, odd ? b.z : r0, odd ? b.w : r1};
+}
+
+// The words of a thread's own elements from the block it drew.
+template <int DT>
+__device__ __forceinline__ DzU4 thread_words(const DzU4& b) {
+  if constexpr (DT == DZ_F32) return exchange_halves(b);
+  return b;
+}
+
 // Registers of one full tile: kVecs 16-byte vectors per thread.
 template <int DT, int MODE>
 struct TileRegs {
@@ -609,11 +637,17 @@ __device__ __forceinline__ bool full_tile(const DzChunk& ch) {
   return ch.n == (uint32_t)RmwTraits<DT, MODE>::kChunk;
 }
 
-// Lane layout of a full tile: a thread's groups of 8 elements are
-// threadIdx.x + u * 1024 for u < G (tile-local group indices), so each load
-// instruction of the workgroup covers contiguous memory. at(i) is the byte
-// offset of the thread's vector i from the tile's start: group u = i (16-bit)
-// or i / 2 (fp32, two vectors per group). A tile holds at most 64 KB. The
+// Lane layout of a full tile: each load instruction of a wave covers contiguous
+// memory. 16-bit T: a thread's groups of 8 elements (one vector each) are
+// threadIdx.x + u * 1024 for u < G (tile-local group indices). fp32 groups are
+// two vectors: a wave's 64 groups of set u are 128 consecutive vectors, of
+// which lane l holds l and 64 + l, that is half l mod 2 of groups l / 2 and 32
+// + l / 2 (tile_group and exchange_halves hand the Philox words on). With a
+// group's two vectors in one thread, each instruction took every other 16
+// bytes of its lines, and every fp32 pass ran 7-12 % slower: OPT-125m 121.5
+// against 108.5 us, 2^29 elements 702 / 721 against 656 / 653 us (perturb /
+// three-way). at(i) is the byte offset of the thread's vector i from the tile's
+// start: set u = i (16-bit) or i / 2 (fp32). A tile holds at most 64 KB. The
 // offsets are loop-invariant 64-bit values, so each access adds one to the
 // tile's base (one v_lshl_add_u64).
 //
@@ -622,8 +656,9 @@ __device__ __forceinline__ bool full_tile(const DzChunk& ch) {
 template <int DT, int MODE, bool kPlain>
 struct TileAccess {
   __device__ __forceinline__ size_t at(int i) const {
-    const size_t g0 = threadIdx.x;
-    return DT != DZ_F32 ? (g0 + (size_t)i * kRmwThreads) * 16 : (g0 + (size_t)(i >> 1) * kRmwThreads) * 32 + (size_t)(i & 1) * 16;
+    if constexpr (DT != DZ_F32) return ((size_t)threadIdx.x + (size_t)i * kRmwThreads) * 16;
+    return ((size_t)(threadIdx.x & ~63u) + (size_t)(i >> 1) * kRmwThreads) * 32 + (size_t)(i & 1) * 1024 +
+           (size_t)(threadIdx.x & 63u) * 16;
   }
   __device__ __forceinline__ dz_u32x4 load(const void* p) const { return kPlain ? ld_any(p) : ld_stream(p); }
   __device__ __forceinline__ void store(void* p, dz_u32x4 v) const {
@@ -640,14 +675,14 @@ __device__ __forceinline__ void load_tile_at(uint64_t addr, const Access& to, Ti
   for (int i = 0; i < TileRegs<DT, MODE>::kVecs; ++i) r.v[i] = to.load((const char*)addr + to.at(i));
 }
 
-// Philox block of group threadIdx.x + u * 1024 of a tile: counter zgroup +
-// that group. kUniformHi: the counters' high words agree across the tile (the
+// Philox block of a thread's group of set u of a tile (tile_group): counter
+// zgroup + that group. kUniformHi: the counters' high words agree across the tile (the
 // low word does not wrap inside it), so the high word is wave-uniform and the
 // counter's other uniform words keep round 0 and a product of rounds 1 and 2
 // on the scalar unit.
-template <bool kUniformHi>
+template <int DT, bool kUniformHi>
 __device__ __forceinline__ DzU4 tile_block(const DzChunk& ch, uint64_t seed, int u) {
-  const uint32_t g = threadIdx.x + (uint32_t)u * kRmwThreads;
+  const uint32_t g = tile_group<DT>(u);
   if constexpr (kUniformHi) {
     return dz_philox_counter(seed, kDzStreamParam, (uint32_t)ch.zgroup + g, (uint32_t)(ch.zgroup >> 32));
   } else {
@@ -660,8 +695,10 @@ __device__ __forceinline__ DzU4 tile_block(const DzChunk& ch, uint64_t seed, int
 template <int DT, int MODE, class Access>
 __device__ __forceinline__ void apply_store_group32(uint64_t base, const Access& to,
                                                     const TileRegs<DT, MODE>& r, int u,
-                                                    const DzU4& w, const DzU4& w2,
+                                                    const DzU4& wb, const DzU4& wb2,
                                                     const typename RmwTraits<DT, MODE>::E* tab, const DzScalars& sc) {
+  const DzU4 w = exchange_halves(wb);
+  const DzU4 w2 = MODE == kModeRestoreUpdatePerturb ? exchange_halves(wb2) : w;
   const dz_u32x4 a = r.v[2 * u], b = r.v[2 * u + 1];
   dz_u32x4 o0, o1;
   o0.x = apply_one<DT, MODE>(a.x, w.x & 0xffffu, w2.x & 0xffffu, tab, sc);
@@ -684,8 +721,9 @@ __device__ __forceinline__ void apply_store_group32(uint64_t base, const Access&
 // two ran one after the other (three-way pass at OPT-13B: 8.9 -> 8.2 ms at
 // equal Philox rounds).
 // kLoadNext (the prefetching tile loop): the next tile's loads, from nptr
-// into *nxt, go out once the first group is stored (for one group per
-// thread, before the Philox chains), held there by scheduling barriers.
+// into *nxt, go out once the first group is stored (for fp32's one group per
+// thread at the tile's end: 2^28 elements 324 us, before the Philox chains 335,
+// OPT-125m the same), held there by scheduling barriers.
 // Measured at OPT-13B fp16, three-way pass, kernel microbench, same box,
 // alternating builds: 7.86-7.90 ms with the loads issued before the Philox
 // chains, 7.69-7.70 after them, 7.58-7.59 half-way, 7.59 a quarter in, 7.60
@@ -704,19 +742,13 @@ __device__ __forceinline__ void tile_body(const DzChunk& ch, const Access& to,
                                           const typename RmwTraits<DT, MODE>::E* tab, const DzScalars& sc,
                                           uint64_t nptr = 0, TileRegs<DT, MODE>* nxt = nullptr) {
   constexpr int G = RmwTraits<DT, MODE>::kGroups;
-  // the next tile's loads go out after group kLoadAfter's stores (-1: first)
-  constexpr int kLoadAfter = G > 1 ? 0 : -1;
-  if constexpr (kLoadNext && kLoadAfter < 0) {
-    load_tile_at<DT, MODE>(nptr, to, *nxt);
-    __builtin_amdgcn_sched_barrier(0);
-  }
   constexpr bool kTwoSeeds = MODE == kModeRestoreUpdatePerturb;
   const uint64_t base = ch.ptr;
   DzU4 w[G], w2[G];
 #pragma unroll
   for (int u = 0; u < G; ++u) {
-    w[u] = tile_block<kUniformHi>(ch, sc.seed, u);
-    w2[u] = kTwoSeeds ? tile_block<kUniformHi>(ch, sc.seed2, u) : w[u];
+    w[u] = tile_block<DT, kUniformHi>(ch, sc.seed, u);
+    w2[u] = kTwoSeeds ? tile_block<DT, kUniformHi>(ch, sc.seed2, u) : w[u];
   }
 #pragma unroll
   for (int u = 0; u < G; ++u) {
@@ -730,8 +762,8 @@ __device__ __forceinline__ void tile_body(const DzChunk& ch, const Access& to,
       o.w = combine_pair16<DT, MODE>(r.v[u].w, w[u].w, w2[u].w, lookup_pair16<DT, MODE>(w[u].w, w2[u].w, tab));
       to.store((char*)base + to.at(u), o);
     }
-    if constexpr (kLoadNext && kLoadAfter >= 0) {
-      if (u == kLoadAfter) {
+    if constexpr (kLoadNext) {
+      if (u == 0) {
         __builtin_amdgcn_sched_barrier(0);
         load_tile_at<DT, MODE>(nptr, to, *nxt);
         __builtin_amdgcn_sched_barrier(0);
@@ -1201,46 +1233,63 @@ __device__ __forceinline__ ZVec<DT> z_vec(const typename DT_<DT>::S* tab, const 
   return r;
 }
 
-// A thread's group of 8 elements of a short table's tile.
+// A thread's 8 elements of a short table's tile: one vector of 16-bit T, or two
+// of fp32 laid out as in TileAccess.
 template <int DT>
 struct ShortGroup {
   using S = typename DT_<DT>::S;
   static constexpr int kVecs = ZVec<DT>::kVecs;
-  char* p;      // its first element
-  uint32_t n;   // elements of it inside the tile (0: none)
+  static constexpr uint32_t kPer = 16 / (uint32_t)sizeof(S);
+  char* base;       // the tile
+  uint32_t n;       // its elements
   dz_u32x4 v[kVecs];
 
+  // First element of the thread's vector k.
+  static __device__ __forceinline__ uint32_t first(int k) {
+    return DT != DZ_F32 ? threadIdx.x * 8u : (threadIdx.x & ~63u) * 8u + (uint32_t)k * 256u + (threadIdx.x & 63u) * 4u;
+  }
+  __device__ __forceinline__ uint32_t get(int k, int j) const {
+    return DT == DZ_F32 ? v[k][j & 3] : v[k][j >> 1] >> (16 * (j & 1));
+  }
   __device__ __forceinline__ ShortGroup() {}
   __device__ __forceinline__ explicit ShortGroup(const DzChunk& ch) {
-    p = (char*)ch.ptr + (size_t)threadIdx.x * (8 * sizeof(S));
-    const uint32_t first = threadIdx.x * 8u;
-    n = first < ch.n ? min(ch.n - first, 8u) : 0u;
-    if (n == 8u) {
+    base = (char*)ch.ptr;
+    n = ch.n;
 #pragma unroll
-      for (int k = 0; k < kVecs; ++k) v[k] = ld_any(p + 16 * k);
-    } else if (n > 0u) {  // the tensor's last elements
+    for (int k = 0; k < kVecs; ++k) {
+      const uint32_t e = first(k);
+      const S* p = (const S*)base + e;
+      if (e + kPer <= n) {
+        v[k] = ld_any(p);
+      } else if (e < n) {  // the tensor's last elements
 #pragma unroll
-      for (int j = 0; j < 8; ++j) set(j, (uint32_t)j < n ? (uint32_t)((const S*)p)[j] : 0u);
-    }
-  }
-  __device__ __forceinline__ void set(int j, uint32_t x) {
-    if constexpr (DT == DZ_F32)
-      v[j >> 2][j & 3] = x;
-    else
-      v[0][j >> 1] = j & 1 ? v[0][j >> 1] | (x << 16) : x;
-  }
-  __device__ __forceinline__ void store() const {
-    if (n == 8u) {
-#pragma unroll
-      for (int k = 0; k < kVecs; ++k) st_any(p + 16 * k, v[k]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t x = DT == DZ_F32 ? v[DT == DZ_F32 ? j >> 2 : 0][j & 3] : v[0][j >> 1] >> (16 * (j & 1));
-        if ((uint32_t)j < n) ((S*)p)[j] = (S)x;
+        for (int j = 0; j < (int)kPer; ++j) {
+          const uint32_t x = e + (uint32_t)j < n ? (uint32_t)p[j] : 0u;
+          if constexpr (DT == DZ_F32)
+            v[k][j & 3] = x;
+          else
+            v[k][j >> 1] = j & 1 ? v[k][j >> 1] | (x << 16) : x;
+        }
       }
     }
   }
+  __device__ __forceinline__ void store() const {
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k) {
+      const uint32_t e = first(k);
+      S* p = (S*)base + e;
+      if (e + kPer <= n) {
+        st_any(p, v[k]);
+      } else if (e < n) {
+#pragma unroll
+        for (int j = 0; j < (int)kPer; ++j)
+          if (e + (uint32_t)j < n) p[j] = (S)get(k, j);
+      }
+    }
+  }
+  // Whether any lane of the wave holds elements of the tile (the lanes of an
+  // fp32 pair exchange words, so a wave runs whole or not at all).
+  __device__ __forceinline__ bool wave_active() const { return (threadIdx.x & ~63u) * 8u < n; }
 };
 
 template <int DT, int MODE>
@@ -1265,7 +1314,7 @@ __global__ void __launch_bounds__(kRmwThreads, DT == DZ_F32 ? 4 : 8)
   const DzScalars sc = resolve_scalars<DT>(sc_in, sp);
   __syncthreads();
   for (;;) {
-    const uint64_t q = ch.zgroup + threadIdx.x;
+    const uint64_t q = ch.zgroup + tile_group<DT>(0);
     const uint32_t tn = t + gridDim.x;
     const bool more = tn < nchunks;
     ShortGroup<DT> nxt;
@@ -1273,9 +1322,9 @@ __global__ void __launch_bounds__(kRmwThreads, DT == DZ_F32 ? 4 : 8)
       ch = chunks[tn];
       nxt = ShortGroup<DT>(ch);
     }
-    if (cur.n > 0u) {
-      const ZVec<DT> z = z_vec<DT>(tab, dz_philox_group(sc.seed, kDzStreamParam, q));
-      const ZVec<DT> z2 = kNext ? z_vec<DT>(tab, dz_philox_group(sc.seed2, kDzStreamParam, q)) : z;
+    if (cur.wave_active()) {
+      const ZVec<DT> z = z_vec<DT>(tab, thread_words<DT>(dz_philox_group(sc.seed, kDzStreamParam, q)));
+      const ZVec<DT> z2 = kNext ? z_vec<DT>(tab, thread_words<DT>(dz_philox_group(sc.seed2, kDzStreamParam, q))) : z;
 #pragma unroll
       for (int k = 0; k < ZVec<DT>::kVecs; ++k) {
 #pragma unroll
@@ -1701,21 +1750,21 @@ __global__ void __launch_bounds__(256) static_plan_kernel(StaticPlanBatch b, DzC
   }
 }
 
-// The launch's range of z: n elements from element `offset` of the stream, so
-// group g (8 elements, one Philox block) covers outputs 8 g - skip .. 8 g -
-// skip + 7 for skip = offset mod 8. Element indices wrap modulo 2^64.
-template <int DT>
-__device__ __forceinline__ void store_z_group(const ZVec<DT>& z, uint64_t g, uint32_t skip, uint64_t n, void* out) {
+// One vector of z (kPer elements of T) from element e of the launch's groups:
+// n elements from element `offset` of the stream make groups of 8 (one Philox
+// block each) whose element e is output e - skip, skip = offset mod 8. Element
+// indices wrap modulo 2^64.
+template <int DT, int kPer>
+__device__ __forceinline__ void store_z(dz_u32x4 v, uint64_t e, uint32_t skip, uint64_t n, void* out) {
   using S = typename DT_<DT>::S;
-  const int64_t i0 = (int64_t)(g * 8u) - (int64_t)skip;
+  const int64_t i0 = (int64_t)e - (int64_t)skip;
   S* p = (S*)out + i0;
-  if (i0 >= 0 && (uint64_t)i0 + 8u <= n) {
-#pragma unroll
-    for (int k = 0; k < ZVec<DT>::kVecs; ++k) st_any((char*)p + 16 * k, z.v[k]);
+  if (i0 >= 0 && (uint64_t)i0 + kPer <= n) {
+    st_any(p, v);
   } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t b = DT == DZ_F32 ? z.v[DT == DZ_F32 ? j >> 2 : 0][j & 3] : z.v[0][j >> 1] >> (16 * (j & 1));
+    for (int j = 0; j < kPer; ++j) {
+      const uint32_t b = DT == DZ_F32 ? v[j & 3] : v[(j >> 1) & 3] >> (16 * (j & 1));
       if (i0 + j >= 0 && (uint64_t)(i0 + j) < n) p[j] = (S)b;
     }
   }
@@ -1733,7 +1782,10 @@ __global__ void __launch_bounds__(256) normals_kernel(const void* __restrict__ g
   const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g * 8u >= n + skip) return;
   const DzU4 w = dz_philox_group(seed, stream, (offset - skip + g * 8u) >> 3);
-  store_z_group<DT>(z_vec<DT>((const typename DT_<DT>::S*)gtab, w), g, skip, n, out);
+  const ZVec<DT> z = z_vec<DT>((const typename DT_<DT>::S*)gtab, w);
+#pragma unroll
+  for (int k = 0; k < ZVec<DT>::kVecs; ++k)
+    store_z<DT, 8 / ZVec<DT>::kVecs>(z.v[k], g * 8u + (uint64_t)k * (8 / ZVec<DT>::kVecs), skip, n, out);
 }
 
 // The same for long ranges: persistent workgroups copy the quantile table to
@@ -1762,15 +1814,23 @@ __global__ void __launch_bounds__(kNormalsThreads, DT == DZ_F32 ? 4 : 8)
   const uint64_t groups = (n + skip + 7u) >> 3;
   const uint64_t first = offset - skip;
   for (uint64_t t = blockIdx.x; t * kNormalsThreads < groups; t += gridDim.x) {
-    const uint64_t g = t * kNormalsThreads + threadIdx.x;
-    if (g >= groups) break;
-    const uint64_t q = (first + t * (kNormalsThreads * 8u)) >> 3;  // of the tile's first group
+    const uint64_t g0 = t * kNormalsThreads;  // the tile's first group
+    if (g0 + (threadIdx.x & ~63u) >= groups) break;  // whole waves: fp32 lanes exchange words
+    const uint32_t g = tile_group<DT>(0);
+    const uint64_t q = (first + g0 * 8u) >> 3;
     // the counters' high word is uniform over the tile unless the low word
     // (or the element index) wraps in it
     const DzU4 w = (uint32_t)q <= 0xffffffffu - (kNormalsThreads - 1u)
-                       ? dz_philox_counter(seed, stream, (uint32_t)q + threadIdx.x, (uint32_t)(q >> 32))
-                       : dz_philox_group(seed, stream, (first + g * 8u) >> 3);
-    store_z_group<DT>(z_vec<DT>(tab, w), g, skip, n, out);
+                       ? dz_philox_counter(seed, stream, (uint32_t)q + g, (uint32_t)(q >> 32))
+                       : dz_philox_group(seed, stream, (first + (g0 + g) * 8u) >> 3);
+    const ZVec<DT> z = z_vec<DT>(tab, thread_words<DT>(w));
+    if constexpr (DT == DZ_F32) {
+      const uint64_t e = (g0 + (threadIdx.x & ~63u)) * 8u + (threadIdx.x & 63u) * 4u;
+      store_z<DT, 4>(z.v[0], e, skip, n, out);
+      store_z<DT, 4>(z.v[1], e + 256u, skip, n, out);
+    } else {
+      store_z<DT, 8>(z.v[0], (g0 + g) * 8u, skip, n, out);
+    }
   }
 }
 
