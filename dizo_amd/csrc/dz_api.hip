@@ -343,14 +343,13 @@ void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
   for (int32_t i = 0; i < t->n; ++i) {
     const int64_t ne = t->numels[i];
     const uint64_t p = t->ptrs[i], a = t->aux[i], z = t->zoff[i];
-    const bool aligned = (p % 16 == 0) && (a % 16 == 0);
     for (int64_t s = 0; s < ne; s += elems) {
       DzChunk c;
       c.ptr = p + (uint64_t)s * es;
       c.aux = t->projection ? a + (uint64_t)s * es : 0;
       c.zgroup = t->projection ? (uint64_t)s : (z + (uint64_t)s) >> 3;
       c.n = (uint32_t)((ne - s) < (int64_t)elems ? (ne - s) : elems);
-      c.meta = (uint32_t)i | (aligned ? kDzMetaAligned : 0u);
+      c.meta = (uint32_t)i;
       out->push_back(c);
     }
     if (group_begin) group_begin->push_back((uint32_t)out->size());
@@ -502,7 +501,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
   if (!out) return fail(DZ_ERR_INVALID, "out is NULL");
   *out = nullptr;
   if (!ptrs || !numels) return fail(DZ_ERR_INVALID, "ptrs/numels is NULL");
-  if (n <= 0 || n > (int32_t)kDzMetaGroupMask) return fail(DZ_ERR_INVALID, "tensor count out of range");
+  if (n <= 0 || n > kDzMaxTensors) return fail(DZ_ERR_INVALID, "tensor count out of range");
   if (!valid_dtype(dtype)) return fail(DZ_ERR_INVALID, "unknown dtype");
   int cur;
   int32_t rc = current_device(&cur);

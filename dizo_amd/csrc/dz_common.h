@@ -75,12 +75,11 @@ struct DzChunk {
   uint64_t zgroup;  // ZO tables: Philox counter q of the chunk's first element (e / 8);
                     // projection tables: element offset of the chunk in its tensor
   uint32_t n;       // number of elements in the chunk
-  uint32_t meta;    // bits 0..23: tensor/group index; bit 31: all pointers 16-byte aligned
+  uint32_t meta;    // tensor/group index
 };
 static_assert(sizeof(DzChunk) == 32, "DzChunk must stay 32 bytes");
 
-constexpr uint32_t kDzMetaAligned = 0x80000000u;
-constexpr uint32_t kDzMetaGroupMask = 0x00ffffffu;
+constexpr int32_t kDzMaxTensors = 0x00ffffff;  // in one table
 
 struct DzU4 {
   uint32_t x, y, z, w;

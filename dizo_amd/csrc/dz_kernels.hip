@@ -1481,10 +1481,58 @@ __device__ __forceinline__ double block_sum_f64(double x, double* red) {
   return t;
 }
 
-// A chunk the vector path takes whole: full size and 16-byte aligned.
+// A chunk the vector path takes whole.
 template <int DT>
 __device__ __forceinline__ bool proj_full_chunk(const DzChunk& ch) {
-  return ch.n == (uint32_t)proj_chunk_elems(DT) && (ch.meta & kDzMetaAligned) != 0u;
+  return ch.n == (uint32_t)proj_chunk_elems(DT);
+}
+
+// The operation on one 16-byte vector of theta with its anchor's. What depends
+// on the group's alpha is made once per chunk (ProjScalars).
+template <int DT, int MODE>
+struct ProjScalars {
+  float alpha;
+  uint32_t alpha2;  // alpha in both 16-bit lanes (the ZO modes' alpha is a value of T)
+  RecipDiv rd;
+  __device__ __forceinline__ explicit ProjScalars(float a)
+      : alpha(a),
+        alpha2((DT != DZ_F32 && MODE != kProjApplyF32) ? DT_<DT>::from_f(a) * 0x10001u : 0u),
+        rd((DT == DZ_BF16 && (MODE == kProjReverse || MODE == kProjReverseSumsq)) ? recip_div(a)
+                                                                                : RecipDiv{0.0f, false}) {}
+};
+template <int DT, int MODE>
+__device__ __forceinline__ dz_u32x4 proj_vec(dz_u32x4 vt, dz_u32x4 va, const ProjScalars<DT, MODE>& ps, double* acc) {
+  dz_u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (DT != DZ_F32 && MODE != kProjApplyF32) {
+      o[i] = proj_word16<DT, MODE>(vt[i], va[i], ps.alpha2, ps.alpha, ps.rd, acc);
+    } else if constexpr (DT != DZ_F32) {
+      uint32_t r0, r1;
+      proj_elem<DT>(MODE, vt[i] & 0xffffu, va[i] & 0xffffu, ps.alpha, &r0, acc);
+      proj_elem<DT>(MODE, vt[i] >> 16, va[i] >> 16, ps.alpha, &r1, acc);
+      o[i] = (r0 & 0xffffu) | (r1 << 16);
+    } else {
+      uint32_t r;
+      proj_elem<DT>(MODE, vt[i], va[i], ps.alpha, &r, acc);
+      o[i] = r;
+    }
+  }
+  return o;
+}
+// Elements e .. n - 1 of a chunk, one by one (its last, incomplete vector; the
+// rest of a partial chunk goes vector by vector. With all of it one by one, and
+// misaligned groups too, 128 groups of 20,480 fp16 elements took 26 us to apply,
+// 12 now).
+template <int DT, int MODE>
+__device__ __forceinline__ void proj_tail(char* tp, const char* ap, uint32_t e, uint32_t n, float alpha, double* acc) {
+  using S = typename DT_<DT>::S;
+  for (; e < n; ++e) {
+    S* p = (S*)tp + e;
+    uint32_t r;
+    proj_elem<DT>(MODE, (uint32_t)*p, (uint32_t)((const S*)ap)[e], alpha, &r, acc);
+    if constexpr (MODE != kProjSumsq) *p = (S)r;
+  }
 }
 
 // Vector-memory operations a thread issues for a full chunk: its 16-byte
@@ -1507,11 +1555,7 @@ __device__ __forceinline__ void proj_chunk(const DzChunk& ch, float alpha, doubl
   double acc = 0.0;
   if (proj_full_chunk<DT>(ch)) {
     constexpr int kVecsPerThread = ProjChunkOps<DT, MODE>::kVecs;
-    // alpha in both 16-bit lanes (the ZO modes' alpha is a value of T)
-    const uint32_t alpha2 = (kES == 2 && MODE != kProjApplyF32) ? DT_<DT>::from_f(alpha) * 0x10001u : 0u;
-    const RecipDiv rd = (DT == DZ_BF16 && (MODE == kProjReverse || MODE == kProjReverseSumsq))
-                            ? recip_div(alpha)
-                            : RecipDiv{0.0f, false};
+    const ProjScalars<DT, MODE> ps(alpha);
     dz_u32x4 vt[kVecsPerThread], va[kVecsPerThread];
 #pragma unroll
     for (int u = 0; u < kVecsPerThread; ++u) {
@@ -1521,31 +1565,19 @@ __device__ __forceinline__ void proj_chunk(const DzChunk& ch, float alpha, doubl
     }
 #pragma unroll
     for (int u = 0; u < kVecsPerThread; ++u) {
-      dz_u32x4 o;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (kES == 2 && MODE != kProjApplyF32) {
-          o[i] = proj_word16<DT, MODE>(vt[u][i], va[u][i], alpha2, alpha, rd, &acc);
-        } else if constexpr (kES == 2) {
-          uint32_t r0, r1;
-          proj_elem<DT>(MODE, vt[u][i] & 0xffffu, va[u][i] & 0xffffu, alpha, &r0, &acc);
-          proj_elem<DT>(MODE, vt[u][i] >> 16, va[u][i] >> 16, alpha, &r1, &acc);
-          o[i] = (r0 & 0xffffu) | (r1 << 16);
-        } else {
-          uint32_t r;
-          proj_elem<DT>(MODE, vt[u][i], va[u][i], alpha, &r, &acc);
-          o[i] = r;
-        }
-      }
+      const dz_u32x4 o = proj_vec<DT, MODE>(vt[u], va[u], ps, &acc);
       if constexpr (MODE != kProjSumsq) st_stream(tp + (size_t)(threadIdx.x + u * kProjThreads) * 16, o);
     }
   } else {
-    for (uint32_t e = threadIdx.x; e < ch.n; e += kProjThreads) {
-      S* p = (S*)(tp + (size_t)e * kES);
-      const S* q = (const S*)(ap + (size_t)e * kES);
-      uint32_t r;
-      proj_elem<DT>(MODE, (uint32_t)*p, (uint32_t)*q, alpha, &r, &acc);
-      if constexpr (MODE != kProjSumsq) *p = (S)r;
+    const ProjScalars<DT, MODE> ps(alpha);
+    constexpr uint32_t kPer = 16 / kES;
+    for (uint32_t e = threadIdx.x * kPer; e < ch.n; e += kProjThreads * kPer) {
+      if (e + kPer <= ch.n) {
+        const dz_u32x4 o = proj_vec<DT, MODE>(ld_stream(tp + (size_t)e * kES), ld_stream(ap + (size_t)e * kES), ps, &acc);
+        if constexpr (MODE != kProjSumsq) st_stream(tp + (size_t)e * kES, o);
+      } else {
+        proj_tail<DT, MODE>(tp, ap, e, ch.n, alpha, &acc);
+      }
     }
   }
   if constexpr (MODE == kProjSumsq || MODE == kProjReverseSumsq) {
@@ -1609,7 +1641,7 @@ __global__ void __launch_bounds__(kProjThreads) proj_kernel(const DzChunk* __res
     const uint32_t c = sidx[k % 4];
     if (c >= nchunks) break;
     const DzChunk ch = uniform_proj_chunk(sdesc[k % 3]);
-    const uint32_t grp = ch.meta & kDzMetaGroupMask;
+    const uint32_t grp = ch.meta;
     const float alpha = MODE == kProjSumsq ? 0.0f
                         : alpha_in_lds     ? salpha[grp]
                                            : group_alpha<DT, MODE>(alpha_T, grp);
@@ -1675,7 +1707,7 @@ __global__ void __launch_bounds__(kProjThreads) dot_kernel(const DzChunk* __rest
   __shared__ double red[kProjThreads / 64];
   const uint32_t c = blockIdx.x;
   const DzChunk ch = chunks[c];
-  const uint32_t grp = ch.meta & kDzMetaGroupMask;
+  const uint32_t grp = ch.meta;
   const S* tp = (const S*)ch.ptr;
   const S* ap = (const S*)ch.aux;
   const S* op = (const S*)(other.p[grp - group_base] + ch.zgroup * (uint64_t)kES);
@@ -1715,9 +1747,8 @@ __global__ void __launch_bounds__(kProjThreads) finalize_kernel(const double* __
 
 // Chunk descriptors of a projection launch planned on the device (the
 // table-free norm pass): block g writes group g's chunks, split as
-// dz_table_create splits them (proj_chunk_elems(dtype) elements, the last one shorter;
-// aligned when theta and theta0 are 16-byte aligned), and its first chunk
-// index; the last batch also writes the end index of the last group. The
+// dz_table_create splits them (proj_chunk_elems(dtype) elements, the last one
+// shorter), and its first chunk index; the last batch also writes the end index of the last group. The
 // first batch zeroes the work counters the projection kernel takes chunks
 // from.
 __global__ void __launch_bounds__(256) static_plan_kernel(StaticPlanBatch b, DzChunk* __restrict__ chunks,
@@ -1731,7 +1762,7 @@ __global__ void __launch_bounds__(256) static_plan_kernel(StaticPlanBatch b, DzC
   const uint32_t gi = b.group_base + g;
   const uint64_t p = b.ptr[g], a = b.anchor[g];
   const int64_t ne = b.numel[g];
-  const uint32_t meta = gi | ((p % 16 == 0 && a % 16 == 0) ? kDzMetaAligned : 0u);
+  const uint32_t meta = gi;
   const int64_t cn = b.chunk_elems;
   const uint32_t nch = (uint32_t)((ne + cn - 1) / cn);
   for (uint32_t k = threadIdx.x; k < nch; k += blockDim.x) {

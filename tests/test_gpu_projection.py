@@ -107,6 +107,54 @@ def test_apply_reverse_match_torch_on_device(dt):
     tab.close()
 
 
+def _packed_groups(dt, sizes, first):
+    """Groups of odd sizes end to end in one buffer, their anchors in another from a different start
+    address; (buffer, groups, anchors, their bits)."""
+    ths, t0s, th_h, t0_h = _groups(dt, 77, sizes=sizes)
+    total = sum(sizes)
+    buf = torch.full((first + total + 9,), 3.0, dtype=DT_TORCH[dt], device="cuda")
+    anchor = torch.zeros(total + 2, dtype=DT_TORCH[dt], device="cuda")
+    out, out0, at = [], [], 0
+    for t, t0 in zip(ths, t0s):
+        buf[first + at:first + at + t.numel()] = t
+        anchor[2 + at:2 + at + t.numel()] = t0
+        out.append(buf[first + at:first + at + t.numel()])
+        out0.append(anchor[2 + at:2 + at + t.numel()])
+        at += t.numel()
+    return buf, out, out0, th_h, t0_h
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("first", [1, 3])
+@pytest.mark.parametrize("sizes", [[1, 7, 32768 + 5, 8193, 3, 2 * 32768, 999], [5, 6_000_001, 32768, 6_000_003]])
+def test_packed_odd_groups_match_oracle(dt, first, sizes):
+    """Norms, apply and reverse over groups that start anywhere, short and long tables: values against
+    the oracle, sums against its fp64 sums, the elements around the groups untouched."""
+    from dizo_amd._lib import DZ_PROJ_APPLY, DZ_PROJ_REVERSE_SUMSQ
+    from dizo_amd.table import ProjTable
+    buf, ths, t0s, th_h, t0_h = _packed_groups(dt, sizes, first)
+    G = len(sizes)
+    alphas = from_f32(np.linspace(0.85, 1.1, G).astype(np.float32), dt)
+    alpha_t = to_torch(alphas, dt, "cuda")
+    sums = [torch.empty(G, dtype=torch.float64, device="cuda") for _ in range(3)]
+    tab = ProjTable(ths, t0s)
+    tab.group_sumsq(sums[0])
+    tab.project(alpha_t, DZ_PROJ_APPLY)
+    tab.group_sumsq(sums[1])
+    app = [A.apply(th_h[g], t0_h[g], alphas[g:g + 1], dt) for g in range(G)]
+    for g in range(G):
+        assert_bits_equal(to_bits(ths[g]), app[g], dt, f"apply group {g}")
+    tab.project(alpha_t, DZ_PROJ_REVERSE_SUMSQ, sumsq=sums[2])
+    rev = [A.reverse(app[g], t0_h[g], alphas[g:g + 1], dt) for g in range(G)]
+    for g in range(G):
+        assert_bits_equal(to_bits(ths[g]), rev[g], dt, f"reverse group {g}")
+        for got, x in zip(sums, (th_h[g], app[g], rev[g])):
+            # fp64 sums of n exact squares: n / 2 roundings of at most 2^-53 apart
+            assert float(got[g]) == pytest.approx(A.group_sumsq(x, t0_h[g], dt), rel=max(sizes) * 2.0**-53, abs=0)
+    assert bool((buf[:first] == 3.0).all()) and bool((buf[first + sum(sizes):] == 3.0).all())
+    tab.close()
+
+
 def test_empty_and_rejects():
     from dizo_amd._lib import DZ_PROJ_APPLY, DzError
     from dizo_amd.table import ProjTable
