@@ -189,7 +189,8 @@ int32_t check_range(uint64_t p, uint64_t bytes, const char* what, int32_t i) {
 // Scratch of the allocation-free entry point (dz_group_sumsq_static): device
 // memory the library never allocates at run time. Layout: the projection
 // kernel's work counters, the group -> first chunk index, the chunk
-// descriptors and the per-chunk partial sums, for at most kStaticMaxGroups
+// descriptors, the per-chunk partial sums and (zero between launches) the
+// groups' finished-chunk counts of short inputs, for at most kStaticMaxGroups
 // groups and kStaticMaxChunks chunks of proj_chunk_elems(dtype) elements (8.6 G
 // elements of a 16-bit type, 2.1 G of fp32).
 // Each device holds its own copy, at its own address (see static_scratch).
@@ -197,11 +198,15 @@ int32_t check_range(uint64_t p, uint64_t bytes, const char* what, int32_t i) {
 namespace {
 constexpr uint32_t kStaticMaxGroups = 4096;
 constexpr uint32_t kStaticMaxChunks = 1u << 18;
+// short inputs: at most one chunk more for each group than their elements fill
+static_assert(dz::kShortProjTotal / (uint64_t)dz::short_proj_elems(DZ_F32) + kStaticMaxGroups <= kStaticMaxChunks,
+              "partial sums of short inputs");
 constexpr size_t kStaticOffCounters = 0;
 constexpr size_t kStaticOffGroupBegin = 4096;
 constexpr size_t kStaticOffChunks = kStaticOffGroupBegin + ((kStaticMaxGroups + 1) * 4 + 255) / 256 * 256;
 constexpr size_t kStaticOffPartials = kStaticOffChunks + (size_t)kStaticMaxChunks * sizeof(DzChunk);
-constexpr size_t kStaticBytes = kStaticOffPartials + (size_t)kStaticMaxChunks * sizeof(double);
+constexpr size_t kStaticOffDone = kStaticOffPartials + (size_t)kStaticMaxChunks * sizeof(double);
+constexpr size_t kStaticBytes = kStaticOffDone + (size_t)kStaticMaxGroups * dz::kDoneStride * sizeof(uint32_t);
 static_assert(dz::kCounterWords * 4 <= kStaticOffGroupBegin, "work counters overflow their scratch slot");
 }  // namespace
 
@@ -230,6 +235,8 @@ struct dz_table {
   DzChunk* d_short_chunks = nullptr;
   uint32_t* d_group_begin = nullptr;
   double* d_partials = nullptr;
+  bool short_proj = false;         // a short projection table: its chunks are proj_short_kernel's
+  uint32_t* d_group_done = nullptr;  // finished chunks of each group (short projection tables)
   uint32_t* d_counters = nullptr;  // work counters of the persistent RMW / projection kernels
   DeviceState* dev = nullptr;
   dz::LaunchEvents timing;  // dz_table_time_next's request for the next launching call
@@ -276,6 +283,7 @@ void free_table(dz_table* t) {
   if (t->d_short_chunks) (void)hipFree(t->d_short_chunks);
   if (t->d_group_begin) (void)hipFree(t->d_group_begin);
   if (t->d_partials) (void)hipFree(t->d_partials);
+  if (t->d_group_done) (void)hipFree(t->d_group_done);
   if (t->d_counters) (void)hipFree(t->d_counters);
   delete t;
 }
@@ -334,6 +342,15 @@ int32_t rmw(dz_table* t, int mode, const dz::DzScalars& s, const dz::DzScalarPtr
   return DZ_OK;
 }
 
+// A projection launch over a short table.
+int32_t proj_short(dz_table* t, int mode, const void* alpha, const dz::GroupOutputs& out, const dz::LaunchEvents& ev,
+                   void* stream) {
+  const dz::ProjShort a{t->d_chunks, t->d_group_begin, t->d_group_done, alpha, t->d_partials, out};
+  const hipError_t e = dz::launch_proj_short(t->dtype, mode, t->nchunks, a, (hipStream_t)stream, ev);
+  if (e != hipSuccess) return hip_fail(e, "projection kernel launch");
+  return DZ_OK;
+}
+
 // Tiles of `elems` elements over every registered tensor, in tensor order.
 void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
                   std::vector<uint32_t>* group_begin) {
@@ -352,6 +369,8 @@ void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
       c.meta = (uint32_t)i;
       out->push_back(c);
     }
+    // a chunk of no elements, so that the group's results are written
+    if (t->short_proj && ne == 0) out->push_back(DzChunk{p, a, 0, 0, (uint32_t)i});
     if (group_begin) group_begin->push_back((uint32_t)out->size());
   }
 }
@@ -565,6 +584,11 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     free_table(t);
     return rc;
   }
+  for (int64_t ne : t->numels) t->bytes += (uint64_t)ne * es;
+  if (t->projection && t->bytes <= dz::kShortProjTotal * es) {
+    t->short_proj = true;
+    t->chunk_elems = (uint32_t)dz::short_proj_elems(dtype);
+  }
   std::vector<DzChunk> chunks;
   build_chunks(t, t->chunk_elems, &chunks, t->projection ? &t->group_begin : nullptr);
   t->nchunks = (uint32_t)chunks.size();
@@ -579,7 +603,6 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     t->fused_nchunks = (uint32_t)fc.size();
     e = upload_chunks(fc, &t->d_fused_chunks);
   }
-  for (int64_t ne : t->numels) t->bytes += (uint64_t)ne * es;
   if (e == hipSuccess && !t->projection && t->bytes <= dz::short_elems(dtype) * es) {
     std::vector<DzChunk> sc;
     build_chunks(t, dz::kShortTile, &sc, nullptr);
@@ -593,6 +616,11 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
       e = hipMemcpy(t->d_group_begin, t->group_begin.data(), t->group_begin.size() * sizeof(uint32_t),
                     hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMalloc(&t->d_partials, (size_t)(t->nchunks ? t->nchunks : 1) * sizeof(double));
+    if (e == hipSuccess && t->short_proj) {
+      const size_t bytes = (size_t)t->n * dz::kDoneStride * sizeof(uint32_t);
+      e = hipMalloc(&t->d_group_done, bytes);
+      if (e == hipSuccess) e = hipMemset(t->d_group_done, 0, bytes);
+    }
   }
   if (e == hipSuccess) {
     // zeroed once here; every RMW and projection launch leaves them at zero again
@@ -725,6 +753,7 @@ int32_t dz_group_sumsq(dz_table* t, double* d_sumsq, float* d_norm_f32, void* d_
   if (!t->projection) return fail(DZ_ERR_INVALID, "group_sumsq needs a projection table");
   rc = check_group_outputs(t, d_sumsq, d_norm_f32, d_norm_T);
   if (rc) return rc;
+  if (t->short_proj) return proj_short(t, dz::kProjSumsq, nullptr, {d_sumsq, d_norm_f32, d_norm_T}, ev, stream);
   hipError_t e = hipSuccess;
   if (t->nchunks > 0) {
     e = dz::launch_proj(t->dtype, dz::kProjSumsq, t->d_chunks, t->nchunks, (uint32_t)t->n, proj_grid(t),
@@ -784,6 +813,33 @@ int32_t dz_group_sumsq_static(const uint64_t* ptrs, const uint64_t* anchor_ptrs,
   DzChunk* chunks = (DzChunk*)(sc->ptr + kStaticOffChunks);
   double* partials = (double*)(sc->ptr + kStaticOffPartials);
   const hipStream_t st = (hipStream_t)stream;
+  // short inputs: one launch for kStaticPlanGroups groups, chunks as in a short table
+  uint64_t elems = 0;
+  for (int32_t i = 0; i < n; ++i) elems += (uint64_t)numels[i];
+  if (elems <= dz::kShortProjTotal) {
+    const uint64_t sn = (uint64_t)dz::short_proj_elems(dtype);
+    uint32_t begin = 0;
+    for (int32_t g0 = 0; g0 < n; g0 += dz::kStaticPlanGroups) {
+      dz::StaticGroups sg;
+      sg.ngroups = (uint32_t)std::min<int32_t>(dz::kStaticPlanGroups, n - g0);
+      sg.group_base = (uint32_t)g0;
+      uint32_t at = 0;
+      for (uint32_t k = 0; k < sg.ngroups; ++k) {
+        sg.ptr[k] = ptrs[g0 + k];
+        sg.anchor[k] = anchor_ptrs[g0 + k];
+        sg.numel[k] = numels[g0 + k];
+        sg.chunk_begin[k] = at;
+        at += (uint32_t)std::max<uint64_t>(1, ((uint64_t)numels[g0 + k] + sn - 1) / sn);
+      }
+      sg.chunk_begin[sg.ngroups] = at;
+      const dz::ProjShort a{nullptr, nullptr, (uint32_t*)(sc->ptr + kStaticOffDone), nullptr, partials + begin,
+                            {d_sumsq, d_norm_f32, d_norm_T}};
+      const hipError_t e = dz::launch_static_sumsq(dtype, at, a, sg, st);
+      if (e != hipSuccess) return hip_fail(e, "sumsq kernel launch");
+      begin += at;
+    }
+    return DZ_OK;
+  }
   // the chunk plan, kStaticPlanGroups groups per launch (the group list travels as a kernel argument)
   uint32_t next = 0;
   for (int32_t g0 = 0; g0 < n; g0 += dz::kStaticPlanGroups) {
@@ -831,7 +887,9 @@ int32_t dz_project(dz_table* t, const void* d_alpha, int32_t mode, double* d_sum
   if (!rc) rc = check_group_outputs(t, d_sumsq, d_norm_f32, d_norm_T);
   if (rc) return rc;
   const bool finalize = mode == DZ_PROJ_REVERSE_SUMSQ;
-  if (t->nchunks > 0) {
+  if (t->short_proj && (finalize || t->bytes > 0))
+    return proj_short(t, mode, d_alpha, {d_sumsq, d_norm_f32, d_norm_T}, ev, stream);
+  if (t->nchunks > 0 && !t->short_proj) {
     hipError_t e = dz::launch_proj(t->dtype, mode, t->d_chunks, t->nchunks, (uint32_t)t->n, proj_grid(t),
                                    d_alpha, t->d_partials, t->d_counters, (hipStream_t)stream,
                                    {ev.start, finalize ? nullptr : ev.stop});

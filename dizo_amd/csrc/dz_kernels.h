@@ -134,6 +134,24 @@ __host__ __device__ constexpr int proj_chunk_elems(int dtype) { return dtype == 
 // beyond that each chunk reads its group's alpha from memory.
 constexpr int kProjAlphaLds = 4096;
 
+// Short projection tables: up to kShortProjTotal elements in all, whose launches
+// run proj_short_kernel over chunks of short_proj_elems(dtype) elements, a
+// workgroup of kShortProjThreads each. Pass times in us (norms / apply / reverse
+// + norms; a norm pass with its group sums), against the persistent kernel:
+// fp16 128 x 20,480 elements 5.6 / 4.6 / 6.4 and 14.9 / 11.9 / 22.1, 24 x
+// 589,824 12.6 / 13.0 / 17.4 and 20.9 / 21.4 / 31.4, 48 x 1,048,576 38.7 / 42.2
+// / 47.2 and 41.6 / 51.0 / 59.2, 64 x 2,097,152 100 / 123 / 149 and 93 / 127 /
+// 136; fp32 24 x 589,824 26.5 / 24.5 / 31.1 and 30.3 / 31.0 / 38.3, 48 x
+// 1,048,576 78 / 91 / 108 and 78 / 95 / 115, 64 x 2,097,152 214 / 274 / 314 and
+// 184 / 244 / 293. Chunks of half the size cost more counting (fp16 24 x
+// 589,824: norms 17.4), of twice the size run the same.
+constexpr int kShortProjThreads = 256;
+__host__ __device__ constexpr int short_proj_elems(int dtype) { return dtype == DZ_F32 ? 2048 : 4096; }
+constexpr uint64_t kShortProjTotal = 3u << 24;
+// The groups' finished-chunk counts lie 128 bytes apart: side by side, every
+// workgroup's atomic met in the same line (22 ns each: 43 us for the norms of fp16 24 x 589,824).
+constexpr int kDoneStride = 32;  // uint32 slots
+
 // By-value scalars of one RMW launch.
 struct DzScalars {
   uint64_t seed;
@@ -175,6 +193,37 @@ hipError_t launch_rmw_short(int dtype, int mode, const DzChunk* chunks, uint32_t
 hipError_t launch_proj(int dtype, int mode, const DzChunk* chunks, uint32_t nchunks, uint32_t ngroups,
                        uint32_t grid, const void* alpha, double* partials, uint32_t* counters, hipStream_t st,
                        const LaunchEvents& ev = {});
+// Per-group results of a norm pass; any may be NULL.
+struct GroupOutputs {
+  double* sumsq;
+  float* norm_f32;
+  void* norm_T;
+};
+// A projection launch over a short table: its chunk list (nchunks of them; an
+// empty group has one of no elements) and each group's first chunk, the groups'
+// finished-chunk counts (zero before the launch, which leaves them at zero).
+struct ProjShort {
+  const DzChunk* chunks;
+  const uint32_t* group_begin;
+  uint32_t* group_done;
+  const void* alpha;
+  double* partials;
+  GroupOutputs out;
+};
+// The groups of a norm pass without a table: they travel as kernel arguments,
+// kStaticPlanGroups to a launch.
+constexpr int kStaticPlanGroups = 64;
+struct StaticGroups {
+  uint64_t ptr[kStaticPlanGroups];
+  uint64_t anchor[kStaticPlanGroups];
+  int64_t numel[kStaticPlanGroups];
+  uint32_t chunk_begin[kStaticPlanGroups + 1];  // within the launch
+  uint32_t ngroups;
+  uint32_t group_base;
+};
+hipError_t launch_proj_short(int dtype, int mode, uint32_t nchunks, const ProjShort& a, hipStream_t st,
+                             const LaunchEvents& ev = {});
+hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, const ProjShort& a, const StaticGroups& sg, hipStream_t st);
 // Chunks of groups group_base .. group_base + kMaxDotGroups - 1; other.p[i]
 // is the tensor of group group_base + i.
 hipError_t launch_dot(int dtype, const DzChunk* chunks, uint32_t nchunks, const DzPtrArray& other,
@@ -186,7 +235,6 @@ hipError_t launch_finalize(int dtype, const double* partials, const uint32_t* gb
 // Chunk plan of a projection launch without a table (dz_group_sumsq_static):
 // kStaticPlanGroups groups per plan launch, their descriptors and the
 // group -> chunk index written into caller-provided device memory.
-constexpr int kStaticPlanGroups = 64;
 struct StaticPlanBatch {
   uint64_t ptr[kStaticPlanGroups];
   uint64_t anchor[kStaticPlanGroups];

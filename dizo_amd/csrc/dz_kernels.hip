@@ -1720,6 +1720,17 @@ __global__ void __launch_bounds__(kProjThreads) dot_kernel(const DzChunk* __rest
   if (threadIdx.x == 0) partials[c] = t;
 }
 
+// A group's results from the sum t of its chunks' partials.
+template <int DT>
+__device__ __forceinline__ void write_group(const GroupOutputs& o, uint32_t g, double t, bool take_sqrt) {
+  using S = typename DT_<DT>::S;
+  // correctly rounded fp32 sqrt of the fp32 sum (a double sqrt rounds once more, exactly)
+  const float n = take_sqrt ? (float)sqrt((double)(float)t) : (float)t;
+  if (o.sumsq) o.sumsq[g] = t;
+  if (o.norm_f32) o.norm_f32[g] = n;
+  if (o.norm_T) ((S*)o.norm_T)[g] = (S)DT_<DT>::from_f(n);
+}
+
 // Per-group reduction of chunk partials, in chunk order. With take_sqrt:
 // norm = R_T(sqrt_f32(fp32(sum)))  (torch.norm: fp32 accumulate, fp32 sqrt, cast to T);
 // without: the fp32 / T outputs hold the rounded sum itself.
@@ -1729,19 +1740,114 @@ __global__ void __launch_bounds__(kProjThreads) finalize_kernel(const double* __
                                                                 double* __restrict__ sumsq,
                                                                 float* __restrict__ norm_f32,
                                                                 void* __restrict__ norm_T, bool take_sqrt) {
-  using S = typename DT_<DT>::S;
   __shared__ double red[kProjThreads / 64];
   const uint32_t g = blockIdx.x;
   const uint32_t b = gbegin[g], e = gbegin[g + 1];
   double x = 0.0;
   for (uint32_t i = b + threadIdx.x; i < e; i += kProjThreads) x += partials[i];
   const double t = block_sum_f64(x, red);
+  if (threadIdx.x == 0) write_group<DT>(GroupOutputs{sumsq, norm_f32, norm_T}, g, t, take_sqrt);
+}
+
+// ---------------------------------------------------------------------------
+// Projection launches over short tables: one workgroup of 256 threads per chunk
+// of short_proj_elems, all of a thread's vectors in flight at once, no work
+// counters. The workgroup that ends a group's last chunk sums the group's
+// partials (in chunk order) and writes its results, so that a norm pass is one
+// launch. Chunks come from the table's list, or (StaticGroups) from the group
+// list in the launch's arguments.
+// ---------------------------------------------------------------------------
+
+// Counts a finished chunk of group g after publishing its partial sum; true in
+// every thread of the workgroup that finished last, which then reads the
+// group's other partials with read_partial. The partial is written through to
+// where every XCD sees it (agent-scope atomic store) and waited for before the
+// count, so the count needs no write-back of the L2 for it.
+__device__ __forceinline__ bool publish_partial(double* slot, double t, uint32_t* done, uint32_t chunks, uint32_t* flag) {
   if (threadIdx.x == 0) {
-    // correctly rounded fp32 sqrt of the fp32 sum (a double sqrt rounds once more, exactly)
-    const float n = take_sqrt ? (float)sqrt((double)(float)t) : (float)t;
-    if (sumsq) sumsq[g] = t;
-    if (norm_f32) norm_f32[g] = n;
-    if (norm_T) ((S*)norm_T)[g] = (S)DT_<DT>::from_f(n);
+    __hip_atomic_store((uint64_t*)slot, __builtin_bit_cast(uint64_t, t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const uint32_t before = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool last = before + 1u == chunks;
+    if (last) __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+    *flag = last ? 1u : 0u;
+  }
+  __syncthreads();
+  return *flag != 0u;
+}
+__device__ __forceinline__ double read_partial(const double* slot) {
+  return __builtin_bit_cast(double, __hip_atomic_load((const uint64_t*)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+struct NoGroups {};  // the chunks come from the table's list
+template <int DT, int MODE, class Groups>
+__global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort a, Groups sg) {
+  constexpr bool kStatic = std::is_same<Groups, StaticGroups>::value;
+  using S = typename DT_<DT>::S;
+  constexpr uint32_t kPer = 16 / (uint32_t)sizeof(S);
+  constexpr int kVecs = short_proj_elems(DT) / (kShortProjThreads * (int)kPer);
+  constexpr bool kSums = MODE == kProjSumsq || MODE == kProjReverseSumsq;
+  __shared__ double red[kShortProjThreads / 64];
+  __shared__ uint32_t flag;
+  uint32_t c = blockIdx.x, grp, first, count;
+  char* tp;
+  const char* ap;
+  uint32_t n;
+  if constexpr (kStatic) {
+    uint32_t lo = 0, hi = sg.ngroups;  // the group whose chunks hold c
+    while (hi - lo > 1u) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (sg.chunk_begin[mid] <= c)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    first = sg.chunk_begin[lo];
+    count = sg.chunk_begin[lo + 1] - first;
+    const int64_t s = (int64_t)(c - first) * short_proj_elems(DT);
+    const int64_t left = sg.numel[lo] - s;
+    tp = (char*)sg.ptr[lo] + s * (int64_t)sizeof(S);
+    ap = (const char*)sg.anchor[lo] + s * (int64_t)sizeof(S);
+    n = (uint32_t)(left < short_proj_elems(DT) ? left : short_proj_elems(DT));
+    grp = sg.group_base + lo;
+  } else {
+    const DzChunk ch = a.chunks[c];
+    tp = (char*)ch.ptr;
+    ap = (const char*)ch.aux;
+    n = ch.n;
+    grp = ch.meta;
+    first = kSums ? a.group_begin[grp] : 0u;
+    count = kSums ? a.group_begin[grp + 1] - first : 0u;
+  }
+  dz_u32x4 vt[kVecs], va[kVecs];
+#pragma unroll
+  for (int u = 0; u < kVecs; ++u) {
+    const uint32_t e = (threadIdx.x + (uint32_t)u * kShortProjThreads) * kPer;
+    if (e + kPer <= n) {
+      vt[u] = ld_any(tp + (size_t)e * sizeof(S));
+      va[u] = ld_any(ap + (size_t)e * sizeof(S));
+    }
+  }
+  const ProjScalars<DT, MODE> ps(group_alpha<DT, MODE>(a.alpha, grp));
+  double acc = 0.0;
+#pragma unroll
+  for (int u = 0; u < kVecs; ++u) {
+    const uint32_t e = (threadIdx.x + (uint32_t)u * kShortProjThreads) * kPer;
+    if (e + kPer <= n) {
+      const dz_u32x4 o = proj_vec<DT, MODE>(vt[u], va[u], ps, &acc);
+      if constexpr (MODE != kProjSumsq) st_any(tp + (size_t)e * sizeof(S), o);
+    } else if (e < n) {
+      proj_tail<DT, MODE>(tp, ap, e, n, ps.alpha, &acc);
+    }
+  }
+  if constexpr (kSums) {
+    const double t = block_sum_f64(acc, red);
+    if (publish_partial(a.partials + c, t, a.group_done + (size_t)grp * kDoneStride, count, &flag)) {
+      double x = 0.0;
+      for (uint32_t i = threadIdx.x; i < count; i += kShortProjThreads) x += read_partial(a.partials + first + i);
+      const double sum = block_sum_f64(x, red);
+      if (threadIdx.x == 0) write_group<DT>(a.out, grp, sum, true);
+    }
   }
 }
 
@@ -2016,6 +2122,46 @@ hipError_t launch_proj(int dtype, int mode, const DzChunk* chunks, uint32_t nchu
       return launch_proj_dt<DZ_BF16>(mode, chunks, nchunks, ngroups, grid, alpha, partials, counters, st, ev);
     default: return hipErrorInvalidValue;
   }
+}
+
+template <int DT>
+static hipError_t launch_proj_short_dt(int mode, uint32_t nchunks, const ProjShort& a, hipStream_t st,
+                                       const LaunchEvents& ev) {
+  const dim3 grid(nchunks), block(kShortProjThreads);
+  const NoGroups none{};
+  switch (mode) {
+    case kProjSumsq: DZ_LAUNCH((proj_short_kernel<DT, kProjSumsq, NoGroups>), grid, block, st, ev, a, none); break;
+    case kProjApply: DZ_LAUNCH((proj_short_kernel<DT, kProjApply, NoGroups>), grid, block, st, ev, a, none); break;
+    case kProjReverse: DZ_LAUNCH((proj_short_kernel<DT, kProjReverse, NoGroups>), grid, block, st, ev, a, none); break;
+    case kProjReverseSumsq:
+      DZ_LAUNCH((proj_short_kernel<DT, kProjReverseSumsq, NoGroups>), grid, block, st, ev, a, none);
+      break;
+    case kProjApplyF32: DZ_LAUNCH((proj_short_kernel<DT, kProjApplyF32, NoGroups>), grid, block, st, ev, a, none); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_proj_short(int dtype, int mode, uint32_t nchunks, const ProjShort& a, hipStream_t st,
+                             const LaunchEvents& ev) {
+  switch (dtype) {
+    case DZ_F32: return launch_proj_short_dt<DZ_F32>(mode, nchunks, a, st, ev);
+    case DZ_F16: return launch_proj_short_dt<DZ_F16>(mode, nchunks, a, st, ev);
+    case DZ_BF16: return launch_proj_short_dt<DZ_BF16>(mode, nchunks, a, st, ev);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, const ProjShort& a, const StaticGroups& sg, hipStream_t st) {
+  const LaunchEvents ev{};
+  const dim3 grid(nchunks), block(kShortProjThreads);
+  switch (dtype) {
+    case DZ_F32: DZ_LAUNCH((proj_short_kernel<DZ_F32, kProjSumsq, StaticGroups>), grid, block, st, ev, a, sg); break;
+    case DZ_F16: DZ_LAUNCH((proj_short_kernel<DZ_F16, kProjSumsq, StaticGroups>), grid, block, st, ev, a, sg); break;
+    case DZ_BF16: DZ_LAUNCH((proj_short_kernel<DZ_BF16, kProjSumsq, StaticGroups>), grid, block, st, ev, a, sg); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
 }
 
 hipError_t launch_dot(int dtype, const DzChunk* chunks, uint32_t nchunks, const DzPtrArray& other,
