@@ -923,13 +923,22 @@ int32_t dz_group_dot(dz_table* t, const uint64_t* other_ptrs, double* d_dot, flo
     const int32_t g1 = std::min<int32_t>(t->n, g0 + dz::kMaxDotGroups);
     const uint32_t c0 = t->group_begin[g0], c1 = t->group_begin[g1];
     if (c1 == c0) continue;
-    dz::DzPtrArray other{};
-    for (int32_t i = g0; i < g1; ++i) other.p[i - g0] = other_ptrs[i];
-    e = dz::launch_dot(t->dtype, t->d_chunks + c0, c1 - c0, other, (uint32_t)g0, t->d_partials + c0,
-                       (hipStream_t)stream, {ev.start, nullptr});
+    dz::DotGroups dg{};
+    dg.group_base = (uint32_t)g0;
+    dg.chunk_base = c0;
+    for (int32_t i = g0; i < g1; ++i) dg.other[i - g0] = other_ptrs[i];
+    if (t->short_proj) {
+      const dz::ProjShort a{t->d_chunks, t->d_group_begin, t->d_group_done, nullptr, t->d_partials, {d_dot, d_dot_f32, nullptr}};
+      e = dz::launch_dot_short(t->dtype, c1 - c0, a, dg, (hipStream_t)stream, {ev.start, g1 == t->n ? ev.stop : nullptr});
+    } else {
+      const uint32_t grid = std::min<uint32_t>(c1 - c0, (uint32_t)t->dev->cus);
+      e = dz::launch_dot(t->dtype, t->d_chunks + c0, c1 - c0, grid, dg, t->d_partials + c0, t->d_counters,
+                         (hipStream_t)stream, {ev.start, nullptr});
+    }
     if (e != hipSuccess) return hip_fail(e, "dot kernel launch");
     ev.start = nullptr;
   }
+  if (t->short_proj) return DZ_OK;  // its launches write the groups' results
   e = dz::launch_finalize(t->dtype, t->d_partials, t->d_group_begin, (uint32_t)t->n, d_dot, d_dot_f32, nullptr,
                           false, (hipStream_t)stream, ev);
   if (e != hipSuccess) return hip_fail(e, "finalize kernel launch");

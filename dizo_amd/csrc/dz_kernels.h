@@ -23,12 +23,20 @@ enum ProjMode : int {
   kProjReverse = 2,       // theta <- R(R(R(theta - theta0) / alpha) + theta0)
   kProjReverseSumsq = 3,  // REVERSE, then the sums of the new theta
   kProjApplyF32 = 4,      // theta <- R_T(fp32(R(theta - theta0)) * alpha + theta0), alpha fp32
+  kProjDot = 5,           // per-chunk sums of fp32(other) * fp32(R_T(theta - theta0))
 };
+// Modes that write theta (and read an alpha), and modes that sum.
+__host__ __device__ constexpr bool proj_stores(int mode) { return mode != kProjSumsq && mode != kProjDot; }
+__host__ __device__ constexpr bool proj_sums(int mode) {
+  return mode == kProjSumsq || mode == kProjReverseSumsq || mode == kProjDot;
+}
 // Most groups one dot launch takes (their pointers travel as kernel
 // arguments); dz_group_dot launches once per batch of groups.
 constexpr int kMaxDotGroups = 128;
-struct DzPtrArray {
-  uint64_t p[kMaxDotGroups];
+struct DotGroups {
+  uint64_t other[kMaxDotGroups];  // of groups group_base, group_base + 1, ...
+  uint32_t group_base;
+  uint32_t chunk_base;  // short tables: the launch's first chunk in the table's list
 };
 
 // Read-modify-write kernel geometry. A workgroup of 1024 threads takes one
@@ -223,11 +231,13 @@ struct StaticGroups {
 };
 hipError_t launch_proj_short(int dtype, int mode, uint32_t nchunks, const ProjShort& a, hipStream_t st,
                              const LaunchEvents& ev = {});
+// DOT launches, over the chunks of the groups in dg. The first: persistent, as
+// launch_proj.
+hipError_t launch_dot(int dtype, const DzChunk* chunks, uint32_t nchunks, uint32_t grid, const DotGroups& dg,
+                      double* partials, uint32_t* counters, hipStream_t st, const LaunchEvents& ev = {});
+hipError_t launch_dot_short(int dtype, uint32_t nchunks, const ProjShort& a, const DotGroups& dg, hipStream_t st,
+                            const LaunchEvents& ev = {});
 hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, const ProjShort& a, const StaticGroups& sg, hipStream_t st);
-// Chunks of groups group_base .. group_base + kMaxDotGroups - 1; other.p[i]
-// is the tensor of group group_base + i.
-hipError_t launch_dot(int dtype, const DzChunk* chunks, uint32_t nchunks, const DzPtrArray& other,
-                      uint32_t group_base, double* partials, hipStream_t st, const LaunchEvents& ev = {});
 // take_sqrt: norms (sqrt of the sums) or plain sums in the fp32 / T outputs.
 hipError_t launch_finalize(int dtype, const double* partials, const uint32_t* gbegin, uint32_t ngroups,
                            double* sumsq, float* norm_f32, void* norm_T, bool take_sqrt, hipStream_t st,

@@ -586,12 +586,13 @@ __device__ __forceinline__ DzChunk uniform_chunk(const DzChunk& c) {
 }
 
 // The same for a projection chunk, whose anchor address (aux) is used and
-// whose z group is not.
+// whose element offset (zgroup) only DOT reads.
+template <bool kOffset>
 __device__ __forceinline__ DzChunk uniform_proj_chunk(const DzChunk& c) {
   DzChunk u;
   u.ptr = rfl_u64(c.ptr);
   u.aux = rfl_u64(c.aux);
-  u.zgroup = 0;
+  u.zgroup = kOffset ? rfl_u64(c.zgroup) : 0;
   u.n = rfl_u32(c.n);
   u.meta = rfl_u32(c.meta);
   return u;
@@ -1352,6 +1353,11 @@ __global__ void __launch_bounds__(kRmwThreads, DT == DZ_F32 ? 4 : 8)
 //   APPLY_F32      theta <- R_T(fp32(R_T(theta - theta0)) * alpha + theta0) with an fp32 alpha:
 //                  the first-order path's apply (trainer.py:428-436 with gamma an fp32
 //                  Parameter, so v and temp stay fp32 and copy_ rounds once)
+//   DOT            partial[c] = sum over chunk of fp32(other) * fp32(R_T(theta - theta0)), other a third
+//                  tensor per group: the gradient of the first-order objective with respect to
+//                  alpha (trainer.py:428-429 under autograd). One workgroup per chunk with an
+//                  element per load took 615 us over 64 x 6,553,600 fp16 elements, these loops
+//                  take 383 (6.6 TB/s)
 // Each chunk is processed by one workgroup; squares and sums in fp64 (exact
 // squares of the fp32-widened differences) in a fixed reduction order, so the
 // per-chunk partials, and the group sums built from them, are deterministic.
@@ -1520,6 +1526,32 @@ __device__ __forceinline__ dz_u32x4 proj_vec(dz_u32x4 vt, dz_u32x4 va, const Pro
   }
   return o;
 }
+// DOT: sum of fp32(other) * fp32(R_T(theta - theta0)) over one vector (fp64:
+// products of two fp32 values are exact, so each sum is rounded once).
+template <int DT>
+__device__ __forceinline__ void dot_vec(dz_u32x4 vt, dz_u32x4 va, dz_u32x4 vo, double* acc) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (DT == DZ_F32) {
+      const float d = __uint_as_float(vt[i]) - __uint_as_float(va[i]);
+      *acc = __builtin_fma((double)__uint_as_float(vo[i]), (double)d, *acc);
+    } else {
+      const F32Pair d = widen_pair<DT>(sub_pair<DT>(vt[i], va[i])), o = widen_pair<DT>(vo[i]);
+      *acc = __builtin_fma((double)o.lo, (double)d.lo, *acc);
+      *acc = __builtin_fma((double)o.hi, (double)d.hi, *acc);
+    }
+  }
+}
+template <int DT>
+__device__ __forceinline__ void dot_tail(const char* tp, const char* ap, const char* op, uint32_t e, uint32_t n,
+                                         double* acc) {
+  using S = typename DT_<DT>::S;
+  for (; e < n; ++e) {
+    const float d = rt<DT>(DT_<DT>::to_f((uint32_t)((const S*)tp)[e]) - DT_<DT>::to_f((uint32_t)((const S*)ap)[e]));
+    *acc = __builtin_fma((double)DT_<DT>::to_f((uint32_t)((const S*)op)[e]), (double)d, *acc);
+  }
+}
+
 // Elements e .. n - 1 of a chunk, one by one (its last, incomplete vector; the
 // rest of a partial chunk goes vector by vector. With all of it one by one, and
 // misaligned groups too, 128 groups of 20,480 fp16 elements took 26 us to apply,
@@ -1536,18 +1568,20 @@ __device__ __forceinline__ void proj_tail(char* tp, const char* ap, uint32_t e, 
 }
 
 // Vector-memory operations a thread issues for a full chunk: its 16-byte
-// loads of theta and theta0, and its stores of theta (none for SUMSQ).
+// loads of theta and theta0, and its stores of theta (none for SUMSQ; for DOT
+// the loads of the third tensor).
 template <int DT, int MODE>
 struct ProjChunkOps {
   static constexpr int kVecs = proj_chunk_elems(DT) / (kProjThreads * (16 / (int)sizeof(typename DT_<DT>::S)));
-  static constexpr int kAfterTicket = 2 * kVecs + (MODE == kProjSumsq ? 0 : kVecs);
+  static constexpr int kAfterTicket = 2 * kVecs + (MODE == kProjSumsq ? 0 : kVecs);  // DOT: a third load
 };
 
 // One chunk of a projection launch: the chunk's elements read (theta and
 // theta0), updated and written back, and for the SUMSQ modes the chunk's
 // partial sum (fixed reduction order) stored at *partial.
 template <int DT, int MODE>
-__device__ __forceinline__ void proj_chunk(const DzChunk& ch, float alpha, double* partial, double* red) {
+__device__ __forceinline__ void proj_chunk(const DzChunk& ch, float alpha, const char* op, double* partial,
+                                           double* red) {
   using S = typename DT_<DT>::S;
   constexpr int kES = (int)sizeof(S);
   char* tp = (char*)ch.ptr;
@@ -1556,31 +1590,42 @@ __device__ __forceinline__ void proj_chunk(const DzChunk& ch, float alpha, doubl
   if (proj_full_chunk<DT>(ch)) {
     constexpr int kVecsPerThread = ProjChunkOps<DT, MODE>::kVecs;
     const ProjScalars<DT, MODE> ps(alpha);
-    dz_u32x4 vt[kVecsPerThread], va[kVecsPerThread];
+    dz_u32x4 vt[kVecsPerThread], va[kVecsPerThread], vo[MODE == kProjDot ? kVecsPerThread : 1];
 #pragma unroll
     for (int u = 0; u < kVecsPerThread; ++u) {
       const size_t off = (size_t)(threadIdx.x + u * kProjThreads) * 16;
       vt[u] = ld_stream(tp + off);
       va[u] = ld_stream(ap + off);
+      if constexpr (MODE == kProjDot) vo[u] = ld_stream(op + off);
     }
 #pragma unroll
     for (int u = 0; u < kVecsPerThread; ++u) {
+      if constexpr (MODE == kProjDot) {
+        dot_vec<DT>(vt[u], va[u], vo[u], &acc);
+        continue;
+      }
       const dz_u32x4 o = proj_vec<DT, MODE>(vt[u], va[u], ps, &acc);
-      if constexpr (MODE != kProjSumsq) st_stream(tp + (size_t)(threadIdx.x + u * kProjThreads) * 16, o);
+      if constexpr (proj_stores(MODE)) st_stream(tp + (size_t)(threadIdx.x + u * kProjThreads) * 16, o);
     }
   } else {
     const ProjScalars<DT, MODE> ps(alpha);
     constexpr uint32_t kPer = 16 / kES;
     for (uint32_t e = threadIdx.x * kPer; e < ch.n; e += kProjThreads * kPer) {
-      if (e + kPer <= ch.n) {
+      if constexpr (MODE == kProjDot) {
+        const size_t off = (size_t)e * kES;
+        if (e + kPer <= ch.n)
+          dot_vec<DT>(ld_stream(tp + off), ld_stream(ap + off), ld_stream(op + off), &acc);
+        else
+          dot_tail<DT>(tp, ap, op, e, ch.n, &acc);
+      } else if (e + kPer <= ch.n) {
         const dz_u32x4 o = proj_vec<DT, MODE>(ld_stream(tp + (size_t)e * kES), ld_stream(ap + (size_t)e * kES), ps, &acc);
-        if constexpr (MODE != kProjSumsq) st_stream(tp + (size_t)e * kES, o);
+        if constexpr (proj_stores(MODE)) st_stream(tp + (size_t)e * kES, o);
       } else {
         proj_tail<DT, MODE>(tp, ap, e, ch.n, alpha, &acc);
       }
     }
   }
-  if constexpr (MODE == kProjSumsq || MODE == kProjReverseSumsq) {
+  if constexpr (proj_sums(MODE)) {
     const double t = block_sum_f64(acc, red);
     if (threadIdx.x == 0) *partial = t;
   }
@@ -1589,7 +1634,7 @@ __device__ __forceinline__ void proj_chunk(const DzChunk& ch, float alpha, doubl
 // alpha of a group: one value of T, or fp32 for APPLY_F32; none for SUMSQ.
 template <int DT, int MODE>
 __device__ __forceinline__ float group_alpha(const void* __restrict__ alpha_T, uint32_t grp) {
-  if constexpr (MODE == kProjSumsq) {
+  if constexpr (!proj_stores(MODE)) {
     return 0.0f;
   } else if constexpr (MODE == kProjApplyF32) {
     return ((const float*)alpha_T)[grp];
@@ -1597,6 +1642,8 @@ __device__ __forceinline__ float group_alpha(const void* __restrict__ alpha_T, u
     return DT_<DT>::to_f((uint32_t)((const typename DT_<DT>::S*)alpha_T)[grp]);
   }
 }
+
+struct NoGroups {};  // no per-group arguments: the chunks come from the table's list
 
 // Persistent projection kernel: one 1024-thread workgroup per CU takes chunks
 // from the table's work counters, as the RMW kernel does (counter j of the K
@@ -1606,16 +1653,16 @@ __device__ __forceinline__ float group_alpha(const void* __restrict__ alpha_T, u
 // lane 0 takes the index of chunk k + 3 and the wave loads the descriptor of
 // chunk k + 2 with scalar loads, so no descriptor latency sits between two
 // chunks. The last workgroup to finish resets the counters.
-template <int DT, int MODE>
+template <int DT, int MODE, class Groups>
 __global__ void __launch_bounds__(kProjThreads) proj_kernel(const DzChunk* __restrict__ chunks, uint32_t nchunks,
                                                             uint32_t ngroups, const void* __restrict__ alpha_T,
                                                             double* __restrict__ partials,
-                                                            uint32_t* __restrict__ counters) {
+                                                            uint32_t* __restrict__ counters, Groups dg) {
   __shared__ double red[kProjThreads / 64];
   __shared__ uint32_t sidx[4];   // chunk indices of k .. k + 3 (ring)
   __shared__ DzChunk sdesc[3];   // descriptors of k .. k + 2
-  __shared__ float salpha[MODE == kProjSumsq ? 1 : kProjAlphaLds];
-  const bool alpha_in_lds = MODE != kProjSumsq && ngroups <= (uint32_t)kProjAlphaLds;
+  __shared__ float salpha[proj_stores(MODE) ? kProjAlphaLds : 1];
+  const bool alpha_in_lds = proj_stores(MODE) && ngroups <= (uint32_t)kProjAlphaLds;
   if (alpha_in_lds) {
     for (uint32_t g = threadIdx.x; g < ngroups; g += kProjThreads) salpha[g] = group_alpha<DT, MODE>(alpha_T, g);
   }
@@ -1640,13 +1687,16 @@ __global__ void __launch_bounds__(kProjThreads) proj_kernel(const DzChunk* __res
   for (uint32_t k = 0;; ++k) {
     const uint32_t c = sidx[k % 4];
     if (c >= nchunks) break;
-    const DzChunk ch = uniform_proj_chunk(sdesc[k % 3]);
+    const DzChunk ch = uniform_proj_chunk<MODE == kProjDot>(sdesc[k % 3]);
     const uint32_t grp = ch.meta;
-    const float alpha = MODE == kProjSumsq ? 0.0f
+    const float alpha = !proj_stores(MODE) ? 0.0f
                         : alpha_in_lds     ? salpha[grp]
                                            : group_alpha<DT, MODE>(alpha_T, grp);
+    const char* op = nullptr;
+    if constexpr (MODE == kProjDot)
+      op = (const char*)dg.other[grp - dg.group_base] + ch.zgroup * sizeof(typename DT_<DT>::S);
     uint32_t grabbed = 0;
-    uint64_t n_ptr = 0, n_aux = 0;
+    uint64_t n_ptr = 0, n_aux = 0, n_off = 0;
     uint32_t n_n = 0, n_meta = 0;
     bool have_desc = false;
     if ((rfl_u32(threadIdx.x) >> 6) == 0) {  // wave 0 (uniform branch)
@@ -1656,6 +1706,7 @@ __global__ void __launch_bounds__(kProjThreads) proj_kernel(const DzChunk* __res
         const DzChunk* src = chunks + cd;
         n_ptr = src->ptr;
         n_aux = src->aux;
+        if constexpr (MODE == kProjDot) n_off = src->zgroup;
         n_n = src->n;
         n_meta = src->meta;
         have_desc = true;
@@ -1666,10 +1717,10 @@ __global__ void __launch_bounds__(kProjThreads) proj_kernel(const DzChunk* __res
     // partial path waits for everything), and the barrier that ends the chunk
     // waits for LDS alone
     if (proj_full_chunk<DT>(ch)) {
-      proj_chunk<DT, MODE>(ch, alpha, partials + c, red);
+      proj_chunk<DT, MODE>(ch, alpha, op, partials + c, red);
       if (threadIdx.x == 0) ticket_wait<ProjChunkOps<DT, MODE>::kAfterTicket>();
     } else {
-      proj_chunk<DT, MODE>(ch, alpha, partials + c, red);
+      proj_chunk<DT, MODE>(ch, alpha, op, partials + c, red);
       if (threadIdx.x == 0) ticket_wait<0>();
     }
     if (threadIdx.x == 0) {
@@ -1679,7 +1730,7 @@ __global__ void __launch_bounds__(kProjThreads) proj_kernel(const DzChunk* __res
         DzChunk& d = sdesc[(k + 2) % 3];
         d.ptr = n_ptr;
         d.aux = n_aux;
-        d.zgroup = 0;
+        d.zgroup = n_off;
         d.n = n_n;
         d.meta = n_meta;
       }
@@ -1692,32 +1743,6 @@ __global__ void __launch_bounds__(kProjThreads) proj_kernel(const DzChunk* __res
       for (int i = 0; i <= kDoneSlot; ++i) atomicExch(counters + i * kCounterStride, 0u);
     }
   }
-}
-
-// Per-group dot products with other tensors of the same shapes:
-//   partial[c] = sum over chunk of fp32(other) * fp32(R_T(theta - theta0))
-// (fp64 products of fp32 values are exact; fp64 sums). The gradient of the
-// first-order objective with respect to alpha: trainer.py:428-429 under
-// autograd gives sum(fp32(grad theta') * fp32(delta)) per projected tensor.
-template <int DT>
-__global__ void __launch_bounds__(kProjThreads) dot_kernel(const DzChunk* __restrict__ chunks, DzPtrArray other,
-                                                           uint32_t group_base, double* __restrict__ partials) {
-  using S = typename DT_<DT>::S;
-  constexpr int kES = (int)sizeof(S);
-  __shared__ double red[kProjThreads / 64];
-  const uint32_t c = blockIdx.x;
-  const DzChunk ch = chunks[c];
-  const uint32_t grp = ch.meta;
-  const S* tp = (const S*)ch.ptr;
-  const S* ap = (const S*)ch.aux;
-  const S* op = (const S*)(other.p[grp - group_base] + ch.zgroup * (uint64_t)kES);
-  double acc = 0.0;
-  for (uint32_t e = threadIdx.x; e < ch.n; e += kProjThreads) {
-    const float d = rt<DT>(DT_<DT>::to_f((uint32_t)tp[e]) - DT_<DT>::to_f((uint32_t)ap[e]));
-    acc += (double)DT_<DT>::to_f((uint32_t)op[e]) * (double)d;
-  }
-  const double t = block_sum_f64(acc, red);
-  if (threadIdx.x == 0) partials[c] = t;
 }
 
 // A group's results from the sum t of its chunks' partials.
@@ -1779,19 +1804,18 @@ __device__ __forceinline__ double read_partial(const double* slot) {
   return __builtin_bit_cast(double, __hip_atomic_load((const uint64_t*)slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
-struct NoGroups {};  // the chunks come from the table's list
 template <int DT, int MODE, class Groups>
 __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort a, Groups sg) {
   constexpr bool kStatic = std::is_same<Groups, StaticGroups>::value;
   using S = typename DT_<DT>::S;
   constexpr uint32_t kPer = 16 / (uint32_t)sizeof(S);
   constexpr int kVecs = short_proj_elems(DT) / (kShortProjThreads * (int)kPer);
-  constexpr bool kSums = MODE == kProjSumsq || MODE == kProjReverseSumsq;
+  constexpr bool kSums = proj_sums(MODE);
   __shared__ double red[kShortProjThreads / 64];
   __shared__ uint32_t flag;
   uint32_t c = blockIdx.x, grp, first, count;
   char* tp;
-  const char* ap;
+  const char *ap, *op = nullptr;
   uint32_t n;
   if constexpr (kStatic) {
     uint32_t lo = 0, hi = sg.ngroups;  // the group whose chunks hold c
@@ -1811,6 +1835,7 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
     n = (uint32_t)(left < short_proj_elems(DT) ? left : short_proj_elems(DT));
     grp = sg.group_base + lo;
   } else {
+    if constexpr (MODE == kProjDot) c += sg.chunk_base;
     const DzChunk ch = a.chunks[c];
     tp = (char*)ch.ptr;
     ap = (const char*)ch.aux;
@@ -1818,14 +1843,16 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
     grp = ch.meta;
     first = kSums ? a.group_begin[grp] : 0u;
     count = kSums ? a.group_begin[grp + 1] - first : 0u;
+    if constexpr (MODE == kProjDot) op = (const char*)sg.other[grp - sg.group_base] + ch.zgroup * sizeof(S);
   }
-  dz_u32x4 vt[kVecs], va[kVecs];
+  dz_u32x4 vt[kVecs], va[kVecs], vo[MODE == kProjDot ? kVecs : 1];
 #pragma unroll
   for (int u = 0; u < kVecs; ++u) {
     const uint32_t e = (threadIdx.x + (uint32_t)u * kShortProjThreads) * kPer;
     if (e + kPer <= n) {
       vt[u] = ld_any(tp + (size_t)e * sizeof(S));
       va[u] = ld_any(ap + (size_t)e * sizeof(S));
+      if constexpr (MODE == kProjDot) vo[u] = ld_any(op + (size_t)e * sizeof(S));
     }
   }
   const ProjScalars<DT, MODE> ps(group_alpha<DT, MODE>(a.alpha, grp));
@@ -1833,9 +1860,14 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
 #pragma unroll
   for (int u = 0; u < kVecs; ++u) {
     const uint32_t e = (threadIdx.x + (uint32_t)u * kShortProjThreads) * kPer;
-    if (e + kPer <= n) {
+    if constexpr (MODE == kProjDot) {
+      if (e + kPer <= n)
+        dot_vec<DT>(vt[u], va[u], vo[u], &acc);
+      else if (e < n)
+        dot_tail<DT>(tp, ap, op, e, n, &acc);
+    } else if (e + kPer <= n) {
       const dz_u32x4 o = proj_vec<DT, MODE>(vt[u], va[u], ps, &acc);
-      if constexpr (MODE != kProjSumsq) st_any(tp + (size_t)e * sizeof(S), o);
+      if constexpr (proj_stores(MODE)) st_any(tp + (size_t)e * sizeof(S), o);
     } else if (e < n) {
       proj_tail<DT, MODE>(tp, ap, e, n, ps.alpha, &acc);
     }
@@ -1846,7 +1878,7 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
       double x = 0.0;
       for (uint32_t i = threadIdx.x; i < count; i += kShortProjThreads) x += read_partial(a.partials + first + i);
       const double sum = block_sum_f64(x, red);
-      if (threadIdx.x == 0) write_group<DT>(a.out, grp, sum, true);
+      if (threadIdx.x == 0) write_group<DT>(a.out, grp, sum, MODE != kProjDot);
     }
   }
 }
@@ -2085,24 +2117,24 @@ static hipError_t launch_proj_dt(int mode, const DzChunk* chunks, uint32_t nchun
                                  hipStream_t st, const LaunchEvents& ev) {
   switch (mode) {
     case kProjSumsq:
-      DZ_LAUNCH((proj_kernel<DT, kProjSumsq>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
-                         ngroups, alpha, partials, counters);
+      DZ_LAUNCH((proj_kernel<DT, kProjSumsq, NoGroups>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
+                         ngroups, alpha, partials, counters, NoGroups{});
       break;
     case kProjApply:
-      DZ_LAUNCH((proj_kernel<DT, kProjApply>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
-                         ngroups, alpha, partials, counters);
+      DZ_LAUNCH((proj_kernel<DT, kProjApply, NoGroups>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
+                         ngroups, alpha, partials, counters, NoGroups{});
       break;
     case kProjReverse:
-      DZ_LAUNCH((proj_kernel<DT, kProjReverse>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
-                         ngroups, alpha, partials, counters);
+      DZ_LAUNCH((proj_kernel<DT, kProjReverse, NoGroups>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
+                         ngroups, alpha, partials, counters, NoGroups{});
       break;
     case kProjReverseSumsq:
-      DZ_LAUNCH((proj_kernel<DT, kProjReverseSumsq>), dim3(grid), dim3(kProjThreads), st, ev, chunks,
-                         nchunks, ngroups, alpha, partials, counters);
+      DZ_LAUNCH((proj_kernel<DT, kProjReverseSumsq, NoGroups>), dim3(grid), dim3(kProjThreads), st, ev, chunks,
+                         nchunks, ngroups, alpha, partials, counters, NoGroups{});
       break;
     case kProjApplyF32:
-      DZ_LAUNCH((proj_kernel<DT, kProjApplyF32>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
-                         ngroups, alpha, partials, counters);
+      DZ_LAUNCH((proj_kernel<DT, kProjApplyF32, NoGroups>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks,
+                         ngroups, alpha, partials, counters, NoGroups{});
       break;
     default:
       return hipErrorInvalidValue;
@@ -2164,23 +2196,33 @@ hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, const ProjShort& a, 
   return hipGetLastError();
 }
 
-hipError_t launch_dot(int dtype, const DzChunk* chunks, uint32_t nchunks, const DzPtrArray& other,
-                      uint32_t group_base, double* partials, hipStream_t st, const LaunchEvents& ev) {
+template <int DT>
+static void launch_dot_dt(const DzChunk* chunks, uint32_t nchunks, uint32_t grid, const DotGroups& dg, double* partials,
+                          uint32_t* counters, hipStream_t st, const LaunchEvents& ev) {
+  const void* no_alpha = nullptr;
+  DZ_LAUNCH((proj_kernel<DT, kProjDot, DotGroups>), dim3(grid), dim3(kProjThreads), st, ev, chunks, nchunks, 0u, no_alpha,
+            partials, counters, dg);
+}
+
+hipError_t launch_dot(int dtype, const DzChunk* chunks, uint32_t nchunks, uint32_t grid, const DotGroups& dg,
+                      double* partials, uint32_t* counters, hipStream_t st, const LaunchEvents& ev) {
   switch (dtype) {
-    case DZ_F32:
-      DZ_LAUNCH((dot_kernel<DZ_F32>), dim3(nchunks), dim3(kProjThreads), st, ev, chunks, other,
-                         group_base, partials);
-      break;
-    case DZ_F16:
-      DZ_LAUNCH((dot_kernel<DZ_F16>), dim3(nchunks), dim3(kProjThreads), st, ev, chunks, other,
-                         group_base, partials);
-      break;
-    case DZ_BF16:
-      DZ_LAUNCH((dot_kernel<DZ_BF16>), dim3(nchunks), dim3(kProjThreads), st, ev, chunks, other,
-                         group_base, partials);
-      break;
-    default:
-      return hipErrorInvalidValue;
+    case DZ_F32: launch_dot_dt<DZ_F32>(chunks, nchunks, grid, dg, partials, counters, st, ev); break;
+    case DZ_F16: launch_dot_dt<DZ_F16>(chunks, nchunks, grid, dg, partials, counters, st, ev); break;
+    case DZ_BF16: launch_dot_dt<DZ_BF16>(chunks, nchunks, grid, dg, partials, counters, st, ev); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_dot_short(int dtype, uint32_t nchunks, const ProjShort& a, const DotGroups& dg, hipStream_t st,
+                            const LaunchEvents& ev) {
+  const dim3 grid(nchunks), block(kShortProjThreads);
+  switch (dtype) {
+    case DZ_F32: DZ_LAUNCH((proj_short_kernel<DZ_F32, kProjDot, DotGroups>), grid, block, st, ev, a, dg); break;
+    case DZ_F16: DZ_LAUNCH((proj_short_kernel<DZ_F16, kProjDot, DotGroups>), grid, block, st, ev, a, dg); break;
+    case DZ_BF16: DZ_LAUNCH((proj_short_kernel<DZ_BF16, kProjDot, DotGroups>), grid, block, st, ev, a, dg); break;
+    default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }

@@ -159,7 +159,7 @@ def test_packed_odd_groups_match_oracle(dt, first, sizes):
 def test_long_tables_match_short_ones(dt):
     """Groups that together make a long table (more than 3 * 2^24 elements), odd starts and sizes among
     them, against a table of each group by itself (a short one): the same bits from apply, fp32-alpha
-    apply and reverse, and norms equal to the fp64 sums' rounding."""
+    apply and reverse, and sums equal to the fp64 sums' rounding."""
     from dizo_amd import _lib as L
     from dizo_amd.table import ProjTable
     sizes = [30_000_001, 7, 12_345_678, 0, 9_000_003]
@@ -167,32 +167,41 @@ def test_long_tables_match_short_ones(dt):
     gen = torch.Generator(device="cuda").manual_seed(3)
     anchor = torch.empty(total + 1, dtype=DT_TORCH[dt], device="cuda").normal_(0, 0.02, generator=gen)
     theta = anchor + torch.empty_like(anchor).normal_(0, 4e-3, generator=gen)
+    other = torch.empty_like(anchor).normal_(0, 1e-2, generator=gen)
     alpha = torch.linspace(0.85, 1.1, G, device="cuda")
     alpha_t = alpha.to(DT_TORCH[dt])
     flats, sums = [], []
     for long in (True, False):
         flat = theta.clone()
         groups, anchors = list(flat[1:].split(sizes)), list(anchor[1:].split(sizes))
-        out = torch.full((3, G), -1.0, dtype=torch.float64, device="cuda")
+        others = list(other[1:].split(sizes))
+        out = torch.full((4, G), -1.0, dtype=torch.float64, device="cuda")
         for part in ([list(range(G))] if long else [[g] for g in range(G)]):
             tab = ProjTable([groups[g] for g in part], [anchors[g] for g in part])
             o, lo = out[:, part[0]:part[-1] + 1], part[0]
             hi = part[-1] + 1
-            s = [torch.empty(hi - lo, dtype=torch.float64, device="cuda") for _ in range(3)]
+            s = [torch.empty(hi - lo, dtype=torch.float64, device="cuda") for _ in range(4)]
+            tab.group_dot([others[g] for g in part], s[3])
             tab.group_sumsq(s[0])
             tab.project(alpha_t[lo:hi].contiguous(), L.DZ_PROJ_APPLY)
             tab.group_sumsq(s[1])
             tab.project(alpha_t[lo:hi].contiguous(), L.DZ_PROJ_REVERSE_SUMSQ, sumsq=s[2])
             tab.project(alpha[lo:hi].contiguous(), L.DZ_PROJ_APPLY_F32ALPHA)
-            for k in range(3):
+            for k in range(4):
                 o[k] = s[k]
             tab.close()
         flats.append(flat)
         sums.append(out.cpu().numpy())
     assert torch.equal(flats[0].view(torch.int32 if dt == F32 else torch.int16), flats[1].view(torch.int32 if dt == F32 else torch.int16))
     assert float(flats[0][0]) == float(theta[0])
-    np.testing.assert_allclose(sums[0], sums[1], rtol=max(sizes) * 2.0**-53, atol=0)
-    assert (sums[0][:, 3] == 0).all() and (sums[0][:, [0, 1, 2, 4]] > 0).all()
+    np.testing.assert_allclose(sums[0][:3], sums[1][:3], rtol=max(sizes) * 2.0**-53, atol=0)
+    assert (sums[0][:, 3] == 0).all() and (sums[0][:3, [0, 1, 2, 4]] > 0).all()
+    # dots: against torch's fp64 sums; the terms' signs differ, so the bound is on the sum of their sizes
+    for g in range(G):
+        terms = others[g].double() * (theta[1:].split(sizes)[g] - anchor[1:].split(sizes)[g]).double()
+        bound = float(terms.abs().sum()) * sizes[g] * 2.0**-53
+        for got in (sums[0][3, g], sums[1][3, g]):
+            assert abs(float(got) - float(terms.sum())) <= bound, g
 
 
 def test_empty_and_rejects():
