@@ -10,6 +10,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -319,8 +320,19 @@ int32_t rmw(dz_table* t, int mode, const dz::DzScalars& s, const dz::DzScalarPtr
   const dz::LaunchEvents ev = take_timing(t);
   if (t->projection) return fail(DZ_ERR_INVALID, "perturb/update need a ZO table (created without anchors)");
   if (t->short_nchunks > 0 && !t->persistent_only) {
+    // A scale of +-1 or +-2 (the step's own) goes into eps: R(s z) is then s z
+    // itself in every T, and fp32(s z * eps) rounds the same real number as
+    // fp32(z * (s eps)), with s eps exact. It takes a rounding and two products
+    // off each element (fp16 perturb over 2^24 elements 14.0 -> 13.0 us).
+    dz::DzScalars sx = s;
+    const float folded = s.scale * s.eps;
+    if (mode == dz::kModePerturb && (fabsf(s.scale) == 1.0f || fabsf(s.scale) == 2.0f) && std::isfinite(folded)) {
+      mode = dz::kModePerturbUnit;
+      sx.scale = 1.0f;
+      sx.eps = folded;
+    }
     const hipError_t e = dz::launch_rmw_short(t->dtype, mode, t->d_short_chunks, t->short_nchunks,
-                                              (uint32_t)t->dev->cus, t->dev->tab[t->dtype], s, p,
+                                              (uint32_t)t->dev->cus, t->dev->tab[t->dtype], sx, p,
                                               (hipStream_t)stream, ev);
     if (e != hipSuccess) return hip_fail(e, "rmw kernel launch");
     return DZ_OK;
@@ -352,20 +364,29 @@ int32_t proj_short(dz_table* t, int mode, const void* alpha, const dz::GroupOutp
 }
 
 // Tiles of `elems` elements over every registered tensor, in tensor order.
+// split_counters: a tile also ends where the Philox counter's low word wraps.
 void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
-                  std::vector<uint32_t>* group_begin) {
+                  std::vector<uint32_t>* group_begin, bool split_counters = false) {
   const int es = elem_size(t->dtype);
   out->clear();
   if (group_begin) group_begin->assign(1, 0u);
   for (int32_t i = 0; i < t->n; ++i) {
     const int64_t ne = t->numels[i];
     const uint64_t p = t->ptrs[i], a = t->aux[i], z = t->zoff[i];
-    for (int64_t s = 0; s < ne; s += elems) {
+    int64_t len = 0;
+    for (int64_t s = 0; s < ne; s += len) {
       DzChunk c;
+      len = (ne - s) < (int64_t)elems ? (ne - s) : (int64_t)elems;
+      if (split_counters) {
+        // the elements left before the Philox counter's low word wraps
+        const uint64_t q = (z + (uint64_t)s) >> 3;
+        const uint64_t room = ((1ull << 32) - (q & 0xffffffffull)) * 8u;
+        if ((uint64_t)len > room) len = (int64_t)room;
+      }
       c.ptr = p + (uint64_t)s * es;
       c.aux = t->projection ? a + (uint64_t)s * es : 0;
       c.zgroup = t->projection ? (uint64_t)s : (z + (uint64_t)s) >> 3;
-      c.n = (uint32_t)((ne - s) < (int64_t)elems ? (ne - s) : elems);
+      c.n = (uint32_t)len;
       c.meta = (uint32_t)i;
       out->push_back(c);
     }
@@ -605,7 +626,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
   }
   if (e == hipSuccess && !t->projection && t->bytes <= dz::short_elems(dtype) * es) {
     std::vector<DzChunk> sc;
-    build_chunks(t, dz::kShortTile, &sc, nullptr);
+    build_chunks(t, dz::kShortTile, &sc, nullptr, true);
     t->short_nchunks = (uint32_t)sc.size();
     e = upload_chunks(sc, &t->d_short_chunks);
   }

@@ -12,6 +12,7 @@ enum RmwMode : int {
   kModeUpdate = 1,                // theta - d(z)
   kModeRestoreUpdate = 2,         // theta + b(z) - d(z)
   kModeRestoreUpdatePerturb = 3,  // theta + b(z) - d(z) + b(z'), z' from a second seed
+  kModePerturbUnit = 4,           // perturb with scale 1 (rmw_short_kernel only)
 };
 // Modes whose table entries hold the pair (b, -d).
 __host__ __device__ constexpr bool rmw_pair_mode(int mode) {

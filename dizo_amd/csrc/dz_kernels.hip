@@ -1179,11 +1179,12 @@ __global__ void __launch_bounds__(kRmwThreads, kRmwWavesPerEU) rmw_kernel(const 
 // and the next pass (with the non-temporal hint, fp32, 2^24 elements: 30.5
 // against 22.6 us). Pass times in us (perturb / three-way), this kernel and the
 // persistent one with its hints: fp16 2^14 elements 4.0 / 4.1 and 6.8 / 9.0,
-// 2^20 4.3 / 4.4 and 10.2 / 14.3, 2^22 6.1 / 7.7 and 13.1 / 19.5, 2^25 22.2 /
-// 30.8 and 27.2 / 30.3; fp32 2^20 4.6 / 5.4 and 9.9 / 10.4, 2^24 22.7 / 23.5
-// and 27.6 / 28.2. A launch is bound by its latencies (about 4 us) up to 2^20
-// elements, then by the lookups (two in the three-way pass: about 8 clocks a
-// wave and lookup, which 2^25 elements' 30 us are) and the cache.
+// 2^20 4.2 / 4.3 and 10.2 / 14.3, 2^22 6.0 / 7.5 and 13.1 / 19.5, 2^24 12.8 /
+// 19.0, 2^25 21.1 / 30.7 and 27.2 / 30.3; fp32 2^20 4.6 / 5.4 and 9.9 / 10.4,
+// 2^24 21.8 / 22.9 and 27.6 / 28.2. A launch is bound by its latencies (about 4
+// us) up to 2^20 elements, then by the VALU: with one Philox round for seven,
+// fp16 2^25 elements take 21.4 / 22.4 us; with lookups free of bank conflicts,
+// the same time.
 // ---------------------------------------------------------------------------
 
 // The launch's operation on two packed 16-bit elements with their signed z
@@ -1191,7 +1192,7 @@ __global__ void __launch_bounds__(kRmwThreads, kRmwWavesPerEU) rmw_kernel(const 
 template <int DT, int MODE>
 __device__ __forceinline__ uint32_t apply_z_pair(uint32_t th, uint32_t z, uint32_t z2, const DzScalars& sc) {
   if constexpr (MODE == kModeUpdate) return add_pair<DT>(th, delta_nd_pair<DT>(z, sc));
-  uint32_t r = add_pair<DT>(th, delta_b_pair<DT, rmw_pair_mode(MODE)>(z, sc));
+  uint32_t r = add_pair<DT>(th, delta_b_pair<DT, MODE != kModePerturb>(z, sc));
   if constexpr (rmw_pair_mode(MODE)) r = add_pair<DT>(r, delta_nd_pair<DT>(z, sc));
   if constexpr (MODE == kModeRestoreUpdatePerturb) r = add_pair<DT>(r, delta_b_pair<DT, true>(z2, sc));
   return r;
@@ -1201,6 +1202,7 @@ template <int MODE>
 __device__ __forceinline__ uint32_t apply_z_f32(uint32_t th, uint32_t z, uint32_t z2, const DzScalars& sc) {
   const float zf = __uint_as_float(z);
   if constexpr (MODE == kModePerturb) return op_perturb<DZ_F32>(__uint_as_float(th), zf, sc.scale, sc.eps);
+  if constexpr (MODE == kModePerturbUnit) return op_perturb<DZ_F32>(__uint_as_float(th), zf, 1.0f, sc.eps);
   if constexpr (MODE == kModeUpdate) return op_update<DZ_F32>(__uint_as_float(th), zf, sc.grad, sc.lr);
   uint32_t r = op_perturb<DZ_F32>(__uint_as_float(th), zf, 1.0f, sc.eps);
   r = op_update<DZ_F32>(__uint_as_float(r), zf, sc.grad, sc.lr);
@@ -1315,7 +1317,9 @@ __global__ void __launch_bounds__(kRmwThreads, DT == DZ_F32 ? 4 : 8)
   const DzScalars sc = resolve_scalars<DT>(sc_in, sp);
   __syncthreads();
   for (;;) {
-    const uint64_t q = ch.zgroup + tile_group<DT>(0);
+    // the tile's counters share their high word (build_chunks), which stays on
+    // the scalar unit
+    const uint32_t q = (uint32_t)ch.zgroup + tile_group<DT>(0), q_hi = (uint32_t)(ch.zgroup >> 32);
     const uint32_t tn = t + gridDim.x;
     const bool more = tn < nchunks;
     ShortGroup<DT> nxt;
@@ -1324,8 +1328,9 @@ __global__ void __launch_bounds__(kRmwThreads, DT == DZ_F32 ? 4 : 8)
       nxt = ShortGroup<DT>(ch);
     }
     if (cur.wave_active()) {
-      const ZVec<DT> z = z_vec<DT>(tab, thread_words<DT>(dz_philox_group(sc.seed, kDzStreamParam, q)));
-      const ZVec<DT> z2 = kNext ? z_vec<DT>(tab, thread_words<DT>(dz_philox_group(sc.seed2, kDzStreamParam, q))) : z;
+      const ZVec<DT> z = z_vec<DT>(tab, thread_words<DT>(dz_philox_counter(sc.seed, kDzStreamParam, q, q_hi)));
+      const ZVec<DT> z2 =
+          kNext ? z_vec<DT>(tab, thread_words<DT>(dz_philox_counter(sc.seed2, kDzStreamParam, q, q_hi))) : z;
 #pragma unroll
       for (int k = 0; k < ZVec<DT>::kVecs; ++k) {
 #pragma unroll
@@ -2085,6 +2090,9 @@ static hipError_t launch_rmw_short_dt(int mode, const DzChunk* chunks, uint32_t 
   switch (mode) {
     case kModePerturb:
       DZ_LAUNCH((rmw_short_kernel<DT, kModePerturb>), grid, block, st, ev, chunks, nchunks, tab, s, p);
+      break;
+    case kModePerturbUnit:
+      DZ_LAUNCH((rmw_short_kernel<DT, kModePerturbUnit>), grid, block, st, ev, chunks, nchunks, tab, s, p);
       break;
     case kModeUpdate:
       DZ_LAUNCH((rmw_short_kernel<DT, kModeUpdate>), grid, block, st, ev, chunks, nchunks, tab, s, p);
