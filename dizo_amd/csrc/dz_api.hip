@@ -224,6 +224,7 @@ struct dz_table {
   std::vector<uint64_t> ptrs, aux, zoff;
   std::vector<int64_t> numels;
   std::vector<uint32_t> group_begin;  // n + 1 chunk indices (projection tables)
+  unsigned char* d_memory = nullptr;  // one allocation, which the pointers below point into
   DzChunk* d_chunks = nullptr;
   // ZO tables whose restore + update + next perturbation launches use another
   // tile size (rmw_chunk_elems): their own tile list, else empty
@@ -279,13 +280,7 @@ int32_t check_table(const dz_table* t) {
 }
 
 void free_table(dz_table* t) {
-  if (t->d_chunks) (void)hipFree(t->d_chunks);
-  if (t->d_fused_chunks) (void)hipFree(t->d_fused_chunks);
-  if (t->d_short_chunks) (void)hipFree(t->d_short_chunks);
-  if (t->d_group_begin) (void)hipFree(t->d_group_begin);
-  if (t->d_partials) (void)hipFree(t->d_partials);
-  if (t->d_group_done) (void)hipFree(t->d_group_done);
-  if (t->d_counters) (void)hipFree(t->d_counters);
+  if (t->d_memory) (void)hipFree(t->d_memory);
   delete t;
 }
 
@@ -450,12 +445,48 @@ int32_t check_no_overlap(const dz_table* t) {
   return DZ_OK;
 }
 
-hipError_t upload_chunks(const std::vector<DzChunk>& v, DzChunk** d) {
-  if (v.empty()) return hipSuccess;
-  hipError_t e = hipMalloc(d, v.size() * sizeof(DzChunk));
-  if (e == hipSuccess) e = hipMemcpy(*d, v.data(), v.size() * sizeof(DzChunk), hipMemcpyHostToDevice);
-  return e;
-}
+// A table's device memory: the parts given to it, in one allocation, each at a
+// multiple of 256 bytes. Parts without host data start at zero, or (clear
+// false) hold what they hold. Small tables go over in one copy: an allocation
+// or a copy costs the host 10 to 40 us, whatever its size.
+class TableMemory {
+ public:
+  template <class T>
+  void add(T** where, const void* host, size_t count, bool clear = true) {
+    parts_.push_back({(void**)where, host, count * sizeof(T), bytes_, clear});
+    bytes_ += (count * sizeof(T) + 255) / 256 * 256;
+  }
+  hipError_t upload(unsigned char** memory) {
+    hipError_t e = hipMalloc(memory, bytes_ ? bytes_ : 256);
+    if (e != hipSuccess) return e;
+    for (const Part& p : parts_) *p.where = p.bytes ? (void*)(*memory + p.at) : nullptr;
+    if (bytes_ <= kOneCopy) {
+      std::vector<unsigned char> all(bytes_, 0);
+      for (const Part& p : parts_)
+        if (p.host && p.bytes) memcpy(all.data() + p.at, p.host, p.bytes);
+      return bytes_ ? hipMemcpy(*memory, all.data(), bytes_, hipMemcpyHostToDevice) : hipSuccess;
+    }
+    for (const Part& p : parts_) {
+      if (e != hipSuccess || !p.bytes) continue;
+      if (p.host)
+        e = hipMemcpy(*memory + p.at, p.host, p.bytes, hipMemcpyHostToDevice);
+      else if (p.clear)
+        e = hipMemset(*memory + p.at, 0, p.bytes);
+    }
+    return e == hipSuccess ? hipDeviceSynchronize() : e;
+  }
+
+ private:
+  static constexpr size_t kOneCopy = 1 << 20;
+  struct Part {
+    void** where;
+    const void* host;
+    size_t bytes, at;
+    bool clear;
+  };
+  std::vector<Part> parts_;
+  size_t bytes_ = 0;
+};
 
 // The device address of `scratch` on device `dev` (current) and the device's
 // CU count, looked up once per device. In host code `scratch` names a host
@@ -610,45 +641,33 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     t->short_proj = true;
     t->chunk_elems = (uint32_t)dz::short_proj_elems(dtype);
   }
-  std::vector<DzChunk> chunks;
+  TableMemory mem;
+  std::vector<DzChunk> chunks, fused_chunks, short_chunks;
   build_chunks(t, t->chunk_elems, &chunks, t->projection ? &t->group_begin : nullptr);
   t->nchunks = (uint32_t)chunks.size();
   if (!t->projection) (void)full_tiles_first(&chunks, t->chunk_elems);
-  hipError_t e = upload_chunks(chunks, &t->d_chunks);
+  mem.add(&t->d_chunks, chunks.data(), chunks.size());
   const uint32_t fused = (uint32_t)dz::rmw_chunk_elems(dtype, dz::kModeRestoreUpdatePerturb);
-  if (e == hipSuccess && !t->projection && fused != t->chunk_elems) {
-    std::vector<DzChunk> fc;
-    build_chunks(t, fused, &fc, nullptr);
-    (void)full_tiles_first(&fc, fused);
+  if (!t->projection && fused != t->chunk_elems) {
+    build_chunks(t, fused, &fused_chunks, nullptr);
+    (void)full_tiles_first(&fused_chunks, fused);
     t->fused_elems = fused;
-    t->fused_nchunks = (uint32_t)fc.size();
-    e = upload_chunks(fc, &t->d_fused_chunks);
+    t->fused_nchunks = (uint32_t)fused_chunks.size();
+    mem.add(&t->d_fused_chunks, fused_chunks.data(), fused_chunks.size());
   }
-  if (e == hipSuccess && !t->projection && t->bytes <= dz::short_elems(dtype) * es) {
-    std::vector<DzChunk> sc;
-    build_chunks(t, dz::kShortTile, &sc, nullptr, true);
-    t->short_nchunks = (uint32_t)sc.size();
-    e = upload_chunks(sc, &t->d_short_chunks);
+  if (!t->projection && t->bytes <= dz::short_elems(dtype) * es) {
+    build_chunks(t, dz::kShortTile, &short_chunks, nullptr, true);
+    t->short_nchunks = (uint32_t)short_chunks.size();
+    mem.add(&t->d_short_chunks, short_chunks.data(), short_chunks.size());
   }
-  if (e == hipSuccess && t->projection) {
-    // The finalize kernel always runs, so these exist even with no chunks.
-    e = hipMalloc(&t->d_group_begin, t->group_begin.size() * sizeof(uint32_t));
-    if (e == hipSuccess)
-      e = hipMemcpy(t->d_group_begin, t->group_begin.data(), t->group_begin.size() * sizeof(uint32_t),
-                    hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMalloc(&t->d_partials, (size_t)(t->nchunks ? t->nchunks : 1) * sizeof(double));
-    if (e == hipSuccess && t->short_proj) {
-      const size_t bytes = (size_t)t->n * dz::kDoneStride * sizeof(uint32_t);
-      e = hipMalloc(&t->d_group_done, bytes);
-      if (e == hipSuccess) e = hipMemset(t->d_group_done, 0, bytes);
-    }
+  if (t->projection) {
+    mem.add(&t->d_group_begin, t->group_begin.data(), t->group_begin.size());
+    mem.add(&t->d_partials, nullptr, t->nchunks ? t->nchunks : 1, false);
+    if (t->short_proj) mem.add(&t->d_group_done, nullptr, (size_t)t->n * dz::kDoneStride);
   }
-  if (e == hipSuccess) {
-    // zeroed once here; every RMW and projection launch leaves them at zero again
-    e = hipMalloc(&t->d_counters, dz::kCounterWords * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMemset(t->d_counters, 0, dz::kCounterWords * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipDeviceSynchronize();
-  }
+  // work counters: zero here; every RMW and projection launch leaves them at zero again
+  mem.add(&t->d_counters, nullptr, dz::kCounterWords);
+  const hipError_t e = mem.upload(&t->d_memory);
   if (e != hipSuccess) {
     free_table(t);
     return hip_fail(e, "table upload");
