@@ -1431,8 +1431,8 @@ __device__ __forceinline__ void acc_sq_pair(uint32_t d, double* acc) {
 // pairs (RN_bf16 of the fp32 quotient is RN_bf16 of the exact quotient, since
 // fp32 carries 24 >= 2 * 8 + 2 bits, and for normal operands a bf16 quotient
 // is at least 2^-16 of itself away from a bf16 rounding midpoint, where the
-// product's error is under 2^-23). Elements outside that range divide. One
-// multiply replaces the IEEE division sequence per element.
+// product's error is under 2^-23). Vectors with an element outside that range
+// divide. One multiply replaces the IEEE division sequence per element.
 struct RecipDiv {
   float inv;  // fp32(1 / alpha)
   bool ok;    // inv is finite (alpha is neither 0, infinite nor below 2^-128)
@@ -1441,8 +1441,8 @@ __device__ __forceinline__ RecipDiv recip_div(float alpha) {
   const float inv = 1.0f / alpha;
   return RecipDiv{inv, __builtin_isfinite(inv) != 0};
 }
-__device__ __forceinline__ bool recip_quotient_ok(float q) {
-  return !(q != 0.0f && __builtin_fabsf(q) < 0x1p-126f);  // NaN, zero and normal quotients
+__device__ __forceinline__ bool recip_quotient_subnormal(float q) {
+  return __builtin_amdgcn_classf(q, 0x10 | 0x80);  // +- subnormal
 }
 
 // proj_elem for the two 16-bit elements of a word, in packed arithmetic where
@@ -1451,7 +1451,7 @@ __device__ __forceinline__ bool recip_quotient_ok(float q) {
 // (its fp32 alpha keeps v and the sum in fp32).
 template <int DT, int MODE>
 __device__ __forceinline__ uint32_t proj_word16(uint32_t th, uint32_t t0, uint32_t alpha2, float alpha,
-                                                const RecipDiv& rd, double* acc) {
+                                                double* acc) {
   const uint32_t d = sub_pair<DT>(th, t0);
   if constexpr (MODE == kProjSumsq) {
     acc_sq_pair<DT>(d, acc);
@@ -1460,14 +1460,6 @@ __device__ __forceinline__ uint32_t proj_word16(uint32_t th, uint32_t t0, uint32
     uint32_t v;
     if constexpr (MODE == kProjApply) {
       v = mul_pair<DT>(d, alpha2);
-    } else if constexpr (DT == DZ_BF16) {
-      const float x0 = bf16_lo_f(d), x1 = bf16_hi_f(d);
-      float v0 = x0 * rd.inv, v1 = x1 * rd.inv;
-      if (!(rd.ok && recip_quotient_ok(v0) && recip_quotient_ok(v1))) {
-        v0 = x0 / alpha;
-        v1 = x1 / alpha;
-      }
-      v = pack_bf16(v0, v1);
     } else {
       const float v0 = DT_<DT>::to_f(d & 0xffffu) / alpha;
       const float v1 = DT_<DT>::to_f(d >> 16) / alpha;
@@ -1514,19 +1506,47 @@ struct ProjScalars {
 template <int DT, int MODE>
 __device__ __forceinline__ dz_u32x4 proj_vec(dz_u32x4 vt, dz_u32x4 va, const ProjScalars<DT, MODE>& ps, double* acc) {
   dz_u32x4 o;
+  if constexpr (DT == DZ_BF16 && (MODE == kProjReverse || MODE == kProjReverseSumsq)) {
+    // the quotients of the whole vector by the reciprocal, or by division if one
+    // of them asks for it: one branch for eight elements (with one for two, the
+    // reverse + norm pass over 64 x 26,214,400 elements took 1684 us, 1622 now)
+    float q[8];
+    bool divide = !ps.rd.ok;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (DT != DZ_F32 && MODE != kProjApplyF32) {
-      o[i] = proj_word16<DT, MODE>(vt[i], va[i], ps.alpha2, ps.alpha, ps.rd, acc);
-    } else if constexpr (DT != DZ_F32) {
-      uint32_t r0, r1;
-      proj_elem<DT>(MODE, vt[i] & 0xffffu, va[i] & 0xffffu, ps.alpha, &r0, acc);
-      proj_elem<DT>(MODE, vt[i] >> 16, va[i] >> 16, ps.alpha, &r1, acc);
-      o[i] = (r0 & 0xffffu) | (r1 << 16);
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t d = sub_pair<DT>(vt[i], va[i]);
+      q[2 * i] = bf16_lo_f(d);
+      q[2 * i + 1] = bf16_hi_f(d);
+      divide |= recip_quotient_subnormal(q[2 * i] * ps.rd.inv);
+      divide |= recip_quotient_subnormal(q[2 * i + 1] * ps.rd.inv);
+    }
+    if (divide) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] /= ps.alpha;
     } else {
-      uint32_t r;
-      proj_elem<DT>(MODE, vt[i], va[i], ps.alpha, &r, acc);
-      o[i] = r;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] *= ps.rd.inv;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] = add_pair<DT>(pack_bf16(q[2 * i], q[2 * i + 1]), va[i]);
+      if constexpr (MODE == kProjReverseSumsq) acc_sq_pair<DT>(sub_pair<DT>(o[i], va[i]), acc);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (DT != DZ_F32 && MODE != kProjApplyF32) {
+        o[i] = proj_word16<DT, MODE>(vt[i], va[i], ps.alpha2, ps.alpha, acc);
+      } else if constexpr (DT != DZ_F32) {
+        uint32_t r0, r1;
+        proj_elem<DT>(MODE, vt[i] & 0xffffu, va[i] & 0xffffu, ps.alpha, &r0, acc);
+        proj_elem<DT>(MODE, vt[i] >> 16, va[i] >> 16, ps.alpha, &r1, acc);
+        o[i] = (r0 & 0xffffu) | (r1 << 16);
+      } else {
+        uint32_t r;
+        proj_elem<DT>(MODE, vt[i], va[i], ps.alpha, &r, acc);
+        o[i] = r;
+      }
     }
   }
   return o;

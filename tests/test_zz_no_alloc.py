@@ -79,6 +79,20 @@ def test_static_norms_equal_table_norms_two_calls(dt):
         assert float(got[0][3 if len(sizes) > 3 else 0]) >= 0.0
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+def test_static_norms_of_long_inputs_equal_table_norms(dt):
+    """More than 3 * 2^24 elements in 66 groups (the persistent kernel, its chunks planned on the device in
+    two launches), then a short call, then the long one again: the table's bits each time."""
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    sizes = [800_000 + 1000 * i for i in range(66)]
+    flat = torch.empty(sum(sizes), dtype=dt, device="cuda").normal_(0, 0.02, generator=gen)
+    base = flat + torch.empty_like(flat).normal_(0, 1e-3, generator=gen)
+    th, t0 = list(flat.split(sizes)), list(base.split(sizes))
+    for part in (slice(0, 66), slice(0, 5), slice(0, 66)):
+        for g, w, what in zip(_static(th[part], t0[part], dt), _table(th[part], t0[part], dt), ("sumsq", "norm_f32", "norm_T")):
+            assert torch.equal(_bits(g), _bits(w)), what
+
+
 def test_static_rejects_more_than_the_scratch_holds():
     dt = torch.float16
     th, t0 = _groups([8], dt, 3)
