@@ -231,7 +231,7 @@ struct dz_table {
   uint32_t fused_elems = 0;
   uint32_t fused_nchunks = 0;
   DzChunk* d_fused_chunks = nullptr;
-  // short ZO tables: the tile list of their launches (empty in longer tables)
+  // ZO tables with passes short enough for rmw_short_kernel: its tile list
   bool persistent_only = false;  // set by dz_table_set_prefetch_min_tiles
   uint32_t short_nchunks = 0;
   DzChunk* d_short_chunks = nullptr;
@@ -314,7 +314,8 @@ int32_t rmw(dz_table* t, int mode, const dz::DzScalars& s, const dz::DzScalarPtr
   if (rc) return rc;
   const dz::LaunchEvents ev = take_timing(t);
   if (t->projection) return fail(DZ_ERR_INVALID, "perturb/update need a ZO table (created without anchors)");
-  if (t->short_nchunks > 0 && !t->persistent_only) {
+  if (t->short_nchunks > 0 && !t->persistent_only &&
+      t->bytes <= dz::short_elems(t->dtype, mode) * (uint64_t)elem_size(t->dtype)) {
     // A scale of +-1 or +-2 (the step's own) goes into eps: R(s z) is then s z
     // itself in every T, and fp32(s z * eps) rounds the same real number as
     // fp32(z * (s eps)), with s eps exact. It takes a rounding and two products
@@ -655,7 +656,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     t->fused_nchunks = (uint32_t)fused_chunks.size();
     mem.add(&t->d_fused_chunks, fused_chunks.data(), fused_chunks.size());
   }
-  if (!t->projection && t->bytes <= dz::short_elems(dtype) * es) {
+  if (!t->projection && t->bytes <= dz::short_elems(dtype, dz::kModePerturb) * es) {
     build_chunks(t, dz::kShortTile, &short_chunks, nullptr, true);
     t->short_nchunks = (uint32_t)short_chunks.size();
     mem.add(&t->d_short_chunks, short_chunks.data(), short_chunks.size());

@@ -67,14 +67,26 @@ __host__ __device__ constexpr int rmw_chunk_elems(int dtype, int mode) {
   return kRmwThreads * rmw_groups(dtype, mode) * 8;
 }
 
-// Short tables: up to short_elems(dtype) elements in all, whose passes run
-// rmw_short_kernel over tiles of kShortTile elements. Where the line lies: the
-// two passes of a steady step, against the persistent kernel with plain
-// accesses (what tables just above the line run best): fp16 2^24 elements 32.6
-// and 41.5 us, 2^25 53.0 and 52.2, 2^26 96.7 and 87.5; fp32 2^23 26.8 and 31.1,
-// 2^24 44.9 and 46.2, 2^24.5 64.1 and 61.4, 2^25 87.2 and 83.9.
+// Short tables: up to short_elems(dtype, mode) elements in all, where a pass runs
+// rmw_short_kernel over tiles of kShortTile elements. Where the lines lie: pass
+// times in us (perturb / update / restore + update / three-way) of the short
+// kernel and of the persistent one, three tables used in turn: fp16 2^24
+// elements 12.6 / 13.0 / 14.1 / 18.2 and 17.4 / 18.1 / 19.6 / 21.7, 2^24.5 16.5
+// / 17.0 / 18.0 / 23.8 and 19.0 / 19.2 / 20.3 / 22.2, 2^25.5 31.9 / 30.5 / 31.2
+// / 38.2 and 34.1 / 31.7 / 32.0 / 33.8, 2^26 43.7 / 42.3 / 43.1 / 51.4 and 46.0
+// / 41.7 / 42.4 / 43.9; bf16 2^23.5 10.7 / 11.0 / 13.2 / 17.5 and 18.2 / 19.1 /
+// 21.3 / 19.8, 2^24 13.2 / 14.0 / 17.3 / 22.7 and 19.0 / 19.9 / 21.7 / 20.2,
+// 2^25 21.7 / 22.5 / 27.3 / 38.0 and 24.8 / 25.1 / 26.4 / 28.1, 2^26 44.1 / 43.1
+// / 48.1 / 69.4 and 46.0 / 42.8 / 44.1 / 46.6; fp32 2^24 21.8 / 21.8 / 21.8 /
+// 22.7 and 22.4 / 22.6 / 22.5 / 23.6, 2^24.5 32.4 / 30.3 / 30.4 / 31.4 and 30.6
+// / 29.9 / 29.8 / 30.5.
 constexpr uint32_t kShortTile = kRmwThreads * 8;
-constexpr uint64_t short_elems(int dtype) { return dtype == DZ_F32 ? 1u << 24 : 1u << 25; }
+constexpr uint64_t short_elems(int dtype, int mode) {
+  if (dtype == DZ_F32) return 1u << 24;
+  if (mode == kModeRestoreUpdatePerturb) return dtype == DZ_F16 ? 5u << 22 : 3u << 22;
+  if (mode == kModeRestoreUpdate) return dtype == DZ_F16 ? 3u << 24 : 3u << 23;
+  return 1u << 26;
+}
 
 // Tensors of up to kPlainBytes in all, the size of the Infinity Cache, are read
 // and written with plain accesses by the persistent kernel; longer tables'

@@ -108,9 +108,10 @@ int32_t dz_table_time_next(dz_table* t, void* start_event, void* stop_event);
  * The default, 0, selects it for every launch: measured on the MI355X in the
  * ZO step it is the faster loop at 10 K fp32 tiles (OPT-125m), 77 K fp16
  * tiles (OPT-2.7B) and 384 K (OPT-13B). Tests set a large value to run the plain loop.
- * A short table (up to 2^25 elements of a 16-bit type, 2^24 of fp32) runs
- * neither loop but a kernel of its own, until this is called: then every pass
- * of the table runs the long tables' kernel. The values the passes compute do
+ * A short table (this pass: up to 5 * 2^22 fp16, 3 * 2^22 bf16 or 2^24 fp32
+ * elements in all) runs neither loop but a kernel of its own, as its other
+ * passes do, until this is called: then every pass of the table runs the long
+ * tables' kernel. The values the passes compute do
  * not depend on it. */
 int32_t dz_table_set_prefetch_min_tiles(dz_table* t, uint32_t min_tiles);
 

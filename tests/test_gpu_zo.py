@@ -150,11 +150,11 @@ def test_packed_odd_tensors_match_oracle(dt, prefetch, first):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("elems", [8192 * 256 - 3, 8192 * 1500 + 77, 2**24])
+@pytest.mark.parametrize("elems", [8192 * 256 - 3, 3 * 2**22, 8192 * 1500 + 77, 2**24, 3 * 2**24, 2**26 + 9])
 def test_short_tables_match_the_persistent_kernel(dt, elems):
-    """Tables below the short-table line, with one to six tiles per workgroup and odd tensors among
-    them, across a wrap of the z counter's low word: every pass gives the persistent kernel's bits
-    (which the other tests hold against the oracle)."""
+    """Tables at and around the lines below which passes run the short tables' kernel, with one to many
+    tiles per workgroup and odd tensors among them, across a wrap of the z counter's low word: every
+    pass gives the persistent kernel's bits (which the other tests hold against the oracle)."""
     from dizo_amd.table import ZOTable
     cut = [elems // 3 + 1, 5, elems // 2 + 3]
     sizes = cut + [elems - sum(cut)]
