@@ -638,7 +638,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     return rc;
   }
   for (int64_t ne : t->numels) t->bytes += (uint64_t)ne * es;
-  if (t->projection && t->bytes <= dz::kShortProjTotal * es) {
+  if (t->projection && t->bytes <= dz::kShortProjTotal * es && n <= dz::kShortProjGroups) {
     t->short_proj = true;
     t->chunk_elems = (uint32_t)dz::short_proj_elems(dtype);
   }

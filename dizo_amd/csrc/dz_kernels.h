@@ -169,6 +169,7 @@ constexpr int kProjAlphaLds = 4096;
 constexpr int kShortProjThreads = 256;
 __host__ __device__ constexpr int short_proj_elems(int dtype) { return dtype == DZ_F32 ? 2048 : 4096; }
 constexpr uint64_t kShortProjTotal = 3u << 24;
+constexpr int32_t kShortProjGroups = 1 << 16;  // more groups' counts would take over 8 MB
 // The groups' finished-chunk counts lie 128 bytes apart: side by side, every
 // workgroup's atomic met in the same line (22 ns each: 43 us for the norms of fp16 24 x 589,824).
 constexpr int kDoneStride = 32;  // uint32 slots
