@@ -190,10 +190,10 @@ int32_t check_range(uint64_t p, uint64_t bytes, const char* what, int32_t i) {
 // Scratch of the allocation-free entry point (dz_group_sumsq_static): device
 // memory the library never allocates at run time. Layout: the projection
 // kernel's work counters, the group -> first chunk index, the chunk
-// descriptors, the per-chunk partial sums and (zero between launches) the
-// groups' finished-chunk counts of short inputs, for at most kStaticMaxGroups
+// descriptors and the per-chunk partial sums, for at most kStaticMaxGroups
 // groups and kStaticMaxChunks chunks of proj_chunk_elems(dtype) elements (8.6 G
-// elements of a 16-bit type, 2.1 G of fp32).
+// elements of a 16-bit type, 2.1 G of fp32). A call writes what it reads: what
+// earlier calls left does not matter.
 // Each device holds its own copy, at its own address (see static_scratch).
 // ---------------------------------------------------------------------------
 namespace {
@@ -206,8 +206,7 @@ constexpr size_t kStaticOffCounters = 0;
 constexpr size_t kStaticOffGroupBegin = 4096;
 constexpr size_t kStaticOffChunks = kStaticOffGroupBegin + ((kStaticMaxGroups + 1) * 4 + 255) / 256 * 256;
 constexpr size_t kStaticOffPartials = kStaticOffChunks + (size_t)kStaticMaxChunks * sizeof(DzChunk);
-constexpr size_t kStaticOffDone = kStaticOffPartials + (size_t)kStaticMaxChunks * sizeof(double);
-constexpr size_t kStaticBytes = kStaticOffDone + (size_t)kStaticMaxGroups * dz::kDoneStride * sizeof(uint32_t);
+constexpr size_t kStaticBytes = kStaticOffPartials + (size_t)kStaticMaxChunks * sizeof(double);
 static_assert(dz::kCounterWords * 4 <= kStaticOffGroupBegin, "work counters overflow their scratch slot");
 }  // namespace
 
@@ -854,12 +853,18 @@ int32_t dz_group_sumsq_static(const uint64_t* ptrs, const uint64_t* anchor_ptrs,
   DzChunk* chunks = (DzChunk*)(sc->ptr + kStaticOffChunks);
   double* partials = (double*)(sc->ptr + kStaticOffPartials);
   const hipStream_t st = (hipStream_t)stream;
-  // short inputs: one launch for kStaticPlanGroups groups, chunks as in a short table
+  // short inputs: chunks as in a short table, whose groups travel as kernel arguments
   uint64_t elems = 0;
   for (int32_t i = 0; i < n; ++i) elems += (uint64_t)numels[i];
   if (elems <= dz::kShortProjTotal) {
     const uint64_t sn = (uint64_t)dz::short_proj_elems(dtype);
-    uint32_t begin = 0;
+    const auto chunks_of = [&](int32_t g) {
+      return (uint32_t)std::max<uint64_t>(1, ((uint64_t)numels[g] + sn - 1) / sn);
+    };
+    uint32_t begin = 0, most = 0;
+    for (int32_t g = 0; g < n; ++g) most = std::max(most, chunks_of(g));
+    const bool small = most <= dz::kStaticSmallChunks;
+    const dz::GroupOutputs out{d_sumsq, d_norm_f32, d_norm_T};
     for (int32_t g0 = 0; g0 < n; g0 += dz::kStaticPlanGroups) {
       dz::StaticGroups sg;
       sg.ngroups = (uint32_t)std::min<int32_t>(dz::kStaticPlanGroups, n - g0);
@@ -870,14 +875,27 @@ int32_t dz_group_sumsq_static(const uint64_t* ptrs, const uint64_t* anchor_ptrs,
         sg.anchor[k] = anchor_ptrs[g0 + k];
         sg.numel[k] = numels[g0 + k];
         sg.chunk_begin[k] = at;
-        at += (uint32_t)std::max<uint64_t>(1, ((uint64_t)numels[g0 + k] + sn - 1) / sn);
+        at += chunks_of(g0 + (int32_t)k);
       }
       sg.chunk_begin[sg.ngroups] = at;
-      const dz::ProjShort a{nullptr, nullptr, (uint32_t*)(sc->ptr + kStaticOffDone), nullptr, partials + begin,
-                            {d_sumsq, d_norm_f32, d_norm_T}};
-      const hipError_t e = dz::launch_static_sumsq(dtype, at, a, sg, st);
+      const hipError_t e = small ? dz::launch_static_small(dtype, sg, out, st)
+                                 : dz::launch_static_sumsq(dtype, at, partials + begin, sg, st);
       if (e != hipSuccess) return hip_fail(e, "sumsq kernel launch");
       begin += at;
+    }
+    if (small) return DZ_OK;
+    begin = 0;
+    for (int32_t g0 = 0; g0 < n; g0 += dz::kStaticSumGroups) {
+      dz::StaticSums ss;
+      const int32_t count = std::min<int32_t>(dz::kStaticSumGroups, n - g0);
+      ss.group_base = (uint32_t)g0;
+      for (int32_t k = 0; k < count; ++k) {
+        ss.chunk_begin[k] = begin;
+        begin += chunks_of(g0 + k);
+      }
+      ss.chunk_begin[count] = begin;
+      const hipError_t e = dz::launch_static_sums(dtype, (uint32_t)count, partials, ss, out, st);
+      if (e != hipSuccess) return hip_fail(e, "group sum kernel launch");
     }
     return DZ_OK;
   }

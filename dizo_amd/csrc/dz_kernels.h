@@ -223,7 +223,8 @@ struct GroupOutputs {
 };
 // A projection launch over a short table: its chunk list (nchunks of them; an
 // empty group has one of no elements) and each group's first chunk, the groups'
-// finished-chunk counts (zero before the launch, which leaves them at zero).
+// finished-chunk counts (zero before the launch, which leaves them at zero;
+// NULL: the launch stops at the chunks' partial sums).
 struct ProjShort {
   const DzChunk* chunks;
   const uint32_t* group_begin;
@@ -233,7 +234,17 @@ struct ProjShort {
   GroupOutputs out;
 };
 // The groups of a norm pass without a table: they travel as kernel arguments,
-// kStaticPlanGroups to a launch.
+// kStaticPlanGroups to a launch. What short inputs leave in the scratch that all
+// calls of a device share does not matter to the next call. Groups of up to
+// kStaticSmallChunks chunks are summed by one workgroup each, larger ones by a
+// second launch, kStaticSumGroups to a launch. (With a short table's
+// finished-chunk counts, two calls that overlapped once left every later one
+// wrong.) Call times in us, one launch / two launches / with counts, the host's
+// launch work in them: 4 fp16 groups of 4 chunks 4.7-5.8 / 7.0-9.8 / 5.7, of 8
+// 7.1 / 7.0-9.8 / 5.7, of 16 10.6 / 7.0-9.8 / 5.8; 4 fp32 groups of 8 5.7 /
+// 7.0-9.8 / 5.8; 24 fp16 groups of 8 7.7 / 9.3-11.6 / 7.6. Two launches / with
+// counts: 64 fp16 groups of 128 chunks 29 / 30, 24 fp32 groups of 288 (OPT-125m)
+// 23.2-23.7 / 25.2-25.6, one fp16 group of 4,096 18 / 58.
 constexpr int kStaticPlanGroups = 64;
 struct StaticGroups {
   uint64_t ptr[kStaticPlanGroups];
@@ -241,6 +252,12 @@ struct StaticGroups {
   int64_t numel[kStaticPlanGroups];
   uint32_t chunk_begin[kStaticPlanGroups + 1];  // within the launch
   uint32_t ngroups;
+  uint32_t group_base;
+};
+constexpr uint32_t kStaticSmallChunks = 8;
+constexpr int kStaticSumGroups = 512;
+struct StaticSums {
+  uint32_t chunk_begin[kStaticSumGroups + 1];
   uint32_t group_base;
 };
 hipError_t launch_proj_short(int dtype, int mode, uint32_t nchunks, const ProjShort& a, hipStream_t st,
@@ -251,7 +268,10 @@ hipError_t launch_dot(int dtype, const DzChunk* chunks, uint32_t nchunks, uint32
                       double* partials, uint32_t* counters, hipStream_t st, const LaunchEvents& ev = {});
 hipError_t launch_dot_short(int dtype, uint32_t nchunks, const ProjShort& a, const DotGroups& dg, hipStream_t st,
                             const LaunchEvents& ev = {});
-hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, const ProjShort& a, const StaticGroups& sg, hipStream_t st);
+hipError_t launch_static_small(int dtype, const StaticGroups& sg, const GroupOutputs& out, hipStream_t st);
+hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, double* partials, const StaticGroups& sg, hipStream_t st);
+hipError_t launch_static_sums(int dtype, uint32_t ngroups, const double* partials, const StaticSums& ss,
+                              const GroupOutputs& out, hipStream_t st);
 // take_sqrt: norms (sqrt of the sums) or plain sums in the fp32 / T outputs.
 hipError_t launch_finalize(int dtype, const double* partials, const uint32_t* gbegin, uint32_t ngroups,
                            double* sumsq, float* norm_f32, void* norm_T, bool take_sqrt, hipStream_t st,

@@ -1804,8 +1804,9 @@ __global__ void __launch_bounds__(kProjThreads) finalize_kernel(const double* __
 // of short_proj_elems, all of a thread's vectors in flight at once, no work
 // counters. The workgroup that ends a group's last chunk sums the group's
 // partials (in chunk order) and writes its results, so that a norm pass is one
-// launch. Chunks come from the table's list, or (StaticGroups) from the group
-// list in the launch's arguments.
+// launch. Without counts (ProjShort) the launch only writes the partials, and a
+// kernel behind it sums them in the same order. Chunks come from the table's
+// list, or (StaticGroups) from the group list in the launch's arguments.
 // ---------------------------------------------------------------------------
 
 // Counts a finished chunk of group g after publishing its partial sum; true in
@@ -1838,7 +1839,7 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
   constexpr bool kSums = proj_sums(MODE);
   __shared__ double red[kShortProjThreads / 64];
   __shared__ uint32_t flag;
-  uint32_t c = blockIdx.x, grp, first, count;
+  uint32_t c = blockIdx.x, grp, first = 0u, count = 0u;
   char* tp;
   const char *ap, *op = nullptr;
   uint32_t n;
@@ -1851,14 +1852,12 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
       else
         hi = mid;
     }
-    first = sg.chunk_begin[lo];
-    count = sg.chunk_begin[lo + 1] - first;
-    const int64_t s = (int64_t)(c - first) * short_proj_elems(DT);
+    const int64_t s = (int64_t)(c - sg.chunk_begin[lo]) * short_proj_elems(DT);
     const int64_t left = sg.numel[lo] - s;
     tp = (char*)sg.ptr[lo] + s * (int64_t)sizeof(S);
     ap = (const char*)sg.anchor[lo] + s * (int64_t)sizeof(S);
     n = (uint32_t)(left < short_proj_elems(DT) ? left : short_proj_elems(DT));
-    grp = sg.group_base + lo;
+    grp = lo;
   } else {
     if constexpr (MODE == kProjDot) c += sg.chunk_base;
     const DzChunk ch = a.chunks[c];
@@ -1866,8 +1865,10 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
     ap = (const char*)ch.aux;
     n = ch.n;
     grp = ch.meta;
-    first = kSums ? a.group_begin[grp] : 0u;
-    count = kSums ? a.group_begin[grp + 1] - first : 0u;
+    if constexpr (kSums) {
+      first = a.group_begin[grp];
+      count = a.group_begin[grp + 1] - first;
+    }
     if constexpr (MODE == kProjDot) op = (const char*)sg.other[grp - sg.group_base] + ch.zgroup * sizeof(S);
   }
   dz_u32x4 vt[kVecs], va[kVecs], vo[MODE == kProjDot ? kVecs : 1];
@@ -1899,13 +1900,82 @@ __global__ void __launch_bounds__(kShortProjThreads) proj_short_kernel(ProjShort
   }
   if constexpr (kSums) {
     const double t = block_sum_f64(acc, red);
-    if (publish_partial(a.partials + c, t, a.group_done + (size_t)grp * kDoneStride, count, &flag)) {
+    if (kStatic || a.group_done == nullptr) {
+      if (threadIdx.x == 0) a.partials[c] = t;
+    } else if (publish_partial(a.partials + c, t, a.group_done + (size_t)grp * kDoneStride, count, &flag)) {
       double x = 0.0;
       for (uint32_t i = threadIdx.x; i < count; i += kShortProjThreads) x += read_partial(a.partials + first + i);
       const double sum = block_sum_f64(x, red);
       if (threadIdx.x == 0) write_group<DT>(a.out, grp, sum, MODE != kProjDot);
     }
   }
+}
+
+// A table-free norm pass over groups of at most kStaticSmallChunks chunks:
+// workgroup g computes group g's chunk sums, a quarter of its threads one chunk
+// each, and adds them up, all in proj_short_kernel's order.
+template <int DT>
+__global__ void __launch_bounds__(4 * kShortProjThreads) static_small_kernel(StaticGroups sg, GroupOutputs out) {
+  using S = typename DT_<DT>::S;
+  constexpr uint32_t kPer = 16 / (uint32_t)sizeof(S), kElems = short_proj_elems(DT);
+  constexpr int kVecs = short_proj_elems(DT) / (kShortProjThreads * (int)kPer);
+  constexpr int kRounds = kStaticSmallChunks / 4, kWaves = kShortProjThreads / 64;
+  __shared__ double red[kStaticSmallChunks][kWaves];
+  const uint32_t t = threadIdx.x % kShortProjThreads, team = threadIdx.x / kShortProjThreads;
+  char* tp = (char*)sg.ptr[blockIdx.x];
+  const char* ap = (const char*)sg.anchor[blockIdx.x];
+  const uint32_t numel = (uint32_t)sg.numel[blockIdx.x];
+  dz_u32x4 vt[kRounds][kVecs], va[kRounds][kVecs];
+#pragma unroll
+  for (int k = 0; k < kRounds; ++k) {
+#pragma unroll
+    for (int u = 0; u < kVecs; ++u) {
+      const uint32_t e = (team + 4u * k) * kElems + (t + (uint32_t)u * kShortProjThreads) * kPer;
+      if (e + kPer <= numel) {
+        vt[k][u] = ld_any(tp + (size_t)e * sizeof(S));
+        va[k][u] = ld_any(ap + (size_t)e * sizeof(S));
+      }
+    }
+  }
+  const ProjScalars<DT, kProjSumsq> ps(0.0f);
+#pragma unroll
+  for (int k = 0; k < kRounds; ++k) {
+    double acc = 0.0;
+#pragma unroll
+    for (int u = 0; u < kVecs; ++u) {
+      const uint32_t e = (team + 4u * k) * kElems + (t + (uint32_t)u * kShortProjThreads) * kPer;
+      if (e + kPer <= numel)
+        (void)proj_vec<DT, kProjSumsq>(vt[k][u], va[k][u], ps, &acc);
+      else if (e < numel)
+        proj_tail<DT, kProjSumsq>(tp, ap, e, numel, 0.0f, &acc);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if ((t & 63u) == 0u) red[team + 4u * k][t >> 6] = acc;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  double x = 0.0;
+  if (threadIdx.x < kStaticSmallChunks) {
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) x += red[threadIdx.x][w];
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
+  if (threadIdx.x == 0) write_group<DT>(out, sg.group_base + blockIdx.x, x, true);
+}
+
+// The group sums of a table-free norm pass over short inputs with larger groups,
+// workgroup g for group g of the launch, in proj_short_kernel's order.
+template <int DT>
+__global__ void __launch_bounds__(kShortProjThreads) static_sums_kernel(const double* __restrict__ partials,
+                                                                        StaticSums ss, GroupOutputs out) {
+  __shared__ double red[kShortProjThreads / 64];
+  const uint32_t b = ss.chunk_begin[blockIdx.x], e = ss.chunk_begin[blockIdx.x + 1];
+  double x = 0.0;
+  for (uint32_t i = b + threadIdx.x; i < e; i += kShortProjThreads) x += partials[i];
+  const double t = block_sum_f64(x, red);
+  if (threadIdx.x == 0) write_group<DT>(out, ss.group_base + blockIdx.x, t, true);
 }
 
 // Chunk descriptors of a projection launch planned on the device (the
@@ -2212,13 +2282,39 @@ hipError_t launch_proj_short(int dtype, int mode, uint32_t nchunks, const ProjSh
   }
 }
 
-hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, const ProjShort& a, const StaticGroups& sg, hipStream_t st) {
+hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, double* partials, const StaticGroups& sg, hipStream_t st) {
   const LaunchEvents ev{};
+  const ProjShort a{nullptr, nullptr, nullptr, nullptr, partials, {}};
   const dim3 grid(nchunks), block(kShortProjThreads);
   switch (dtype) {
     case DZ_F32: DZ_LAUNCH((proj_short_kernel<DZ_F32, kProjSumsq, StaticGroups>), grid, block, st, ev, a, sg); break;
     case DZ_F16: DZ_LAUNCH((proj_short_kernel<DZ_F16, kProjSumsq, StaticGroups>), grid, block, st, ev, a, sg); break;
     case DZ_BF16: DZ_LAUNCH((proj_short_kernel<DZ_BF16, kProjSumsq, StaticGroups>), grid, block, st, ev, a, sg); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_static_small(int dtype, const StaticGroups& sg, const GroupOutputs& out, hipStream_t st) {
+  const LaunchEvents ev{};
+  const dim3 grid(sg.ngroups), block(4 * kShortProjThreads);
+  switch (dtype) {
+    case DZ_F32: DZ_LAUNCH((static_small_kernel<DZ_F32>), grid, block, st, ev, sg, out); break;
+    case DZ_F16: DZ_LAUNCH((static_small_kernel<DZ_F16>), grid, block, st, ev, sg, out); break;
+    case DZ_BF16: DZ_LAUNCH((static_small_kernel<DZ_BF16>), grid, block, st, ev, sg, out); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_static_sums(int dtype, uint32_t ngroups, const double* partials, const StaticSums& ss,
+                              const GroupOutputs& out, hipStream_t st) {
+  const LaunchEvents ev{};
+  const dim3 grid(ngroups), block(kShortProjThreads);
+  switch (dtype) {
+    case DZ_F32: DZ_LAUNCH((static_sums_kernel<DZ_F32>), grid, block, st, ev, partials, ss, out); break;
+    case DZ_F16: DZ_LAUNCH((static_sums_kernel<DZ_F16>), grid, block, st, ev, partials, ss, out); break;
+    case DZ_BF16: DZ_LAUNCH((static_sums_kernel<DZ_BF16>), grid, block, st, ev, partials, ss, out); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

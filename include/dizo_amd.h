@@ -190,12 +190,12 @@ int32_t dz_init(int32_t device);
  * groups are theta ptrs[g] with anchors anchor_ptrs[g], numels[g] elements of
  * `dtype` each; the outputs are dz_group_sumsq's, bit for bit. Chunk
  * descriptors, partial sums and work counters live in a static device array
- * of the library (11 MB per device, held until the process ends): at most
+ * of the library (10.5 MB per device, held until the process ends): at most
  * 4096 groups and 262,144 chunks of 32,768 elements of a 16-bit type (8.6 G
  * elements) or of 8,192 fp32 elements (2.1 G); larger inputs return
  * DZ_ERR_INVALID. Every call on one device shares that array,
- * so calls that overlap in time on one device race: order them on one
- * stream. After dz_init(device) a call allocates nothing; without it, the
+ * so calls that overlap in time on one device race (their own outputs may be
+ * wrong; later calls are not affected): order them on one stream. After dz_init(device) a call allocates nothing; without it, the
  * first call on a device does dz_init's work itself. */
 int32_t dz_group_sumsq_static(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const int64_t* numels,
                               int32_t n, int32_t dtype, double* d_sumsq, float* d_norm_f32, void* d_norm_T,

@@ -93,6 +93,42 @@ def test_static_norms_of_long_inputs_equal_table_norms(dt):
             assert torch.equal(_bits(g), _bits(w)), what
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+def test_static_norms_of_small_and_larger_groups_equal_table_norms(dt):
+    """Groups that end around a chunk (4096 elements of a 16-bit type, 2048 of fp32), in calls whose groups
+    one workgroup each sums (up to 8 chunks) and in calls that sum in a second launch: the table's bits."""
+    cn = 2048 if dt == torch.float32 else 4096
+    small = [1, 0, 7, cn - 1, cn, cn + 1, 4 * cn, 5 * cn + 3, 8 * cn]
+    for sizes, mis in ((small, (3, 6)), (small * 15, ()), (small + [8 * cn + 1], (9,)), ([300 * cn + 5] + small * 60, (0,))):
+        th, t0 = _groups(sizes, dt, len(sizes), misaligned=mis)
+        for g, w, what in zip(_static(th, t0, dt), _table(th, t0, dt), ("sumsq", "norm_f32", "norm_T")):
+            assert torch.equal(_bits(g), _bits(w)), f"{what}, {len(sizes)} groups"
+
+
+def test_calls_that_overlapped_leave_later_calls_right():
+    """Calls that overlap in time race on the shared scratch, and their own outputs may be wrong; the calls
+    after them are right. (Short inputs: every address they use travels as a kernel argument.)"""
+    dt = torch.float16
+    a, b = _groups([4096 * 900 + 5, 4096 * 200], dt, 21), _groups([4096 * 70 + 1, 4096 * 650, 9], dt, 22)
+    want = [_table(*x, dt) for x in (a, b)]
+    calls = []
+    for th, t0 in (a, b):
+        n = len(th)
+        out = torch.empty(n, dtype=torch.float64, device="cuda")
+        calls.append((L.u64_array([t.data_ptr() for t in th]), L.u64_array([t.data_ptr() for t in t0]),
+                      L.i64_array([t.numel() for t in th]), n, out))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for (p, q, ns, n, out), st in zip(calls, streams):
+            L.call("dz_group_sumsq_static", p, q, ns, n, dtype_code(dt), out.data_ptr(), None, None, st.cuda_stream)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        for x, w in zip((a, b), want):
+            for g, ww, what in zip(_static(*x, dt), w, ("sumsq", "norm_f32", "norm_T")):
+                assert torch.equal(_bits(g), _bits(ww)), what
+
+
 def test_static_rejects_more_than_the_scratch_holds():
     dt = torch.float16
     th, t0 = _groups([8], dt, 3)
