@@ -200,7 +200,7 @@ namespace {
 constexpr uint32_t kStaticMaxGroups = 4096;
 constexpr uint32_t kStaticMaxChunks = 1u << 18;
 // short inputs: at most one chunk more for each group than their elements fill
-static_assert(dz::kShortProjTotal / (uint64_t)dz::short_proj_elems(DZ_F32) + kStaticMaxGroups <= kStaticMaxChunks,
+static_assert(dz::kShortProjBytes / 4 / (uint64_t)dz::short_proj_elems(DZ_F32) + kStaticMaxGroups <= kStaticMaxChunks,
               "partial sums of short inputs");
 constexpr size_t kStaticOffCounters = 0;
 constexpr size_t kStaticOffGroupBegin = 4096;
@@ -237,7 +237,7 @@ struct dz_table {
   uint32_t* d_group_begin = nullptr;
   double* d_partials = nullptr;
   bool short_proj = false;         // a short projection table: its chunks are proj_short_kernel's
-  uint32_t* d_group_done = nullptr;  // finished chunks of each group (short projection tables)
+  uint32_t* d_group_done = nullptr;  // finished chunks of each group (short projection tables of small groups)
   uint32_t* d_counters = nullptr;  // work counters of the persistent RMW / projection kernels
   DeviceState* dev = nullptr;
   dz::LaunchEvents timing;  // dz_table_time_next's request for the next launching call
@@ -353,8 +353,14 @@ int32_t rmw(dz_table* t, int mode, const dz::DzScalars& s, const dz::DzScalarPtr
 int32_t proj_short(dz_table* t, int mode, const void* alpha, const dz::GroupOutputs& out, const dz::LaunchEvents& ev,
                    void* stream) {
   const dz::ProjShort a{t->d_chunks, t->d_group_begin, t->d_group_done, alpha, t->d_partials, out};
-  const hipError_t e = dz::launch_proj_short(t->dtype, mode, t->nchunks, a, (hipStream_t)stream, ev);
+  const bool second = dz::proj_sums(mode) && !t->d_group_done;  // a launch that adds up the chunk sums
+  hipError_t e = dz::launch_proj_short(t->dtype, mode, t->nchunks, a, (hipStream_t)stream,
+                                       {ev.start, second ? nullptr : ev.stop});
   if (e != hipSuccess) return hip_fail(e, "projection kernel launch");
+  if (!second) return DZ_OK;
+  e = dz::launch_short_sums(t->dtype, (uint32_t)t->n, t->d_partials, {t->d_group_begin, 0u}, out, true,
+                            (hipStream_t)stream, {nullptr, ev.stop});
+  if (e != hipSuccess) return hip_fail(e, "group sum kernel launch");
   return DZ_OK;
 }
 
@@ -637,7 +643,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     return rc;
   }
   for (int64_t ne : t->numels) t->bytes += (uint64_t)ne * es;
-  if (t->projection && t->bytes <= dz::kShortProjTotal * es && n <= dz::kShortProjGroups) {
+  if (t->projection && t->bytes <= dz::kShortProjBytes && n <= dz::kShortProjGroups) {
     t->short_proj = true;
     t->chunk_elems = (uint32_t)dz::short_proj_elems(dtype);
   }
@@ -663,7 +669,10 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
   if (t->projection) {
     mem.add(&t->d_group_begin, t->group_begin.data(), t->group_begin.size());
     mem.add(&t->d_partials, nullptr, t->nchunks ? t->nchunks : 1, false);
-    if (t->short_proj) mem.add(&t->d_group_done, nullptr, (size_t)t->n * dz::kDoneStride);
+    uint32_t most = 0;
+    for (int32_t i = 0; i < n; ++i) most = std::max(most, t->group_begin[i + 1] - t->group_begin[i]);
+    if (t->short_proj && most <= dz::kShortCountChunks)
+      mem.add(&t->d_group_done, nullptr, (size_t)t->n * dz::kDoneStride);
   }
   // work counters: zero here; every RMW and projection launch leaves them at zero again
   mem.add(&t->d_counters, nullptr, dz::kCounterWords);
@@ -856,7 +865,7 @@ int32_t dz_group_sumsq_static(const uint64_t* ptrs, const uint64_t* anchor_ptrs,
   // short inputs: chunks as in a short table, whose groups travel as kernel arguments
   uint64_t elems = 0;
   for (int32_t i = 0; i < n; ++i) elems += (uint64_t)numels[i];
-  if (elems <= dz::kShortProjTotal) {
+  if (elems * (uint64_t)es <= dz::kShortProjBytes) {
     const uint64_t sn = (uint64_t)dz::short_proj_elems(dtype);
     const auto chunks_of = [&](int32_t g) {
       return (uint32_t)std::max<uint64_t>(1, ((uint64_t)numels[g] + sn - 1) / sn);
@@ -988,7 +997,8 @@ int32_t dz_group_dot(dz_table* t, const uint64_t* other_ptrs, double* d_dot, flo
     for (int32_t i = g0; i < g1; ++i) dg.other[i - g0] = other_ptrs[i];
     if (t->short_proj) {
       const dz::ProjShort a{t->d_chunks, t->d_group_begin, t->d_group_done, nullptr, t->d_partials, {d_dot, d_dot_f32, nullptr}};
-      e = dz::launch_dot_short(t->dtype, c1 - c0, a, dg, (hipStream_t)stream, {ev.start, g1 == t->n ? ev.stop : nullptr});
+      e = dz::launch_dot_short(t->dtype, c1 - c0, a, dg, (hipStream_t)stream,
+                               {ev.start, t->d_group_done && g1 == t->n ? ev.stop : nullptr});
     } else {
       const uint32_t grid = std::min<uint32_t>(c1 - c0, (uint32_t)t->dev->cus);
       e = dz::launch_dot(t->dtype, t->d_chunks + c0, c1 - c0, grid, dg, t->d_partials + c0, t->d_counters,
@@ -997,9 +1007,13 @@ int32_t dz_group_dot(dz_table* t, const uint64_t* other_ptrs, double* d_dot, flo
     if (e != hipSuccess) return hip_fail(e, "dot kernel launch");
     ev.start = nullptr;
   }
-  if (t->short_proj) return DZ_OK;  // its launches write the groups' results
-  e = dz::launch_finalize(t->dtype, t->d_partials, t->d_group_begin, (uint32_t)t->n, d_dot, d_dot_f32, nullptr,
-                          false, (hipStream_t)stream, ev);
+  if (t->d_group_done) return DZ_OK;  // the launches wrote the groups' results
+  if (t->short_proj)
+    e = dz::launch_short_sums(t->dtype, (uint32_t)t->n, t->d_partials, {t->d_group_begin, 0u}, {d_dot, d_dot_f32, nullptr},
+                              false, (hipStream_t)stream, ev);
+  else
+    e = dz::launch_finalize(t->dtype, t->d_partials, t->d_group_begin, (uint32_t)t->n, d_dot, d_dot_f32, nullptr,
+                            false, (hipStream_t)stream, ev);
   if (e != hipSuccess) return hip_fail(e, "finalize kernel launch");
   return DZ_OK;
 }

@@ -155,23 +155,38 @@ __host__ __device__ constexpr int proj_chunk_elems(int dtype) { return dtype == 
 // beyond that each chunk reads its group's alpha from memory.
 constexpr int kProjAlphaLds = 4096;
 
-// Short projection tables: up to kShortProjTotal elements in all, whose launches
-// run proj_short_kernel over chunks of short_proj_elems(dtype) elements, a
-// workgroup of kShortProjThreads each. Pass times in us (norms / apply / reverse
-// + norms; a norm pass with its group sums), against the persistent kernel:
-// fp16 128 x 20,480 elements 5.6 / 4.6 / 6.4 and 14.9 / 11.9 / 22.1, 24 x
-// 589,824 12.6 / 13.0 / 17.4 and 20.9 / 21.4 / 31.4, 48 x 1,048,576 38.7 / 42.2
-// / 47.2 and 41.6 / 51.0 / 59.2, 64 x 2,097,152 100 / 123 / 149 and 93 / 127 /
-// 136; fp32 24 x 589,824 26.5 / 24.5 / 31.1 and 30.3 / 31.0 / 38.3, 48 x
-// 1,048,576 78 / 91 / 108 and 78 / 95 / 115, 64 x 2,097,152 214 / 274 / 314 and
-// 184 / 244 / 293. Chunks of half the size cost more counting (fp16 24 x
-// 589,824: norms 17.4), of twice the size run the same.
+// Short projection tables: up to kShortProjBytes in all, whose launches run
+// proj_short_kernel over chunks of short_proj_elems(dtype) elements, a workgroup
+// of kShortProjThreads each. Pass times in us (norms / apply / reverse + norms /
+// dot; with the group sums), against the persistent kernel, three tables used in
+// turn: fp16 128 x 20,480 elements 5.6 / 4.6 / 6.4 and 14.9 / 11.9 / 22.1 (norms
+// to reverse), 24 x 174,762 6.7 / 5.9 / 9.2 / 8.3 and 16.8 / 16.2 / 25.9 / 21.0,
+// 24 x 699,050 15.1 / 16.0 / 20.4 / 20.8 and 22.3 / 25.3 / 30.7 / 29.0, 2^24 in
+// one group 15.2 / 15.5 / 20.9 / 21.7 and 20.2 / 22.1 / 29.4 / 25.8, 24 x
+// 1,398,101 26.8 / 35.4 / 39.1 / 39.1 and 29.8 / 40.8 / 47.2 / 40.3, 2^25 in one
+// group 28.4 / 35.3 / 40.8 / 41.7 and 28.7 / 35.6 / 41.3 / 37.9; fp32 2^24 in
+// eight groups 26.6 / 35.4 / 39.5 / 38.3 and 31.5 / 35.9 / 43.0 / 39.8. Beyond 64
+// MB the persistent kernel applies faster (its streaming stores): fp16 24 x
+// 1,572,864 30.0 / 41.5 / 45.5 / 44.2 and 32.1 / 39.7 / 47.1 / 42.8, 24 x
+// 2,097,152 36.9 / 55.1 / 59.3 / 55.2 and 39.3 / 50.7 / 56.8 / 54.9; fp32 48 x
+// 1,048,576 69.4 / 110.5 / 113.1 / 102.3 and 74.1 / 95.1 / 113.2 / 102.0. Chunks
+// of half the size cost more counting (fp16 24 x 589,824: norms 17.4 against
+// 12.6), of twice the size run the same.
 constexpr int kShortProjThreads = 256;
 __host__ __device__ constexpr int short_proj_elems(int dtype) { return dtype == DZ_F32 ? 2048 : 4096; }
-constexpr uint64_t kShortProjTotal = 3u << 24;
+constexpr uint64_t kShortProjBytes = 1u << 26;
 constexpr int32_t kShortProjGroups = 1 << 16;  // more groups' counts would take over 8 MB
+// Tables whose largest group has more chunks than this keep no counts: a second
+// launch adds up the chunk sums (short_sums_kernel). A group's counts queue up,
+// 13 ns each: norms in us with counts and with a second launch, fp16 2^20 elements
+// in one group (256 chunks) 7.0 and 8.8, 2^22 in four (256) 8.6 and 8.3, in two
+// (512) 13.5 and 8.5, in one (1,024) 17.4 and 8.8, 2^23 in 12 (171) 10.2 and 10.8,
+// in eight (256) 10.6 and 10.4, 2^24 in 16 (256) 16.2 and 14.6, in one (4,096) 57.5
+// and 15.0; fp32 2^24 in one (8,192) 109.8 and 28.3.
+constexpr uint32_t kShortCountChunks = 256;
 // The groups' finished-chunk counts lie 128 bytes apart: side by side, every
-// workgroup's atomic met in the same line (22 ns each: 43 us for the norms of fp16 24 x 589,824).
+// workgroup's atomic met in the same lines (12 ns each: the norms of fp16 24 x
+// 589,824, 3,456 counts, took 43 us against 13).
 constexpr int kDoneStride = 32;  // uint32 slots
 
 // By-value scalars of one RMW launch.
@@ -256,8 +271,14 @@ struct StaticGroups {
 };
 constexpr uint32_t kStaticSmallChunks = 8;
 constexpr int kStaticSumGroups = 512;
+// First chunks of the groups (and of the one behind the last) whose chunk sums a
+// launch adds up: as arguments, or a table's list in device memory.
 struct StaticSums {
   uint32_t chunk_begin[kStaticSumGroups + 1];
+  uint32_t group_base;
+};
+struct TableSums {
+  const uint32_t* chunk_begin;
   uint32_t group_base;
 };
 hipError_t launch_proj_short(int dtype, int mode, uint32_t nchunks, const ProjShort& a, hipStream_t st,
@@ -272,6 +293,9 @@ hipError_t launch_static_small(int dtype, const StaticGroups& sg, const GroupOut
 hipError_t launch_static_sumsq(int dtype, uint32_t nchunks, double* partials, const StaticGroups& sg, hipStream_t st);
 hipError_t launch_static_sums(int dtype, uint32_t ngroups, const double* partials, const StaticSums& ss,
                               const GroupOutputs& out, hipStream_t st);
+// The group sums of a launch over a short table without counts.
+hipError_t launch_short_sums(int dtype, uint32_t ngroups, const double* partials, const TableSums& ts,
+                             const GroupOutputs& out, bool take_sqrt, hipStream_t st, const LaunchEvents& ev = {});
 // take_sqrt: norms (sqrt of the sums) or plain sums in the fp32 / T outputs.
 hipError_t launch_finalize(int dtype, const double* partials, const uint32_t* gbegin, uint32_t ngroups,
                            double* sumsq, float* norm_f32, void* norm_T, bool take_sqrt, hipStream_t st,

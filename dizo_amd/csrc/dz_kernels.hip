@@ -1965,17 +1965,29 @@ __global__ void __launch_bounds__(4 * kShortProjThreads) static_small_kernel(Sta
   if (threadIdx.x == 0) write_group<DT>(out, sg.group_base + blockIdx.x, x, true);
 }
 
-// The group sums of a table-free norm pass over short inputs with larger groups,
-// workgroup g for group g of the launch, in proj_short_kernel's order.
-template <int DT>
-__global__ void __launch_bounds__(kShortProjThreads) static_sums_kernel(const double* __restrict__ partials,
-                                                                        StaticSums ss, GroupOutputs out) {
+// The group sums of a launch of proj_short_kernel without counts, workgroup g for
+// group g of the launch, in that kernel's order, with kAhead loads of a thread in
+// flight (one by one, the norms of one group of 8,192 chunks took 34.9 us, now
+// 27.8).
+template <int DT, class Sums>
+__global__ void __launch_bounds__(kShortProjThreads) short_sums_kernel(const double* __restrict__ partials, Sums ss,
+                                                                       GroupOutputs out, bool take_sqrt) {
+  constexpr int kAhead = 8;
   __shared__ double red[kShortProjThreads / 64];
   const uint32_t b = ss.chunk_begin[blockIdx.x], e = ss.chunk_begin[blockIdx.x + 1];
   double x = 0.0;
-  for (uint32_t i = b + threadIdx.x; i < e; i += kShortProjThreads) x += partials[i];
+  for (uint32_t i = b + threadIdx.x; i < e; i += kAhead * kShortProjThreads) {
+    double v[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const uint32_t at = i + (uint32_t)k * kShortProjThreads;
+      v[k] = at < e ? partials[at] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) x += v[k];
+  }
   const double t = block_sum_f64(x, red);
-  if (threadIdx.x == 0) write_group<DT>(out, ss.group_base + blockIdx.x, t, true);
+  if (threadIdx.x == 0) write_group<DT>(out, ss.group_base + blockIdx.x, t, take_sqrt);
 }
 
 // Chunk descriptors of a projection launch planned on the device (the
@@ -2307,17 +2319,27 @@ hipError_t launch_static_small(int dtype, const StaticGroups& sg, const GroupOut
   return hipGetLastError();
 }
 
-hipError_t launch_static_sums(int dtype, uint32_t ngroups, const double* partials, const StaticSums& ss,
-                              const GroupOutputs& out, hipStream_t st) {
-  const LaunchEvents ev{};
+template <class Sums>
+static hipError_t launch_sums(int dtype, uint32_t ngroups, const double* partials, const Sums& ss, const GroupOutputs& out,
+                              bool take_sqrt, hipStream_t st, const LaunchEvents& ev) {
   const dim3 grid(ngroups), block(kShortProjThreads);
   switch (dtype) {
-    case DZ_F32: DZ_LAUNCH((static_sums_kernel<DZ_F32>), grid, block, st, ev, partials, ss, out); break;
-    case DZ_F16: DZ_LAUNCH((static_sums_kernel<DZ_F16>), grid, block, st, ev, partials, ss, out); break;
-    case DZ_BF16: DZ_LAUNCH((static_sums_kernel<DZ_BF16>), grid, block, st, ev, partials, ss, out); break;
+    case DZ_F32: DZ_LAUNCH((short_sums_kernel<DZ_F32, Sums>), grid, block, st, ev, partials, ss, out, take_sqrt); break;
+    case DZ_F16: DZ_LAUNCH((short_sums_kernel<DZ_F16, Sums>), grid, block, st, ev, partials, ss, out, take_sqrt); break;
+    case DZ_BF16: DZ_LAUNCH((short_sums_kernel<DZ_BF16, Sums>), grid, block, st, ev, partials, ss, out, take_sqrt); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+hipError_t launch_static_sums(int dtype, uint32_t ngroups, const double* partials, const StaticSums& ss,
+                              const GroupOutputs& out, hipStream_t st) {
+  return launch_sums(dtype, ngroups, partials, ss, out, true, st, {});
+}
+
+hipError_t launch_short_sums(int dtype, uint32_t ngroups, const double* partials, const TableSums& ts,
+                             const GroupOutputs& out, bool take_sqrt, hipStream_t st, const LaunchEvents& ev) {
+  return launch_sums(dtype, ngroups, partials, ts, out, take_sqrt, st, ev);
 }
 
 template <int DT>

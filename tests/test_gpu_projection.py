@@ -157,12 +157,12 @@ def test_packed_odd_groups_match_oracle(dt, first, sizes):
 
 @pytest.mark.parametrize("dt", DTS)
 def test_long_tables_match_short_ones(dt):
-    """Groups that together make a long table (more than 3 * 2^24 elements), odd starts and sizes among
-    them, against a table of each group by itself (a short one): the same bits from apply, fp32-alpha
-    apply and reverse, and sums equal to the fp64 sums' rounding."""
+    """Groups that together make a long table (more than 64 MB), odd starts and sizes among them, against a
+    table of each group by itself (a short one, whose sums take a second launch in all but the smallest):
+    the same bits from apply, fp32-alpha apply and reverse, and sums equal to the fp64 sums' rounding."""
     from dizo_amd import _lib as L
     from dizo_amd.table import ProjTable
-    sizes = [30_000_001, 7, 12_345_678, 0, 9_000_003]
+    sizes = [16_000_001, 7, 12_345_678, 0, 9_000_003]
     G, total = len(sizes), sum(sizes)
     gen = torch.Generator(device="cuda").manual_seed(3)
     anchor = torch.empty(total + 1, dtype=DT_TORCH[dt], device="cuda").normal_(0, 0.02, generator=gen)
@@ -202,6 +202,69 @@ def test_long_tables_match_short_ones(dt):
         bound = float(terms.abs().sum()) * sizes[g] * 2.0**-53
         for got in (sums[0][3, g], sums[1][3, g]):
             assert abs(float(got) - float(terms.sum())) <= bound, g
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("chunks", [256, 257])
+def test_sums_around_the_count_line_match_fp64(dt, chunks):
+    """Short tables whose largest group has 256 chunks (counted) or 257 (a second launch adds up the chunk
+    sums), 130 groups (two dot launches) with an empty one among them: norms, reverse + norms and dots
+    against torch's fp64 sums. The squares are exact in fp64, so n terms are at most n / 2 roundings of
+    2^-53 apart from any other order; the dots' terms differ in sign, so their bound is on their sizes."""
+    from dizo_amd import _lib as L
+    from dizo_amd.table import ProjTable
+    cn = 2048 if dt == F32 else 4096
+    sizes = [(chunks - 1) * cn + 5] + [1000 + i for i in range(127)] + [0, cn]
+    G, total = len(sizes), sum(sizes)
+    gen = torch.Generator(device="cuda").manual_seed(chunks)
+    anchor = torch.empty(total, dtype=DT_TORCH[dt], device="cuda").normal_(0, 0.02, generator=gen)
+    theta = anchor + torch.empty_like(anchor).normal_(0, 4e-3, generator=gen)
+    other = torch.empty_like(anchor).normal_(0, 1e-2, generator=gen)
+    ths, t0s, others = (list(x.split(sizes)) for x in (theta, anchor, other))
+    tab = ProjTable(ths, t0s)
+    sums, dots = (torch.full((G,), -1.0, dtype=torch.float64, device="cuda") for _ in range(2))
+    alpha = torch.ones(G, dtype=DT_TORCH[dt], device="cuda")
+    for mode in ("sumsq", "reverse"):
+        if mode == "sumsq":
+            tab.group_sumsq(sums)
+        else:
+            tab.project(alpha, L.DZ_PROJ_REVERSE_SUMSQ, sumsq=sums)
+        tab.group_dot(others, dots)
+        for g in range(G):
+            d = (ths[g] - t0s[g]).double()
+            assert float(sums[g]) == pytest.approx(float(d.square().sum()), rel=max(1, sizes[g]) * 2.0**-53, abs=0), (mode, g)
+            terms = others[g].double() * d
+            assert abs(float(dots[g]) - float(terms.sum())) <= float(terms.abs().sum()) * max(1, sizes[g]) * 2.0**-53, (mode, g)
+    tab.close()
+
+
+@pytest.mark.parametrize("dt,elems", [(F16, 2**24), (F32, 2**23)])
+def test_the_sums_of_one_large_group_do_not_hold_up_the_pass(dt, elems):
+    """One group of 32 MB: the norm pass reads 64 MB, an apply moves 96. With a count for each chunk of the
+    group the norms took 3.7 times the apply (58 against 15.6 us); they take about as long."""
+    from dizo_amd import _lib as L
+    from dizo_amd.table import ProjTable
+    anchor = torch.zeros(elems, dtype=DT_TORCH[dt], device="cuda")
+    tab = ProjTable([torch.full_like(anchor, 0.5)], [anchor])
+    alpha, out = torch.ones(1, dtype=anchor.dtype, device="cuda"), torch.empty(1, dtype=torch.float64, device="cuda")
+
+    def median_us(call):
+        times = []
+        for _ in range(25):
+            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            for e in ev:
+                e.record()
+            tab.time_next(*ev)
+            call()
+            torch.cuda.synchronize()
+            times.append(ev[0].elapsed_time(ev[1]) * 1e3)
+        return sorted(times)[12]
+
+    apply = median_us(lambda: tab.project(alpha, L.DZ_PROJ_APPLY))
+    norms = median_us(lambda: tab.group_sumsq(out))
+    assert float(out[0]) == 0.25 * elems
+    assert norms <= 2 * apply, (norms, apply)
+    tab.close()
 
 
 def test_empty_and_rejects():
