@@ -41,9 +41,10 @@ def stream_handle(stream: Optional[torch.cuda.Stream] = None) -> int:
     return stream.cuda_stream
 
 
-def _on(device: torch.device):
-    """`device` as the current one; nothing to do where it already is."""
-    if device.index is not None and device.index == torch._C._cuda_getDevice():
+def _on(device):
+    """`device` (in any form that torch.cuda.device takes) as the current one; nothing to do
+    where it already is."""
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index == torch._C._cuda_getDevice():
         return nullcontext()
     return torch.cuda.device(device)
 

@@ -107,6 +107,17 @@ def test_philox_blocks_match_oracle():
         np.testing.assert_array_equal(got, want)
 
 
+def test_normals_and_philox_take_the_device_in_every_form():
+    from dizo_amd.table import normals, philox_blocks
+    z, w = normals(3, 1, 5, 100, torch.float16, torch.device("cuda", 0)), philox_blocks(3, 1, 5, 9, torch.device("cuda", 0))
+    for device in (0, "cuda", "cuda:0", torch.device("cuda")):
+        assert torch.equal(normals(3, 1, 5, 100, torch.float16, device), z)
+        assert torch.equal(philox_blocks(3, 1, 5, 9, device), w)
+    with torch.device("cuda"):  # the default device
+        assert torch.equal(normals(3, 1, 5, 100, torch.float16, None), z)
+        assert torch.equal(philox_blocks(3, 1, 5, 9, None), w)
+
+
 @pytest.mark.parametrize("dt", DTS)
 def test_rmw_uses_exported_z(dt):
     """theta = 0, scale 1, eps 1 leaves exactly z: the kernel's in-register z is the exported z."""

@@ -128,3 +128,23 @@ def test_train_runs_epochs_over_a_short_batch_list(cpu_trainer):
     assert seen == ["x", "y"]
     with pytest.raises(DzError):
         tr.train([], max_steps=2)
+
+
+@pytest.mark.parametrize("device,index", [(0, 0), (1, 1), ("cuda:1", 1), (torch.device("cuda", 1), 1)])
+def test_device_arguments_of_every_form(monkeypatch, device, index):
+    """normals and philox_blocks take a device in every form that torch takes one."""
+    from dizo_amd import table
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0)
+    on = table._on(device)
+    assert isinstance(on, torch.cuda.device) and on.idx == index
+
+
+def test_the_current_device_needs_no_switch_and_the_cpu_is_refused(monkeypatch):
+    import contextlib
+
+    from dizo_amd import table
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0)
+    assert isinstance(table._on(torch.device("cuda", 0)), contextlib.nullcontext)
+    for cpu in (torch.device("cpu"), torch.device("cpu", 0)):
+        with pytest.raises(ValueError, match="Expected a cuda device"):
+            table._on(cpu)
