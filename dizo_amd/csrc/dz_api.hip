@@ -231,7 +231,7 @@ struct dz_table {
   uint32_t fused_nchunks = 0;
   DzChunk* d_fused_chunks = nullptr;
   // ZO tables with passes short enough for rmw_short_kernel: its tile list
-  bool persistent_only = false;  // set by dz_table_set_prefetch_min_tiles
+  bool persistent_only = false;  // dz_table_set_prefetch_min_tiles was called with other than 0
   uint32_t short_nchunks = 0;
   DzChunk* d_short_chunks = nullptr;
   uint32_t* d_group_begin = nullptr;
@@ -717,7 +717,7 @@ int32_t dz_table_set_prefetch_min_tiles(dz_table* t, uint32_t min_tiles) {
   int32_t rc = check_table(t);
   if (rc) return rc;
   t->prefetch_min_tiles = min_tiles;
-  t->persistent_only = true;
+  t->persistent_only = min_tiles != 0;
   return DZ_OK;
 }
 

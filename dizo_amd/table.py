@@ -118,8 +118,9 @@ class _Table:
     def set_prefetch_min_tiles(self, min_tiles: int) -> None:
         """Launches of the fused restore+update+next perturb pass with at least
         min_tiles tiles run the prefetching tile loop (0, the default: every
-        launch; 2**32 - 1: none). The computed values do not
-        depend on it."""
+        launch; 2**32 - 1: none). Other than 0, all passes of a short table leave
+        its kernel for the long tables' one; 0 restores the default. The
+        computed values do not depend on it."""
         L.call("dz_table_set_prefetch_min_tiles", self.handle, int(min_tiles))
 
     def time_next(self, start: "torch.cuda.Event | None", stop: "torch.cuda.Event | None") -> None:

@@ -110,9 +110,9 @@ int32_t dz_table_time_next(dz_table* t, void* start_event, void* stop_event);
  * tiles (OPT-2.7B) and 384 K (OPT-13B). Tests set a large value to run the plain loop.
  * A short table (this pass: up to 5 * 2^22 fp16, 3 * 2^22 bf16 or 2^24 fp32
  * elements in all) runs neither loop but a kernel of its own, as its other
- * passes do, until this is called: then every pass of the table runs the long
- * tables' kernel. The values the passes compute do
- * not depend on it. */
+ * passes do. With min_tiles other than 0 every pass of the table runs the
+ * long tables' kernel (1: with the prefetching loop); 0 restores the default.
+ * The values the passes compute do not depend on it. */
 int32_t dz_table_set_prefetch_min_tiles(dz_table* t, uint32_t min_tiles);
 
 /* ---- ZO step (trainer.py:1429-1444, 1570-1617) -------------------------- */

@@ -44,12 +44,12 @@ def _make_tensors(dt, seed, sizes=SIZES, misaligned=(3, 6)):
 
 
 def _fused_table(tensors, prefetch, **kw):
-    """A ZO table whose 16-bit restore+update+next perturb launches run the
-    prefetching tile loop (prefetch=True, every launch) or the plain tile
-    loop (prefetch=False, no launch)."""
+    """A ZO table on the long tables' kernel, whose restore+update+next perturb
+    launches run the prefetching tile loop (prefetch=True, every launch) or the
+    plain tile loop (prefetch=False, no launch)."""
     from dizo_amd.table import ZOTable
     tab = ZOTable(tensors, **kw)
-    tab.set_prefetch_min_tiles(0 if prefetch else 0xFFFFFFFF)
+    tab.set_prefetch_min_tiles(1 if prefetch else 0xFFFFFFFF)
     return tab
 
 
@@ -186,6 +186,35 @@ def test_short_tables_match_the_persistent_kernel(dt, elems):
         out.append(to_bits(flat))
         tab.close()
     assert_bits_equal(out[0], out[1], dt, f"{elems} elements")
+
+
+def test_prefetch_min_tiles_of_0_restores_the_short_kernel():
+    """2^20 fp16 elements: a pass of the short tables' kernel takes 4 us, of the long tables' one 10 to 14.
+    The default may be set again, also after another value."""
+    from dizo_amd.table import ZOTable
+    tab = ZOTable([torch.zeros(2**20, dtype=torch.float16, device="cuda")])
+
+    def median_us():
+        times = []
+        for _ in range(25):
+            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            for e in ev:
+                e.record()
+            tab.time_next(*ev)
+            tab.restore_update_perturb(1, 2, 1e-3, 0.3, 1e-3)
+            torch.cuda.synchronize()
+            times.append(ev[0].elapsed_time(ev[1]) * 1e3)
+        return sorted(times)[12]
+
+    median_us()
+    default = median_us()
+    tab.set_prefetch_min_tiles(0)
+    assert median_us() < 1.4 * default
+    tab.set_prefetch_min_tiles(1)
+    assert median_us() > 1.4 * default
+    tab.set_prefetch_min_tiles(0)
+    assert median_us() < 1.4 * default
+    tab.close()
 
 
 @pytest.mark.parametrize("dt", DTS)
