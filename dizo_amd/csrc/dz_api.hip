@@ -400,7 +400,7 @@ void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
 // ZO tile lists: full tiles first (in tensor order), then the partial ones;
 // returns the number of full tiles. The order of
 // the tiles changes no result (z is a function of the element index), and it
-// lets the RMW kernel run its full tiles without a per-tile shape test.
+// lets the long tables' kernel run its full tiles without a per-tile shape test.
 uint32_t full_tiles_first(std::vector<DzChunk>* v, uint32_t elems) {
   auto it = std::stable_partition(v->begin(), v->end(), [elems](const DzChunk& c) {
     return c.n == elems;
@@ -663,6 +663,11 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
   }
   if (!t->projection && t->bytes <= dz::short_elems(dtype, dz::kModePerturb) * es) {
     build_chunks(t, dz::kShortTile, &short_chunks, nullptr, true);
+    // full tiles first: a workgroup takes every gridDim.x-th tile, and tensors a
+    // little over a tile make full and small tiles in turn, which left the full
+    // ones to half of the workgroups (bf16 1,200 tensors of 8,200 elements,
+    // three-way pass: 25.1 us, now 17.0; the long tables' kernel 19.6)
+    (void)full_tiles_first(&short_chunks, dz::kShortTile);
     t->short_nchunks = (uint32_t)short_chunks.size();
     mem.add(&t->d_short_chunks, short_chunks.data(), short_chunks.size());
   }
