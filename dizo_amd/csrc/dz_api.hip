@@ -200,7 +200,7 @@ namespace {
 constexpr uint32_t kStaticMaxGroups = 4096;
 constexpr uint32_t kStaticMaxChunks = 1u << 18;
 // short inputs: at most one chunk more for each group than their elements fill
-static_assert(dz::kShortProjBytes / 4 / (uint64_t)dz::short_proj_elems(DZ_F32) + kStaticMaxGroups <= kStaticMaxChunks,
+static_assert(dz::kShortProjTotal / (uint64_t)dz::short_proj_elems(DZ_F32) + kStaticMaxGroups <= kStaticMaxChunks,
               "partial sums of short inputs");
 constexpr size_t kStaticOffCounters = 0;
 constexpr size_t kStaticOffGroupBegin = 4096;
@@ -643,7 +643,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     return rc;
   }
   for (int64_t ne : t->numels) t->bytes += (uint64_t)ne * es;
-  if (t->projection && t->bytes <= dz::kShortProjBytes && n <= dz::kShortProjGroups) {
+  if (t->projection && t->bytes <= dz::kShortProjTotal * es && n <= dz::kShortProjGroups) {
     t->short_proj = true;
     t->chunk_elems = (uint32_t)dz::short_proj_elems(dtype);
   }
@@ -870,7 +870,7 @@ int32_t dz_group_sumsq_static(const uint64_t* ptrs, const uint64_t* anchor_ptrs,
   // short inputs: chunks as in a short table, whose groups travel as kernel arguments
   uint64_t elems = 0;
   for (int32_t i = 0; i < n; ++i) elems += (uint64_t)numels[i];
-  if (elems * (uint64_t)es <= dz::kShortProjBytes) {
+  if (elems <= dz::kShortProjTotal) {
     const uint64_t sn = (uint64_t)dz::short_proj_elems(dtype);
     const auto chunks_of = [&](int32_t g) {
       return (uint32_t)std::max<uint64_t>(1, ((uint64_t)numels[g] + sn - 1) / sn);

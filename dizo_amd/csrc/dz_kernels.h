@@ -155,26 +155,31 @@ __host__ __device__ constexpr int proj_chunk_elems(int dtype) { return dtype == 
 // beyond that each chunk reads its group's alpha from memory.
 constexpr int kProjAlphaLds = 4096;
 
-// Short projection tables: up to kShortProjBytes in all, whose launches run
-// proj_short_kernel over chunks of short_proj_elems(dtype) elements, a workgroup
-// of kShortProjThreads each. Pass times in us (norms / apply / reverse + norms /
-// dot; with the group sums), against the persistent kernel, three tables used in
-// turn: fp16 128 x 20,480 elements 5.6 / 4.6 / 6.4 and 14.9 / 11.9 / 22.1 (norms
-// to reverse), 24 x 174,762 6.7 / 5.9 / 9.2 / 8.3 and 16.8 / 16.2 / 25.9 / 21.0,
-// 24 x 699,050 15.1 / 16.0 / 20.4 / 20.8 and 22.3 / 25.3 / 30.7 / 29.0, 2^24 in
-// one group 15.2 / 15.5 / 20.9 / 21.7 and 20.2 / 22.1 / 29.4 / 25.8, 24 x
-// 1,398,101 26.8 / 35.4 / 39.1 / 39.1 and 29.8 / 40.8 / 47.2 / 40.3, 2^25 in one
-// group 28.4 / 35.3 / 40.8 / 41.7 and 28.7 / 35.6 / 41.3 / 37.9; fp32 2^24 in
-// eight groups 26.6 / 35.4 / 39.5 / 38.3 and 31.5 / 35.9 / 43.0 / 39.8. Beyond 64
-// MB the persistent kernel applies faster (its streaming stores): fp16 24 x
-// 1,572,864 30.0 / 41.5 / 45.5 / 44.2 and 32.1 / 39.7 / 47.1 / 42.8, 24 x
-// 2,097,152 36.9 / 55.1 / 59.3 / 55.2 and 39.3 / 50.7 / 56.8 / 54.9; fp32 48 x
-// 1,048,576 69.4 / 110.5 / 113.1 / 102.3 and 74.1 / 95.1 / 113.2 / 102.0. Chunks
-// of half the size cost more counting (fp16 24 x 589,824: norms 17.4 against
-// 12.6), of twice the size run the same.
+// Short projection tables: up to kShortProjTotal elements in all, whose launches
+// run proj_short_kernel over chunks of short_proj_elems(dtype) elements, a
+// workgroup of kShortProjThreads each. Pass times in us (norms / apply / reverse
+// + norms / dot; with the group sums), against the persistent kernel, passes back
+// to back, three tables used in turn: fp16 128 x 20,480 elements 5.6 / 4.6 / 6.4
+// and 14.9 / 11.9 / 22.1 (norms to reverse), 24 x 174,762 6.7 / 5.9 / 9.2 / 8.3
+// and 16.8 / 16.2 / 25.9 / 21.0, 24 x 699,050 15.1 / 16.0 / 20.4 / 20.8 and 22.3 /
+// 25.3 / 30.7 / 29.0, 2^24 in one group 15.2 / 15.5 / 20.9 / 21.7 and 20.2 / 22.1 /
+// 29.4 / 25.8, 2^25 in 24 26.8 / 35.4 / 39.1 / 39.1 and 29.8 / 40.8 / 47.2 / 40.3,
+// in one 28.4 / 35.3 / 40.8 / 41.7 and 28.7 / 35.6 / 41.3 / 37.9, 3 x 2^24 in 24
+// 36.9 / 55.1 / 59.3 / 55.2 and 39.3 / 50.7 / 56.8 / 54.9; fp32 2^24 in eight 26.6 /
+// 35.4 / 39.5 / 38.3 and 31.5 / 35.9 / 43.0 / 39.8, 5,000 x 4,097 37.0 / 46.5 /
+// 51.0 / - and 64.0 / 50.1 / 75.0 / -, 3 x 2^24 in 48 69.4 / 110.5 / 113.1 / 102.3
+// and 74.1 / 95.1 / 113.2 / 102.0. From 2^26 bytes on the persistent kernel's
+// streaming stores make an apply faster when passes follow one another; with
+// products over the projected weights between them, as in the gamma search, the
+// plain stores are the better ones up to here (they leave the weights in the
+// Infinity Cache): apply + reverse and the products in us, short and persistent,
+// fp16 36 x 2^20 elements 75 + 708 and 88 + 853, 44 x 2^20 89 + 866 and 102 + 1039,
+// fp32 32 x 2^20 133 + 2285 and 146 + 2307, 44 x 2^20 175 + 3059 and 192 + 3068.
+// Chunks of half the size cost more counting (fp16 24 x 589,824: norms 17.4
+// against 12.6), of twice the size run the same.
 constexpr int kShortProjThreads = 256;
 __host__ __device__ constexpr int short_proj_elems(int dtype) { return dtype == DZ_F32 ? 2048 : 4096; }
-constexpr uint64_t kShortProjBytes = 1u << 26;
+constexpr uint64_t kShortProjTotal = 3u << 24;
 constexpr int32_t kShortProjGroups = 1 << 16;  // more groups' counts would take over 8 MB
 // Tables whose largest group has more chunks than this keep no counts: a second
 // launch adds up the chunk sums (short_sums_kernel). A group's counts queue up,

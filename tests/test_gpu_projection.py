@@ -157,12 +157,13 @@ def test_packed_odd_groups_match_oracle(dt, first, sizes):
 
 @pytest.mark.parametrize("dt", DTS)
 def test_long_tables_match_short_ones(dt):
-    """Groups that together make a long table (more than 64 MB), odd starts and sizes among them, against a
-    table of each group by itself (a short one, whose sums take a second launch in all but the smallest):
-    the same bits from apply, fp32-alpha apply and reverse, and sums equal to the fp64 sums' rounding."""
+    """Groups that together make a long table (more than 3 * 2^24 elements), odd starts and sizes among
+    them, against a table of each group by itself (a short one; the larger groups' sums take a second
+    launch): the same bits from apply, fp32-alpha apply and reverse, and sums equal to the fp64 sums'
+    rounding."""
     from dizo_amd import _lib as L
     from dizo_amd.table import ProjTable
-    sizes = [16_000_001, 7, 12_345_678, 0, 9_000_003]
+    sizes = [30_000_001, 7, 12_345_678, 0, 9_000_003]
     G, total = len(sizes), sum(sizes)
     gen = torch.Generator(device="cuda").manual_seed(3)
     anchor = torch.empty(total + 1, dtype=DT_TORCH[dt], device="cuda").normal_(0, 0.02, generator=gen)

@@ -81,7 +81,7 @@ def test_static_norms_equal_table_norms_two_calls(dt):
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
 def test_static_norms_of_long_inputs_equal_table_norms(dt):
-    """More than 64 MB in 66 groups (the persistent kernel, its chunks planned on the device in
+    """More than 3 * 2^24 elements in 66 groups (the persistent kernel, its chunks planned on the device in
     two launches), then a short call, then the long one again: the table's bits each time."""
     gen = torch.Generator(device="cuda").manual_seed(4)
     sizes = [800_000 + 1000 * i for i in range(66)]
