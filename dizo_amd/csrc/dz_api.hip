@@ -397,6 +397,23 @@ void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
   }
 }
 
+// Whether a projection table runs proj_short_kernel (see kShortProjTotal). With
+// at most kStaticMaxGroups groups its first line alone decides, as in
+// dz_group_sumsq_static: small groups fill less than kStaticMaxGroups chunks.
+bool short_projection(const dz_table* t) {
+  const uint64_t cn = (uint64_t)dz::proj_chunk_elems(t->dtype), sn = (uint64_t)dz::short_proj_elems(t->dtype);
+  uint64_t elems = 0, chunks = 0, short_chunks = 0;
+  for (int64_t ne : t->numels) {
+    elems += (uint64_t)ne;
+    chunks += ((uint64_t)ne + cn - 1) / cn;
+    short_chunks += std::max<uint64_t>(1, ((uint64_t)ne + sn - 1) / sn);
+  }
+  return short_chunks <= dz::kShortProjChunks &&
+         (elems <= dz::kShortProjTotal || elems * dz::kShortProjFill <= chunks * cn);
+}
+static_assert(kStaticMaxGroups * (uint64_t)dz::proj_chunk_elems(DZ_F16) / (dz::kShortProjFill - 1) <= dz::kShortProjTotal,
+              "groups that fill a kShortProjFill-th of their chunks, at most kStaticMaxGroups of them");
+
 // ZO tile lists: full tiles first (in tensor order), then the partial ones;
 // returns the number of full tiles. The order of
 // the tiles changes no result (z is a function of the element index), and it
@@ -643,7 +660,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     return rc;
   }
   for (int64_t ne : t->numels) t->bytes += (uint64_t)ne * es;
-  if (t->projection && t->bytes <= dz::kShortProjTotal * es && n <= dz::kShortProjGroups) {
+  if (t->projection && short_projection(t)) {
     t->short_proj = true;
     t->chunk_elems = (uint32_t)dz::short_proj_elems(dtype);
   }
@@ -676,7 +693,7 @@ int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const
     mem.add(&t->d_partials, nullptr, t->nchunks ? t->nchunks : 1, false);
     uint32_t most = 0;
     for (int32_t i = 0; i < n; ++i) most = std::max(most, t->group_begin[i + 1] - t->group_begin[i]);
-    if (t->short_proj && most <= dz::kShortCountChunks)
+    if (t->short_proj && n <= dz::kShortCountGroups && most <= dz::kShortCountChunks)
       mem.add(&t->d_group_done, nullptr, (size_t)t->n * dz::kDoneStride);
   }
   // work counters: zero here; every RMW and projection launch leaves them at zero again

@@ -31,9 +31,11 @@ __host__ __device__ constexpr bool proj_stores(int mode) { return mode != kProjS
 __host__ __device__ constexpr bool proj_sums(int mode) {
   return mode == kProjSumsq || mode == kProjReverseSumsq || mode == kProjDot;
 }
-// Most groups one dot launch takes (their pointers travel as kernel
-// arguments); dz_group_dot launches once per batch of groups.
-constexpr int kMaxDotGroups = 128;
+// Most groups one dot launch takes (their pointers travel as kernel arguments, of
+// which a launch has 4 KB); dz_group_dot launches once per batch of groups. With
+// 128, 3,000 fp16 groups of 33,001 elements took 742 us, with 448 298; 24 groups
+// of 20,480 6.7 and 6.6.
+constexpr int kMaxDotGroups = 448;
 struct DotGroups {
   uint64_t other[kMaxDotGroups];  // of groups group_base, group_base + 1, ...
   uint32_t group_base;
@@ -175,20 +177,28 @@ constexpr int kProjAlphaLds = 4096;
 // Infinity Cache): apply + reverse and the products in us, short and persistent,
 // fp16 36 x 2^20 elements 75 + 708 and 88 + 853, 44 x 2^20 89 + 866 and 102 + 1039,
 // fp32 32 x 2^20 133 + 2285 and 146 + 2307, 44 x 2^20 175 + 3059 and 192 + 3068.
+// Larger tables whose groups fill the persistent kernel's chunks to at most one
+// kShortProjFill-th run it too: fp16 60,000 x 1,100 143 / 84 / 182 and 626 / 394 /
+// 793 (norms to reverse), 20,000 x 3,000 57 / 68 / 71 and 189 / 109 / 234, fp32
+// 30,000 x 2,003 112 / 130 / 149 and 325 / 209 / 399 (fuller chunks: fp16 4,000 x
+// 16,384 50 / 73 / 76 and 67 / 63 / 89).
 // Chunks of half the size cost more counting (fp16 24 x 589,824: norms 17.4
 // against 12.6), of twice the size run the same.
 constexpr int kShortProjThreads = 256;
 __host__ __device__ constexpr int short_proj_elems(int dtype) { return dtype == DZ_F32 ? 2048 : 4096; }
 constexpr uint64_t kShortProjTotal = 3u << 24;
-constexpr int32_t kShortProjGroups = 1 << 16;  // more groups' counts would take over 8 MB
-// Tables whose largest group has more chunks than this keep no counts: a second
-// launch adds up the chunk sums (short_sums_kernel). A group's counts queue up,
+constexpr uint64_t kShortProjFill = 4;
+constexpr uint64_t kShortProjChunks = 1u << 22;  // workgroups of a launch
+// Tables whose largest group has more chunks than this, or of more groups (whose
+// counts would take over 8 MB), keep no counts: a second launch adds up the chunk
+// sums (short_sums_kernel). A group's counts queue up,
 // 13 ns each: norms in us with counts and with a second launch, fp16 2^20 elements
 // in one group (256 chunks) 7.0 and 8.8, 2^22 in four (256) 8.6 and 8.3, in two
 // (512) 13.5 and 8.5, in one (1,024) 17.4 and 8.8, 2^23 in 12 (171) 10.2 and 10.8,
 // in eight (256) 10.6 and 10.4, 2^24 in 16 (256) 16.2 and 14.6, in one (4,096) 57.5
 // and 15.0; fp32 2^24 in one (8,192) 109.8 and 28.3.
 constexpr uint32_t kShortCountChunks = 256;
+constexpr int32_t kShortCountGroups = 1 << 16;
 // The groups' finished-chunk counts lie 128 bytes apart: side by side, every
 // workgroup's atomic met in the same lines (12 ns each: the norms of fp16 24 x
 // 589,824, 3,456 counts, took 43 us against 13).

@@ -209,13 +209,13 @@ def test_long_tables_match_short_ones(dt):
 @pytest.mark.parametrize("chunks", [256, 257])
 def test_sums_around_the_count_line_match_fp64(dt, chunks):
     """Short tables whose largest group has 256 chunks (counted) or 257 (a second launch adds up the chunk
-    sums), 130 groups (two dot launches) with an empty one among them: norms, reverse + norms and dots
+    sums), 460 groups (two dot launches) with an empty one among them: norms, reverse + norms and dots
     against torch's fp64 sums. The squares are exact in fp64, so n terms are at most n / 2 roundings of
     2^-53 apart from any other order; the dots' terms differ in sign, so their bound is on their sizes."""
     from dizo_amd import _lib as L
     from dizo_amd.table import ProjTable
     cn = 2048 if dt == F32 else 4096
-    sizes = [(chunks - 1) * cn + 5] + [1000 + i for i in range(127)] + [0, cn]
+    sizes = [(chunks - 1) * cn + 5] + [1000 + i for i in range(457)] + [0, cn]
     G, total = len(sizes), sum(sizes)
     gen = torch.Generator(device="cuda").manual_seed(chunks)
     anchor = torch.empty(total, dtype=DT_TORCH[dt], device="cuda").normal_(0, 0.02, generator=gen)
@@ -248,24 +248,74 @@ def test_the_sums_of_one_large_group_do_not_hold_up_the_pass(dt, elems):
     anchor = torch.zeros(elems, dtype=DT_TORCH[dt], device="cuda")
     tab = ProjTable([torch.full_like(anchor, 0.5)], [anchor])
     alpha, out = torch.ones(1, dtype=anchor.dtype, device="cuda"), torch.empty(1, dtype=torch.float64, device="cuda")
-
-    def median_us(call):
-        times = []
-        for _ in range(25):
-            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-            for e in ev:
-                e.record()
-            tab.time_next(*ev)
-            call()
-            torch.cuda.synchronize()
-            times.append(ev[0].elapsed_time(ev[1]) * 1e3)
-        return sorted(times)[12]
-
-    apply = median_us(lambda: tab.project(alpha, L.DZ_PROJ_APPLY))
-    norms = median_us(lambda: tab.group_sumsq(out))
+    apply = _median_us(tab, lambda: tab.project(alpha, L.DZ_PROJ_APPLY))
+    norms = _median_us(tab, lambda: tab.group_sumsq(out))
     assert float(out[0]) == 0.25 * elems
     assert norms <= 2 * apply, (norms, apply)
     tab.close()
+
+
+def _median_us(tab, call, passes=15):
+    """Median time of the call's kernels."""
+    times = []
+    for _ in range(passes):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        for e in ev:
+            e.record()
+        tab.time_next(*ev)
+        call()
+        torch.cuda.synchronize()
+        times.append(ev[0].elapsed_time(ev[1]) * 1e3)
+    return sorted(times)[passes // 2]
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("G,lo,hi", [(66_000, 1, 200), (20_000, 2500, 2700)])
+def test_many_small_groups_match_torch(dt, G, lo, hi):
+    """More groups than keep counts (65,536), and groups that fill little of the long tables' chunks in a
+    table of more than 3 * 2^24 elements (fp32: more than a quarter, on the persistent kernel, whose groups'
+    alphas come from memory): apply and reverse against torch's own roundings, the sums against fp64 sums."""
+    from dizo_amd import _lib as L
+    from dizo_amd.table import ProjTable
+    r = np.random.default_rng(G)
+    sizes = r.integers(lo, hi + 1, size=G).tolist()
+    gen = torch.Generator(device="cuda").manual_seed(G)
+    t0 = torch.empty(sum(sizes), dtype=DT_TORCH[dt], device="cuda").normal_(0, 0.02, generator=gen)
+    th = t0 + torch.empty_like(t0).normal_(0, 4e-3, generator=gen)
+    alpha = torch.empty(G, device="cuda").uniform_(0.8, 1.2, generator=gen).to(DT_TORCH[dt])
+    each = alpha.repeat_interleave(torch.tensor(sizes, device="cuda"))
+    first = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    want = (th - t0) * each + t0
+    tab = ProjTable(list(th.split(sizes)), list(t0.split(sizes)))
+    sums = torch.empty(G, dtype=torch.float64, device="cuda")
+    for mode in (L.DZ_PROJ_APPLY, L.DZ_PROJ_REVERSE_SUMSQ, L.DZ_PROJ_APPLY, L.DZ_PROJ_REVERSE):
+        tab.project(alpha, mode, **({"sumsq": sums} if mode == L.DZ_PROJ_REVERSE_SUMSQ else {}))
+        assert torch.equal(th.view(torch.int32 if dt == F32 else torch.int16), want.view(torch.int32 if dt == F32 else torch.int16)), mode
+        if mode == L.DZ_PROJ_REVERSE_SUMSQ:
+            exact = np.add.reduceat((th - t0).double().square().cpu().numpy(), first)
+            np.testing.assert_allclose(sums.cpu().numpy(), exact, rtol=hi * 2.0**-53, atol=0)
+        d = want - t0
+        want = (d * each if mode in (L.DZ_PROJ_REVERSE, L.DZ_PROJ_REVERSE_SUMSQ) else d / each) + t0
+    tab.group_sumsq(sums)
+    exact = np.add.reduceat((th - t0).double().square().cpu().numpy(), first)
+    np.testing.assert_allclose(sums.cpu().numpy(), exact, rtol=hi * 2.0**-53, atol=0)
+    tab.close()
+
+
+def test_many_small_groups_do_not_wait_one_after_another():
+    """66,000 fp16 groups of 100 elements apply in at most 15 times what the same elements take in 64 groups
+    (43 against 10 us; through the long tables' chunks, one small group after another, 480)."""
+    from dizo_amd import _lib as L
+    from dizo_amd.table import ProjTable
+    total = 66_000 * 100
+    th, t0 = torch.full((total,), 0.5, dtype=torch.float16, device="cuda"), torch.zeros(total, dtype=torch.float16, device="cuda")
+    times = []
+    for G in (66_000, 64):
+        tab = ProjTable(list(th.split(total // G)), list(t0.split(total // G)))
+        alpha = torch.ones(tab.n, dtype=torch.float16, device="cuda")
+        times.append(_median_us(tab, lambda: tab.project(alpha, L.DZ_PROJ_APPLY)))
+        tab.close()
+    assert times[0] <= 15 * times[1], times
 
 
 def test_empty_and_rejects():
@@ -335,19 +385,19 @@ def test_group_dot_matches_fp64(dt):
 
 
 def test_group_dot_more_groups_than_one_launch_takes():
-    """200 groups (more than the 128 one dot launch takes): every group's sum
+    """500 groups (more than the 448 one dot launch takes): every group's sum
     against float64 torch, including empty groups at a batch boundary."""
     from dizo_amd.table import ProjTable
     dev = torch.device("cuda", 0)
     gen = torch.Generator(device=dev).manual_seed(6)
-    sizes = [(1000 + 37 * i) if i not in (127, 128) else 0 for i in range(200)]
+    sizes = [(1000 + 37 * i) if i not in (447, 448) else 0 for i in range(500)]
     ths = [(torch.randn(n, device=dev, generator=gen) * 0.02).half() for n in sizes]
     t0s = [(t.float() - 1e-3).half() for t in ths]
     others = [torch.randn(n, device=dev, generator=gen).half() for n in sizes]
-    dot = torch.empty(200, dtype=torch.float64, device=dev)
+    dot = torch.empty(500, dtype=torch.float64, device=dev)
     tab = ProjTable(ths, t0s)
     tab.group_dot(others, dot)
-    for g in range(200):
+    for g in range(500):
         want = float((others[g].double() * (ths[g] - t0s[g]).double()).sum())
         assert float(dot[g]) == pytest.approx(want, rel=1e-12, abs=1e-300), g
     tab.close()
