@@ -239,6 +239,20 @@ def test_sums_around_the_count_line_match_fp64(dt, chunks):
     tab.close()
 
 
+def _median_us(tab, call, passes=15):
+    """Median time of the call's kernels."""
+    times = []
+    for _ in range(passes):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        for e in ev:
+            e.record()
+        tab.time_next(*ev)
+        call()
+        torch.cuda.synchronize()
+        times.append(ev[0].elapsed_time(ev[1]) * 1e3)
+    return sorted(times)[passes // 2]
+
+
 @pytest.mark.parametrize("dt,elems", [(F16, 2**24), (F32, 2**23)])
 def test_the_sums_of_one_large_group_do_not_hold_up_the_pass(dt, elems):
     """One group of 32 MB: the norm pass reads 64 MB, an apply moves 96. With a count for each chunk of the
@@ -253,20 +267,6 @@ def test_the_sums_of_one_large_group_do_not_hold_up_the_pass(dt, elems):
     assert float(out[0]) == 0.25 * elems
     assert norms <= 2 * apply, (norms, apply)
     tab.close()
-
-
-def _median_us(tab, call, passes=15):
-    """Median time of the call's kernels."""
-    times = []
-    for _ in range(passes):
-        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-        for e in ev:
-            e.record()
-        tab.time_next(*ev)
-        call()
-        torch.cuda.synchronize()
-        times.append(ev[0].elapsed_time(ev[1]) * 1e3)
-    return sorted(times)[passes // 2]
 
 
 @pytest.mark.parametrize("dt", DTS)
@@ -384,13 +384,18 @@ def test_group_dot_matches_fp64(dt):
     tab.close()
 
 
-def test_group_dot_more_groups_than_one_launch_takes():
+@pytest.mark.parametrize("large", [False, True])
+def test_group_dot_more_groups_than_one_launch_takes(large):
     """500 groups (more than the 448 one dot launch takes): every group's sum
-    against float64 torch, including empty groups at a batch boundary."""
+    against float64 torch, including empty groups at a batch boundary. With a
+    large group in the second launch (more than 3 * 2^24 elements) the table is
+    a long one, whose launches share its work counters and partial sums."""
     from dizo_amd.table import ProjTable
     dev = torch.device("cuda", 0)
     gen = torch.Generator(device=dev).manual_seed(6)
     sizes = [(1000 + 37 * i) if i not in (447, 448) else 0 for i in range(500)]
+    if large:
+        sizes[460] = 51_000_007
     ths = [(torch.randn(n, device=dev, generator=gen) * 0.02).half() for n in sizes]
     t0s = [(t.float() - 1e-3).half() for t in ths]
     others = [torch.randn(n, device=dev, generator=gen).half() for n in sizes]
@@ -398,17 +403,22 @@ def test_group_dot_more_groups_than_one_launch_takes():
     tab = ProjTable(ths, t0s)
     tab.group_dot(others, dot)
     for g in range(500):
-        want = float((others[g].double() * (ths[g] - t0s[g]).double()).sum())
-        assert float(dot[g]) == pytest.approx(want, rel=1e-12, abs=1e-300), g
+        terms = others[g].double() * (ths[g] - t0s[g]).double()
+        want = float(terms.sum())
+        # the large group's 5e7 terms all but cancel (sum 7, sizes 4e4): bounded by their sizes
+        near = 0.0 if sizes[g] < 10**6 else float(terms.abs().sum()) * sizes[g] * 2.0**-53
+        assert float(dot[g]) == pytest.approx(want, rel=1e-12, abs=max(near, 1e-300)), g
     tab.close()
 
 
 @pytest.mark.parametrize("dt", [F16, F32])
 def test_more_groups_than_the_lds_alpha_table(dt):
-    """More groups (4100) than a projection workgroup keeps alphas for in LDS
+    """More groups (4100, and a large one that makes the table a long one) than
+    a workgroup of the persistent projection kernel keeps alphas for in LDS
     (4096): each chunk then reads its group's alpha from memory. Apply, reverse
-    and the group norms against the oracle, on views of one buffer."""
-    from dizo_amd._lib import DZ_PROJ_APPLY, DZ_PROJ_REVERSE_SUMSQ
+    and the group norms against the oracle, on views of one buffer (the large
+    group against torch's roundings)."""
+    from dizo_amd._lib import DZ_PROJ_APPLY, DZ_PROJ_REVERSE, DZ_PROJ_REVERSE_SUMSQ
     from dizo_amd.table import ProjTable
     G, n = 4100, 37
     dev = torch.device("cuda", 0)
@@ -418,20 +428,34 @@ def test_more_groups_than_the_lds_alpha_table(dt):
     th_buf, t0_buf = to_torch(th_all, dt, dev), to_torch(t0_all, dt, dev)
     ths = [th_buf[g * n:(g + 1) * n] for g in range(G)]
     t0s = [t0_buf[g * n:(g + 1) * n] for g in range(G)]
-    alphas = from_f32(np.linspace(0.6, 1.2, G).astype(np.float32), dt)
-    tab = ProjTable(ths, t0s)
-    tab.project(to_torch(alphas, dt, dev), DZ_PROJ_APPLY)
+    alphas = from_f32(np.linspace(0.6, 1.2, G + 1).astype(np.float32), dt)
+    alpha_t = to_torch(alphas, dt, dev)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    t0_large = torch.empty(3 * 2**24 + 10_000_019, dtype=DT_TORCH[dt], device=dev).normal_(0, 0.02, generator=gen)
+    large = t0_large + torch.empty_like(t0_large).normal_(0, 4e-3, generator=gen)
+    want_large = (large - t0_large) * alpha_t[G:] + t0_large
+    tab = ProjTable(ths + [large], t0s + [t0_large])
+    tab.project(alpha_t, DZ_PROJ_APPLY)
+    assert torch.equal(large, want_large)
     got = to_bits(th_buf)
     want = np.concatenate([A.apply(th_all[g * n:(g + 1) * n], t0_all[g * n:(g + 1) * n], alphas[g:g + 1], dt)
                            for g in range(G)])
     assert_bits_equal(got, want, dt, "apply")
-    sumsq = torch.empty(G, dtype=torch.float64, device=dev)
-    tab.project(to_torch(alphas, dt, dev), DZ_PROJ_REVERSE_SUMSQ, sumsq=sumsq)
+    sumsq = torch.empty(G + 1, dtype=torch.float64, device=dev)
+    tab.project(alpha_t, DZ_PROJ_REVERSE_SUMSQ, sumsq=sumsq)
+    want_large = (want_large - t0_large) / alpha_t[G:] + t0_large
+    assert torch.equal(large, want_large)
+    exact = float((large - t0_large).double().square().sum())
+    assert float(sumsq[G]) == pytest.approx(exact, rel=large.numel() * 2.0**-53)
     rev = [A.reverse(want[g * n:(g + 1) * n], t0_all[g * n:(g + 1) * n], alphas[g:g + 1], dt) for g in range(G)]
     assert_bits_equal(to_bits(th_buf), np.concatenate(rev), dt, "reverse")
     s = sumsq.cpu().numpy()
     for g in range(0, G, 97):
         assert s[g] == pytest.approx(A.group_sumsq(rev[g], t0_all[g * n:(g + 1) * n], dt), rel=1e-12), g
+    tab.project(alpha_t, DZ_PROJ_REVERSE)
+    rev = [A.reverse(rev[g], t0_all[g * n:(g + 1) * n], alphas[g:g + 1], dt) for g in range(G)]
+    assert_bits_equal(to_bits(th_buf), np.concatenate(rev), dt, "reverse without norms")
+    assert torch.equal(large, (want_large - t0_large) / alpha_t[G:] + t0_large)
     tab.close()
 
 

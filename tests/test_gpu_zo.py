@@ -46,10 +46,12 @@ def _make_tensors(dt, seed, sizes=SIZES, misaligned=(3, 6)):
 def _fused_table(tensors, prefetch, **kw):
     """A ZO table on the long tables' kernel, whose restore+update+next perturb
     launches run the prefetching tile loop (prefetch=True, every launch) or the
-    plain tile loop (prefetch=False, no launch)."""
+    plain tile loop (prefetch=False, no launch); prefetch=None: on the kernel
+    that its size gives it, the short tables' one for most sizes here."""
     from dizo_amd.table import ZOTable
     tab = ZOTable(tensors, **kw)
-    tab.set_prefetch_min_tiles(1 if prefetch else 0xFFFFFFFF)
+    if prefetch is not None:
+        tab.set_prefetch_min_tiles(1 if prefetch else 0xFFFFFFFF)
     return tab
 
 
@@ -132,7 +134,7 @@ def test_rmw_uses_exported_z(dt):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("prefetch", [True, False])
+@pytest.mark.parametrize("prefetch", [True, False, None])
 @pytest.mark.parametrize("first", [1, 3, 7])
 def test_packed_odd_tensors_match_oracle(dt, prefetch, first):
     """Tensors of odd sizes end to end in one buffer, from every kind of start address, full tiles
@@ -160,12 +162,16 @@ def test_packed_odd_tensors_match_oracle(dt, prefetch, first):
     tab.close()
 
 
-@pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("elems", [8192 * 256 - 3, 3 * 2**22, 8192 * 1500 + 77, 2**24, 3 * 2**24, 2**26 + 9])
+# the lines up to which the three-way pass, restore + update, and perturb and update run the short tables' kernel
+SHORT_LINES = {F16: (5 * 2**22, 3 * 2**24, 2**26), BF16: (3 * 2**22, 3 * 2**23, 2**26), F32: (2**24,)}
+
+
+@pytest.mark.parametrize("dt,elems", [(dt, n) for dt in DTS for n in (8192 * 256 - 3, 8192 * 1500 + 77, *SHORT_LINES[dt])])
 def test_short_tables_match_the_persistent_kernel(dt, elems):
-    """Tables at and around the lines below which passes run the short tables' kernel, with one to many
-    tiles per workgroup and odd tensors among them, across a wrap of the z counter's low word: every
-    pass gives the persistent kernel's bits (which the other tests hold against the oracle)."""
+    """Tables below and on the lines up to which passes run the short tables' kernel (at least one pass does
+    at each size), with one to many tiles per workgroup and odd tensors among them, across a wrap of the z
+    counter's low word: every pass gives the persistent kernel's bits (which the other tests hold against
+    the oracle)."""
     from dizo_amd.table import ZOTable
     cut = [elems // 3 + 1, 5, elems // 2 + 3]
     sizes = cut + [elems - sum(cut)]
@@ -263,10 +269,10 @@ def test_tables_around_the_cache_size_agree(dt):
 
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("scale", [1.0, -2.0, 0.5])
-def test_perturb_matches_oracle(dt, scale):
-    from dizo_amd.table import ZOTable
+@pytest.mark.parametrize("prefetch", [True, None])
+def test_perturb_matches_oracle(dt, scale, prefetch):
     tensors, host, keep = _make_tensors(dt, 7)
-    tab = ZOTable(tensors)
+    tab = _fused_table(tensors, prefetch)
     seed, eps = 123456789, 1e-3
     tab.perturb(seed, scale, eps)
     for i, (t, h, z) in enumerate(zip(tensors, host, _z_host(tab, seed, dt))):
@@ -275,11 +281,11 @@ def test_perturb_matches_oracle(dt, scale):
 
 
 @pytest.mark.parametrize("dt", DTS)
-def test_full_step_sequence_matches_oracle(dt):
+@pytest.mark.parametrize("prefetch", [True, None])
+def test_full_step_sequence_matches_oracle(dt, prefetch):
     """perturb +1, -2, then fused restore+update; and the unfused restore, update."""
-    from dizo_amd.table import ZOTable
     tensors, host, keep = _make_tensors(dt, 21)
-    tab = ZOTable(tensors)
+    tab = _fused_table(tensors, prefetch)
     seed, eps, g, lr = 424242, 1e-3, -0.734375, 9.93875e-07
     zs = _z_host(tab, seed, dt)
     tab.perturb(seed, 1.0, eps)
@@ -303,7 +309,7 @@ def test_full_step_sequence_matches_oracle(dt):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("prefetch", [False, True])
+@pytest.mark.parametrize("prefetch", [False, True, None])
 def test_restore_update_perturb_matches_oracle(dt, prefetch):
     """Restore + update of step seed, then +1 of step next_seed, in one pass: the
     same bits as the three passes, and as the oracle (plain and prefetching
@@ -328,11 +334,11 @@ def test_restore_update_perturb_matches_oracle(dt, prefetch):
 
 
 @pytest.mark.parametrize("dt", DTS)
-def test_device_scalar_overrides(dt):
+@pytest.mark.parametrize("prefetch", [True, None])
+def test_device_scalar_overrides(dt, prefetch):
     """Seed / grad / lr read from device memory give the by-value results."""
-    from dizo_amd.table import ZOTable
     tensors, host, keep = _make_tensors(dt, 33, sizes=[40000, 77])
-    tab = ZOTable(tensors)
+    tab = _fused_table(tensors, prefetch)
     seed, eps, g, lr = 55555, 1e-3, 1.25, 2e-6
     dev = torch.device("cuda", 0)
     d_seed = torch.tensor([seed], dtype=torch.int64, device=dev)
@@ -380,7 +386,7 @@ def _opt_like_sizes(target_elems: int, d: int = 768):
 
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("target", [200_000, 1_200_000, 6_000_000, 90_000_000])
-@pytest.mark.parametrize("prefetch", [False, True])
+@pytest.mark.parametrize("prefetch", [False, True, None])
 def test_multi_tile_launches_match_torch(dt, target, prefetch):
     """Tables of 3 to ~1400 tiles (grids below and above the counter fan-out,
     several tiles per workgroup): every element is processed exactly once per
@@ -569,7 +575,7 @@ def test_single_tensor_beyond_2_32_elements(prefetch):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("prefetch", [False, True])
+@pytest.mark.parametrize("prefetch", [False, True, None])
 def test_tiles_across_the_2_32_counter_boundary(dt, prefetch):
     """Philox counters q = e >> 3 past 2^32: z offsets put one tile of each tile
     size across q = 2^32 (its counters' high word changes inside the tile),
@@ -612,7 +618,7 @@ def test_tiles_across_the_2_32_counter_boundary(dt, prefetch):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("prefetch", [False, True])
+@pytest.mark.parametrize("prefetch", [False, True, None])
 def test_special_values_follow_ieee_like_the_oracle(dt, prefetch):
     """theta holding +-inf, NaN, +-0, the largest finite value and the smallest
     subnormal, among ordinary values: every RMW mode, then the projection's
