@@ -398,8 +398,10 @@ void build_chunks(const dz_table* t, uint32_t elems, std::vector<DzChunk>* out,
 }
 
 // Whether a projection table runs proj_short_kernel (see kShortProjTotal). With
-// at most kStaticMaxGroups groups its first line alone decides, as in
-// dz_group_sumsq_static: small groups fill less than kStaticMaxGroups chunks.
+// at most kStaticMaxGroups groups the elements alone decide, as in
+// dz_group_sumsq_static: n groups have at most n more chunks than their elements
+// fill, so groups that fill a kShortProjFill-th of theirs hold at most n * cn /
+// (kShortProjFill - 1).
 bool short_projection(const dz_table* t) {
   const uint64_t cn = (uint64_t)dz::proj_chunk_elems(t->dtype), sn = (uint64_t)dz::short_proj_elems(t->dtype);
   uint64_t elems = 0, chunks = 0, short_chunks = 0;
@@ -412,7 +414,7 @@ bool short_projection(const dz_table* t) {
          (elems <= dz::kShortProjTotal || elems * dz::kShortProjFill <= chunks * cn);
 }
 static_assert(kStaticMaxGroups * (uint64_t)dz::proj_chunk_elems(DZ_F16) / (dz::kShortProjFill - 1) <= dz::kShortProjTotal,
-              "groups that fill a kShortProjFill-th of their chunks, at most kStaticMaxGroups of them");
+              "the table-free pass and a table take the same kernel");
 
 // ZO tile lists: full tiles first (in tensor order), then the partial ones;
 // returns the number of full tiles. The order of
@@ -782,7 +784,7 @@ int32_t dz_restore_update_perturb(dz_table* t, uint64_t seed, uint64_t next_seed
 int32_t dz_normals(uint64_t seed, uint32_t stream_id, uint64_t offset, int64_t n, int32_t dtype, void* d_out,
                    void* stream) {
   if (!valid_dtype(dtype)) return fail(DZ_ERR_INVALID, "unknown dtype");
-  // one thread per element, 256 per block: keep the grid below 2^31 blocks
+  // more than any device holds
   if (n < 0 || n > ((int64_t)1 << 38)) return fail(DZ_ERR_INVALID, "n out of range");
   if (n == 0) return DZ_OK;
   int dev;

@@ -92,12 +92,19 @@ constexpr uint64_t short_elems(int dtype, int mode) {
 
 // Tensors of up to kPlainBytes in all, the size of the Infinity Cache, are read
 // and written with plain accesses by the persistent kernel; longer tables'
-// accesses carry the non-temporal hint. Pass times in us (perturb / three-way)
-// with the hint and without, three tables used in turn: fp16 2^26 elements (128
-// MB) 47.0 / 51.0 and 47.3 / 45.7, 2^27 87.5 / 91.6 and 82.9 / 84.7, 2^27.25
-// 104 / 110 and 113 / 115, 2^28 169 / 173 and 183 / 185; fp32 2^25 44.9 / 45.4
-// and 43.1 / 40.8, 2^26 (256 MB) 83.7 / 85.0 and 78.2 / 78.0, 2^26.25 99 / 101
-// and 111 / 104, 2^28 323 / 326 and 358 / 356.
+// accesses carry the non-temporal hint. What a plain pass leaves in the cache the
+// forward reads there: GPU time in us of perturb + products of 1,536 tokens with
+// all the weights + three-way pass + products, with the hint and without, fp16 81
+// MB 908 and 859, 121 MB 1340 and 1258, 162 MB 1879 and 1664, 229 MB 2638 and 2429
+// (of 256 tokens 1977 and 1598), bf16 229 MB 2609 and 2398, fp32 108 MB 2041 and
+// 2017, 216 MB 3856 and 3821. The passes themselves, kernel time in us (perturb /
+// three-way), three tables used in turn: fp16 2^26 elements (128 MB) 47.0 / 51.0
+// and 47.3 / 45.7, 2^27 87.5 / 91.6 and 82.9 / 84.7, 2^27.25 104 / 110 and 113 /
+// 115, 2^28 169 / 173 and 183 / 185; fp32 2^25 44.9 / 45.4 and 43.1 / 40.8, 2^26
+// (256 MB) 83.7 / 85.0 and 78.2 / 78.0, 2^26.25 99 / 101 and 111 / 104, 2^28 323 /
+// 326 and 358 / 356. (Between 64 and 256 MB a plain pass's write-backs fall into
+// what follows: passes back to back over three tables, fp16 2^27 elements 93.4 /
+// 94.9 a pass, with the hint 88.0 / 92.4.)
 constexpr uint64_t kPlainBytes = 1u << 28;
 
 // LDS bytes of the per-launch delta table of an RMW launch: 16-bit entries

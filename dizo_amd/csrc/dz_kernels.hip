@@ -1180,11 +1180,11 @@ __global__ void __launch_bounds__(kRmwThreads, kRmwWavesPerEU) rmw_kernel(const 
 // against 22.6 us). Pass times in us (perturb / three-way), this kernel and the
 // persistent one with its hints: fp16 2^14 elements 4.0 / 4.1 and 6.8 / 9.0,
 // 2^20 4.2 / 4.3 and 10.2 / 14.3, 2^22 6.0 / 7.5 and 13.1 / 19.5, 2^24 12.8 /
-// 19.0, 2^25 21.1 / 30.7 and 27.2 / 30.3; fp32 2^20 4.6 / 5.4 and 9.9 / 10.4,
-// 2^24 21.8 / 22.9 and 27.6 / 28.2. A launch is bound by its latencies (about 4
-// us) up to 2^20 elements, then by the VALU: with one Philox round for seven,
-// fp16 2^25 elements take 21.4 / 22.4 us; with lookups free of bank conflicts,
-// the same time.
+// 19.0, 2^25 21.1 / 30.7 and 27.2 / 30.3 (the three-way pass runs the persistent
+// kernel there: short_elems); fp32 2^20 4.6 / 5.4 and 9.9 / 10.4, 2^24 21.8 / 22.9
+// and 27.6 / 28.2. A launch is bound by its latencies (about 4 us) up to 2^20
+// elements, then by the VALU: with one Philox round for seven, fp16 2^25 elements
+// take 21.4 / 22.4 us; with lookups free of bank conflicts, the same time.
 // ---------------------------------------------------------------------------
 
 // The launch's operation on two packed 16-bit elements with their signed z

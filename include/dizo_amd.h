@@ -73,8 +73,10 @@ int32_t dz_philox_host(uint64_t seed, uint32_t stream_id, uint64_t q, uint32_t o
  * per 32,768 elements of a 16-bit type or 8,192 fp32 elements; a bf16 ZO
  * table also one per 24,576 elements for its restore + update + next
  * perturbation launches; a short ZO table also one per 8,192 elements; a
- * projection table one per chunk and an fp64 partial sum per chunk) and its
- * work counters.
+ * projection table one per chunk, of as many elements as a ZO table's tile, or
+ * of 4,096 (2,048 fp32) in a short projection table, and an fp64 partial sum
+ * per chunk), its work counters and, for a short projection table of up to
+ * 65,536 groups, 128 bytes per group.
  * Replaces the trainable-set walk of trainer.py:1147-1160 (ZO table) and the
  * exclude_list walk of trainer.py:405-451, 581-584 (projection table). */
 int32_t dz_table_create(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const int64_t* numels,
@@ -194,9 +196,10 @@ int32_t dz_init(int32_t device);
  * 4096 groups and 262,144 chunks of 32,768 elements of a 16-bit type (8.6 G
  * elements) or of 8,192 fp32 elements (2.1 G); larger inputs return
  * DZ_ERR_INVALID. Every call on one device shares that array,
- * so calls that overlap in time on one device race (their own outputs may be
- * wrong; later calls are not affected): order them on one stream. After dz_init(device) a call allocates nothing; without it, the
- * first call on a device does dz_init's work itself. */
+ * so calls that overlap in time on one device race: order them on one
+ * stream. (A call uses nothing that an earlier one left there.) After
+ * dz_init(device) a call allocates nothing; without it, the first call on a
+ * device does dz_init's work itself. */
 int32_t dz_group_sumsq_static(const uint64_t* ptrs, const uint64_t* anchor_ptrs, const int64_t* numels,
                               int32_t n, int32_t dtype, double* d_sumsq, float* d_norm_f32, void* d_norm_T,
                               void* stream);

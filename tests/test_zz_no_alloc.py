@@ -194,13 +194,14 @@ def test_first_call_after_init_allocates_nothing():
         assert abs(got - want) <= 1e-12 * max(want, 1e-300), (got, want)
 
 
-def test_static_call_in_a_captured_graph():
+@pytest.mark.parametrize("sizes", [[50_000, 7, 32768 * 2, 1000], [4000, 7, 20_000, 32768]])
+def test_static_call_in_a_captured_graph(sizes):
     """The entry point recorded in a hipGraph (torch.cuda.graph) after dz_init:
     the capture succeeds, and each of several replays, with eager launches on
     the inputs and synchronisations between them, gives the eager call's
-    outputs bit for bit."""
+    outputs bit for bit. (The first sizes take two launches, the second one.)"""
     dt = torch.bfloat16
-    th, t0 = _groups([50_000, 7, 32768 * 2, 1000], dt, 12, misaligned=(1,))
+    th, t0 = _groups(sizes, dt, 12, misaligned=(1,))
     L.call("dz_init", torch.cuda.current_device())
     want = _static(th, t0, dt)
     n = len(th)
